@@ -1628,8 +1628,8 @@ namespace smr
                         for (size_t j = 0; j < nc; ++j)
                         {
                             const int64_t n = rb[changed[j]].nm.nref;
-                            nu[j]           = static_cast<double*>(dev_alloc(size_t(std::max<int64_t>(n, 1)) * 8, s));
-                            nv[j]           = static_cast<double*>(dev_alloc(size_t(std::max<int64_t>(n, 1)) * 8, s));
+                            nu[j]           = static_cast<double*>(dev_alloc(field_bytes(n), s));
+                            nv[j]           = static_cast<double*>(dev_alloc(field_bytes(n), s));
                         }
                     }
                     std::optional<ScopedTimer> tp(std::in_place, ctx_, "update_fields program");

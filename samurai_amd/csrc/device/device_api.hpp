@@ -345,6 +345,25 @@ namespace smr::dev
     void sequence(int dim, int ps, const SeqItem* items, int i0, int i1, const List& l_proj, const List& l_pred, const List& l_max, double* u,
                   uint8_t* tag, bool has_bc, double bc_value, hipStream_t s);
 
+    // update_ghost_mr as one dataflow launch (ghost_flow.hip): the ghosts in an
+    // order that keeps every source before its readers, cut into items of one
+    // kind and level.  Item k is the indices [c0[k], c1[k]) of the projection
+    // or prediction list or of the recipes, 64 per wave, from wave wave0[k] on;
+    // a recipe is (dst, op | n << 8, first source, first of its n sources in
+    // rsrc), every slot written once.  The 8 bytes after the field's nref
+    // values hold the launch's ticket.
+    constexpr int kFlowItems = 64;
+    struct GhostFlow
+    {
+        List proj, pred;
+        const int32_t* rec;
+        const int32_t* rsrc;
+        int nitems, nwaves;
+        int32_t wave0[kFlowItems], c0[kFlowItems], c1[kFlowItems];
+        int32_t op[kFlowItems]; // SeqOp
+    };
+    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s);
+
     struct Segment
     {
         int32_t op, dim, pred_s, has_bc;

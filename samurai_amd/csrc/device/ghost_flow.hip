@@ -1,0 +1,379 @@
+// update_ghost_mr as one dataflow launch.
+//
+// The update is a chain of stages (per level, finest first: outer ghosts, then
+// the projection into the level below; then the predictions, coarsest level
+// first), about 35 of them on a 2D L4..12 mesh.  Most ghosts do not need that
+// order: a ghost waits only for the ghosts it reads, and on graded meshes 94 %
+// of them read cells or ghosts that read cells (2D L4..12: 41 K and 40 K of
+// 87 K ghosts at depth 1 and 2, the deepest at 10).  So every ghost is written
+// exactly once, by a lane that waits for its own sources: k_ghost_reset stores
+// a mark in every ghost the update writes, then k_ghost_flow computes all of
+// them in one grid, each lane loading its sources again while one still holds
+// the mark.  The values travel through 8-byte agent-scope stores and loads, so
+// a source is seen either as the mark or as its final value: no flags, no
+// fences, no barriers.
+//
+// Bound: latency, launch + index chain + one store-to-load trip per depth.
+// The stages were bound by their launches (3 to 4 us each) and, for the small
+// ones, by a block barrier and a chain of five dependent loads per stage.
+// update_ghost_mr + upwind, one step: 2D L4..12 (158 K cells) 28 us against 90
+// with a launch per stage, 3D L2..8 (234 K cells) 38 against 96, 2D L2..7
+// (5.9 K cells) 19 against 26.
+//
+// Every wait ends.  Blocks take their place in the order of the ghosts from a
+// counter (the ticket), the order keeps every source before its readers, so
+// the lowest unfinished wave waits for nothing that is not done; and a wave
+// gives up after kMaxSpins rounds and uses what it has read (which is the
+// right value when a cell itself holds the bits of the mark).
+#include "cell_ops.hpp"
+
+namespace smr::dev
+{
+    namespace
+    {
+        // a signalling NaN: arithmetic results are never signalling, and a
+        // copied value with these very bits is stored quiet
+        constexpr unsigned long long kMark = 0x7FF05A3C96E1D2B4ull;
+        constexpr unsigned long long kQuiet = 0x0008000000000000ull;
+        constexpr int kMaxSpins            = 1 << 17;
+
+        __device__ __forceinline__ bool marked(double v)
+        {
+            return (unsigned long long)__double_as_longlong(v) == kMark;
+        }
+
+        // the first look at a source: any cache may answer, since a line that
+        // is out of date holds the mark
+        __device__ __forceinline__ double look(const double* p)
+        {
+            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+
+        __device__ __forceinline__ double look_again(const double* p)
+        {
+            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+
+        __device__ __forceinline__ void publish(double* p, double v)
+        {
+            if (marked(v))
+            {
+                v = __longlong_as_double((long long)(kMark | kQuiet));
+            }
+            __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+
+        // runs attempt(last) on the lanes not yet done until all of them are:
+        // it returns true once the lane has published (always when last)
+        template <class F>
+        __device__ __forceinline__ void until_done(bool active, F&& attempt)
+        {
+            bool done = !active;
+            for (int spin = 0; !__all(done); ++spin)
+            {
+                if (!done)
+                {
+                    done = attempt(spin >= kMaxSpins);
+                }
+            }
+        }
+
+        // N sources held in registers; true when none of them is marked
+        template <int N, class Addr>
+        struct Sources
+        {
+            double v[N];
+            bool fresh = true;
+            __device__ __forceinline__ bool ready(const Addr& at)
+            {
+                bool ok = true;
+#pragma unroll
+                for (int k = 0; k < N; ++k)
+                {
+                    if (fresh)
+                    {
+                        v[k] = look(at(k));
+                    }
+                    else if (marked(v[k]))
+                    {
+                        v[k] = look_again(at(k));
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < N; ++k)
+                {
+                    ok = ok && !marked(v[k]);
+                }
+                fresh = false;
+                return ok;
+            }
+        };
+
+        // projection_op_ (op_project_at) on waited-for sources
+        template <int DIM>
+        __device__ __forceinline__ void flow_project(const List& l, int64_t c, bool active, double* u)
+        {
+            constexpr int NR     = 1 << (DIM - 1);
+            constexpr double inv = 1.0 / double(1 << DIM);
+            double* dst          = nullptr;
+            const double* row[NR];
+            if (active)
+            {
+                const Cell cell  = locate(l, c);
+                const int64_t* b = bases(l, cell.run);
+                dst              = u + b[0] + cell.x;
+#pragma unroll
+                for (int r = 0; r < NR; ++r)
+                {
+                    row[r] = u + b[1 + r] + 2 * cell.x;
+                }
+            }
+            auto at = [&](int k) { return row[k >> 1] + (k & 1); };
+            Sources<2 * NR, decltype(at)> s;
+            until_done(active,
+                       [&](bool last)
+                       {
+                           if (!s.ready(at) && !last)
+                           {
+                               return false;
+                           }
+                           double sum = 0;
+#pragma unroll
+                           for (int r = 0; r < NR; ++r)
+                           {
+                               sum += s.v[2 * r] + s.v[2 * r + 1];
+                           }
+                           publish(dst, sum * inv);
+                           return true;
+                       });
+        }
+
+        // prediction_op <s,false> (op_predict_fine_at) on waited-for sources
+        template <int DIM, int S>
+        __device__ __forceinline__ void flow_predict(const List& l, int64_t c, bool active, double* u)
+        {
+            constexpr int NY = 2 * S + 1, NZ = DIM == 3 ? NY : 1, N = NZ * NY * NY;
+            double* dst = nullptr;
+            const double* row[NZ * NY];
+            int px = 0, py = 0, pz = 0;
+            if (active)
+            {
+                const Cell cell  = locate(l, c);
+                const int64_t* b = bases(l, cell.run);
+                dst              = u + b[0] + cell.x;
+                px               = cell.x & 1;
+                py               = cell.y & 1;
+                pz               = cell.z & 1;
+#pragma unroll
+                for (int r = 0; r < NZ * NY; ++r)
+                {
+                    row[r] = u + b[1 + r] + (cell.x >> 1) - S;
+                }
+            }
+            auto at = [&](int k) { return row[k / NY] + k % NY; };
+            Sources<N, decltype(at)> s;
+            until_done(active,
+                       [&](bool last)
+                       {
+                           if (!s.ready(at) && !last)
+                           {
+                               return false;
+                           }
+                           double v;
+                           if constexpr (S == 0)
+                           {
+                               v = s.v[0];
+                           }
+                           else
+                           {
+                               v = 0;
+#pragma unroll
+                               for (int rz = 0; rz < NZ; ++rz)
+                               {
+#pragma unroll
+                                   for (int ry = 0; ry < 3; ++ry)
+                                   {
+#pragma unroll
+                                       for (int sx = 0; sx < 3; ++sx)
+                                       {
+                                           const double f = s.v[(rz * 3 + ry) * 3 + sx];
+                                           double coeff   = 1.;
+                                           coeff *= pcoef(px, sx);
+                                           coeff *= pcoef(py, ry);
+                                           if constexpr (DIM == 3)
+                                           {
+                                               coeff *= pcoef(pz, rz);
+                                           }
+                                           v += f * coeff;
+                                       }
+                                   }
+                               }
+                           }
+                           publish(dst, v);
+                           return true;
+                       });
+        }
+
+        // op_recipe on waited-for sources; (dst, op | n << 8, first source,
+        // first of the n sources in src).  The sources are taken one after the
+        // other as they come, in the recipe's order.
+        __device__ __forceinline__ void flow_recipe(const int32_t* __restrict__ rec, const int32_t* __restrict__ src, int64_t c, bool active,
+                                                    double* u, double bc)
+        {
+            int4 r{};
+            if (active)
+            {
+                r = reinterpret_cast<const int4*>(rec)[c];
+            }
+            const int op = r.y & 255, n = r.y >> 8;
+            double acc = 0;
+            int k      = 0;
+            bool first = true;
+            until_done(active,
+                       [&](bool last)
+                       {
+                           for (; k < n; ++k)
+                           {
+                               const double* p = u + (k == 0 ? r.z : src[r.w + k]);
+                               double x        = first ? look(p) : look_again(p);
+                               if (marked(x) && first)
+                               {
+                                   x = look_again(p);
+                               }
+                               if (marked(x) && !last)
+                               {
+                                   first = false;
+                                   return false;
+                               }
+                               first = true;
+                               if (op == 0)
+                               {
+                                   acc = x;
+                               }
+                               else if (op == 1)
+                               {
+                                   acc = 2 * bc - x;
+                               }
+                               else if (op == 2)
+                               {
+                                   acc += x;
+                               }
+                               else if (k == 0)
+                               {
+                                   acc = x;
+                               }
+                               else if (n == 3)
+                               {
+                                   // u0 - u1 * 3 + u2 * 3
+                                   acc = k == 1 ? acc - x * 3.0 : acc + x * 3.0;
+                               }
+                               else
+                               {
+                                   // u0 - u1 * 5 + u2 * 10 - u3 * 10 + u4 * 5
+                                   const double w = x * (k == 1 || k == 4 ? 5.0 : 10.0);
+                                   acc            = (k & 1) ? acc - w : acc + w;
+                               }
+                           }
+                           if (op == 2 && n > 0)
+                           {
+                               acc /= n;
+                           }
+                           publish(u + r.x, acc);
+                           return true;
+                       });
+        }
+
+        // the item of wave w: the last one whose first wave is at most w
+        // (at most 64 items, one per lane)
+        __device__ __forceinline__ int item_of(const GhostFlow& f, int w)
+        {
+            const int lane   = int(threadIdx.x & 63);
+            const bool ok    = lane < f.nitems && f.wave0[lane] <= w;
+            const uint64_t m = __ballot(ok);
+            return __builtin_amdgcn_readfirstlane(63 - __clzll(m));
+        }
+
+        // stores the mark in every ghost of the update and clears its ticket
+        __global__ __launch_bounds__(256) void k_ghost_reset(GhostFlow f, double* u, int64_t nref)
+        {
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+            {
+                *reinterpret_cast<unsigned*>(u + nref) = 0;
+            }
+            const int w = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+            if (w >= f.nwaves)
+            {
+                return;
+            }
+            const int k     = item_of(f, w);
+            const int64_t c = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
+            if (c >= f.c1[k])
+            {
+                return;
+            }
+            int64_t dst;
+            if (f.op[k] == SEQ_RECIPES)
+            {
+                dst = f.rec[4 * c];
+            }
+            else
+            {
+                const List& l  = f.op[k] == SEQ_PROJECT ? f.proj : f.pred;
+                const int64_t r = l.cellrun[c];
+                dst             = l.base[r * l.ntaps] + l.iv[5 * r] + (c - l.pref[r]);
+            }
+            u[dst] = __longlong_as_double((long long)kMark);
+        }
+
+        template <int DIM, int S>
+        __global__ __launch_bounds__(256) void k_ghost_flow(GhostFlow f, double* u, int64_t nref, double bc)
+        {
+            __shared__ unsigned ticket;
+            if (threadIdx.x == 0)
+            {
+                ticket = atomicAdd(reinterpret_cast<unsigned*>(u + nref), 1u);
+            }
+            __syncthreads();
+            const int w = __builtin_amdgcn_readfirstlane(int(ticket) * 4 + int(threadIdx.x >> 6));
+            if (w >= f.nwaves)
+            {
+                return;
+            }
+            const int k       = item_of(f, w);
+            const int64_t c   = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
+            const bool active = c < f.c1[k];
+            switch (f.op[k])
+            {
+                case SEQ_RECIPES: flow_recipe(f.rec, f.rsrc, c, active, u, bc); break;
+                case SEQ_PROJECT: flow_project<DIM>(f.proj, c, active, u); break;
+                default: flow_predict<DIM, S>(f.pred, c, active, u); break;
+            }
+        }
+    } // namespace
+
+    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s)
+    {
+        if (f.nwaves <= 0)
+        {
+            return;
+        }
+        const dim3 g(unsigned((f.nwaves + 3) / 4)), b(256);
+        hipLaunchKernelGGL(k_ghost_reset, g, b, 0, s, f, u, nref);
+        if (dim == 2 && ps == 0)
+        {
+            hipLaunchKernelGGL((k_ghost_flow<2, 0>), g, b, 0, s, f, u, nref, bc);
+        }
+        else if (dim == 2)
+        {
+            hipLaunchKernelGGL((k_ghost_flow<2, 1>), g, b, 0, s, f, u, nref, bc);
+        }
+        else if (ps == 0)
+        {
+            hipLaunchKernelGGL((k_ghost_flow<3, 0>), g, b, 0, s, f, u, nref, bc);
+        }
+        else
+        {
+            hipLaunchKernelGGL((k_ghost_flow<3, 1>), g, b, 0, s, f, u, nref, bc);
+        }
+    }
+} // namespace smr::dev

@@ -189,6 +189,121 @@ namespace smr
         *this = std::move(out);
     }
 
+    RecipeFlow build_recipe_flow(const std::vector<const Recipes*>& outer, int64_t nref)
+    {
+        RecipeFlow f;
+        f.level.assign(MAXL + 1, 0);
+        if (nref > kFlowSlots)
+        {
+            return f;
+        }
+        // per slot the last recipe that wrote it and the last one that read it
+        // unwritten, as numbers counted on from call to call, so that an old
+        // entry is never taken for one of this call
+        thread_local std::vector<uint32_t> wrote, read;
+        thread_local uint32_t base = 0;
+        size_t n = 0, ns = 0;
+        for (const Recipes* r : outer)
+        {
+            n += r->size();
+            ns += r->src.size();
+        }
+        if (ns > INT32_MAX || n > (1u << 28))
+        {
+            return f;
+        }
+        if (wrote.size() < size_t(nref) || base > (3u << 30))
+        {
+            wrote.assign(size_t(nref), 0);
+            read.assign(size_t(nref), 0);
+            base = 0;
+        }
+        const uint32_t first = base + 1;
+        std::vector<uint8_t> used, dead;
+        used.reserve(n);
+        dead.reserve(n);
+        f.rec.reserve(4 * n);
+        f.src.reserve(ns);
+        uint32_t id = base;
+        for (int l = MAXL - 1; l >= 0; --l)
+        {
+            f.level[size_t(l) + 1] = int32_t(f.rec.size() / 4);
+            if (size_t(l) >= outer.size())
+            {
+                continue;
+            }
+            const Recipes& r = *outer[size_t(l)];
+            for (size_t q = 0; q < r.size(); ++q)
+            {
+                if (r.op[q] == RECIPE_COPY_NO_BC)
+                {
+                    continue;
+                }
+                ++id;
+                const int64_t a = r.src_ptr[q], b = r.src_ptr[q + 1], d = r.dst[q];
+                for (int64_t k = a; k < b; ++k)
+                {
+                    const size_t s = size_t(r.src[size_t(k)]);
+                    if (wrote[s] >= first)
+                    {
+                        used[wrote[s] - first] = 1;
+                    }
+                    else
+                    {
+                        read[s] = id;
+                    }
+                    f.src.push_back(int32_t(s));
+                }
+                if (read[size_t(d)] >= first)
+                {
+                    base = id;
+                    return f;
+                }
+                if (wrote[size_t(d)] >= first)
+                {
+                    if (used[wrote[size_t(d)] - first])
+                    {
+                        base = id;
+                        return f;
+                    }
+                    dead[wrote[size_t(d)] - first] = 1;
+                }
+                wrote[size_t(d)] = id;
+                used.push_back(0);
+                dead.push_back(0);
+                f.rec.insert(f.rec.end(), {int32_t(d), r.op[q] | int32_t(b - a) << 8, b > a ? int32_t(r.src[size_t(a)]) : 0,
+                                           int32_t(f.src.size()) - int32_t(b - a)});
+            }
+        }
+        f.level[0] = int32_t(f.rec.size() / 4);
+        base       = id;
+        // the overwritten ones leave (their sources stay, unread)
+        if (std::find(dead.begin(), dead.end(), 1) != dead.end())
+        {
+            size_t out = 0;
+            int l      = MAXL;
+            for (size_t q = 0; q < dead.size(); ++q)
+            {
+                while (l > 0 && f.level[size_t(l)] <= int32_t(q))
+                {
+                    f.level[size_t(l--)] = int32_t(out);
+                }
+                if (!dead[q])
+                {
+                    std::copy_n(f.rec.begin() + std::ptrdiff_t(4 * q), 4, f.rec.begin() + std::ptrdiff_t(4 * out));
+                    ++out;
+                }
+            }
+            while (l >= 0)
+            {
+                f.level[size_t(l--)] = int32_t(out);
+            }
+            f.rec.resize(4 * out);
+        }
+        f.ok = true;
+        return f;
+    }
+
     namespace
     {
         void add_row_taps(WorkList& w, int8_t table, int8_t dl, int8_t dx, int lo, int hi, int dim, int8_t wlo, int8_t whi)
@@ -964,6 +1079,94 @@ namespace smr
         return "";
     }
 
+    std::string validate_recipe_flow(const std::vector<Recipes>& outer, int64_t nref)
+    {
+        std::vector<const Recipes*> levels;
+        for (const Recipes& r : outer)
+        {
+            levels.push_back(&r);
+        }
+        const RecipeFlow f = build_recipe_flow(levels, nref);
+        if (!f.ok)
+        {
+            return "";
+        }
+        // both forms on the same values, every slot compared
+        auto evaluate = [](int op, const std::vector<double>& x)
+        {
+            if (op == RECIPE_DIRICHLET)
+            {
+                return 2 * 0.25 - x[0];
+            }
+            if (op == RECIPE_AVERAGE)
+            {
+                double v = 0;
+                for (double y : x)
+                {
+                    v += y;
+                }
+                return x.empty() ? v : v / double(x.size());
+            }
+            if (op == RECIPE_EXTRAPOLATE)
+            {
+                return x.size() == 3 ? x[0] - x[1] * 3.0 + x[2] * 3.0 : x[0] - x[1] * 5.0 + x[2] * 10.0 - x[3] * 10.0 + x[4] * 5.0;
+            }
+            return x[0];
+        };
+        std::vector<double> a(static_cast<size_t>(nref));
+        for (size_t i = 0; i < a.size(); ++i)
+        {
+            a[i] = 1.0 + double((i * 2654435761u) % 1000003u) / 1000003.0;
+        }
+        std::vector<double> b = a, x;
+        for (size_t l = outer.size(); l-- > 0;)
+        {
+            const Recipes& r = outer[l];
+            for (size_t q = 0; q < r.size(); ++q)
+            {
+                if (r.op[q] != RECIPE_COPY_NO_BC)
+                {
+                    x.clear();
+                    for (int64_t k = r.src_ptr[q]; k < r.src_ptr[q + 1]; ++k)
+                    {
+                        x.push_back(a[size_t(r.src[size_t(k)])]);
+                    }
+                    a[size_t(r.dst[q])] = evaluate(r.op[q], x);
+                }
+            }
+        }
+        std::vector<char> written(size_t(nref), 0), to_write(size_t(nref), 0);
+        for (size_t q = 0; q < f.rec.size(); q += 4)
+        {
+            to_write[size_t(f.rec[q])] += 1;
+        }
+        if (f.level[0] != int32_t(f.rec.size() / 4) || f.level[MAXL] != 0)
+        {
+            return "level offsets";
+        }
+        for (size_t q = 0; q < f.rec.size(); q += 4)
+        {
+            const int n = f.rec[q + 1] >> 8;
+            x.clear();
+            for (int k = 0; k < n; ++k)
+            {
+                const size_t s = size_t(f.src[size_t(f.rec[q + 3] + k)]);
+                if (to_write[s] && !written[s])
+                {
+                    return "a source comes after its reader";
+                }
+                x.push_back(b[s]);
+            }
+            if ((n > 0 && f.rec[q + 2] != f.src[size_t(f.rec[q + 3])]) || to_write[size_t(f.rec[q])] != 1)
+            {
+                return "first source or second write";
+            }
+            b[size_t(f.rec[q])]       = evaluate(f.rec[q + 1] & 255, x);
+            written[size_t(f.rec[q])] = 1;
+        }
+        return a == b ? "" : "values differ from the staged recipes";
+    }
+
     std::string validate_programs(const MRMeshData& m)
     {
         std::string why = validate_list(build_cells_list(m), m, m);
@@ -979,6 +1182,10 @@ namespace smr
         if (!(why = validate_list(g.prediction, m, m)).empty())
         {
             return "prediction: " + why;
+        }
+        if (!(why = validate_recipe_flow(g.outer, m.nref)).empty())
+        {
+            return "recipe flow: " + why;
         }
         AdaptProgram a = build_adapt_program(m);
         if (!(why = validate_list(a.detail, m, m)).empty())

@@ -81,6 +81,23 @@ namespace smr
         bool stage_without_bc_only(size_t k) const;
     };
 
+    // The recipes of every level, finest first, for a field with a B.C. whose
+    // ghosts are written once each: a recipe whose value is overwritten before
+    // anything reads it is left out.  ok is false when a recipe reads a slot
+    // that a later recipe writes (then only the staged order gives its value).
+    // Recipes read cells and slots outside the domain only, so projections
+    // and predictions (inside) are no part of this.
+    struct RecipeFlow
+    {
+        bool ok = false;
+        std::vector<int32_t> rec;     // 4 per recipe: dst, op | n << 8, first source, first of its n sources in src
+        std::vector<int32_t> src;
+        std::vector<int32_t> level;   // recipes of level l: [level[l + 1], level[l]), MAXL + 1 entries
+    };
+    // (at most kFlowSlots slots: two words of scratch per slot and thread)
+    constexpr int64_t kFlowSlots = int64_t(1) << 21;
+    RecipeFlow build_recipe_flow(const std::vector<const Recipes*>& outer, int64_t nref);
+
     // update_ghost_mr (algorithm/update_ghost_mr.hpp:194-237) for one mesh
     struct GhostProgram
     {
@@ -130,6 +147,9 @@ namespace smr
     // Host restatement of the device resolve check: every (run, tap) row exists
     // and its access window lies in one reference run.  Returns "" or a message.
     std::string validate_list(const WorkList& w, const MRMeshData& t0, const MRMeshData& t1);
-    // validate_list over every list of the mesh's programs
+    // the recipe flow writes each slot once, after its sources, and leaves the
+    // values of the staged recipes
+    std::string validate_recipe_flow(const std::vector<Recipes>& outer, int64_t nref);
+    // validate_list over every list of the mesh's programs, and the recipe flow
     std::string validate_programs(const MRMeshData& m);
 } // namespace smr

@@ -217,6 +217,13 @@ namespace smr
         std::unique_ptr<Conv> heterogeneous;
         // the WENO5 convection terms of this image (one-level meshes of ghost width 3)
         std::unique_ptr<Conv> weno5;
+        // the dataflow form of update_ghost_mr (fields with a B.C.): the
+        // recipes, uploaded with the others, and the launch, put together on
+        // first use once the lists are in place
+        RecipeFlow recipe_flow;
+        const int32_t *flow_rec = nullptr, *flow_src = nullptr;
+        std::unique_ptr<dev::GhostFlow> ghost_flow;
+        std::unique_ptr<Blob> flow_blob;
         // launch plans of update_ghost_mr and of the tag finalization
         SeqPlan ghost_plan, max_plan;
         SeqPlan ghost_plan_nobc; // update_ghost_mr of a field without a B.C.
@@ -248,6 +255,8 @@ namespace smr
         // several lists, their host arrays prepared in parallel
         void lists(const std::vector<DevWorkList*>& ls);
         void recipes(DevRecipes& r);
+        // the dataflow form of dm's recipes (dm.outer, whose host arrays are set)
+        void recipe_flow(DevMesh& dm, int64_t nref);
         // a list whose runs, prefixes and hints the device built (at iv,
         // pref, hint); its taps come from l.host
         void device_list(DevWorkList& l, const int32_t* iv, const int64_t* pref, const int32_t* hint, int64_t nruns, int64_t ncells);
@@ -282,6 +291,10 @@ namespace smr
         void ensure_host_lists();
         void replace(MRMeshData&& m, std::unique_ptr<DevMesh>&& d);
     };
+
+    // device bytes of a field of n values: the values, then the ticket of its
+    // update_ghost_mr (dev::ghost_flow)
+    inline size_t field_bytes(int64_t n) { return (size_t(n) + 1) * sizeof(double); }
 
     struct Field
     {
