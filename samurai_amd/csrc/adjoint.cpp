@@ -17,6 +17,35 @@ namespace smr
             double w;
         };
 
+        // by source, then by output; long lists of ascending outputs by counting
+        void sort_by_source(std::vector<Triplet>& t)
+        {
+            const auto by_dst = [](const Triplet& a, const Triplet& b) { return a.dst < b.dst; };
+            if (t.size() < 64 || !std::is_sorted(t.begin(), t.end(), by_dst))
+            {
+                std::sort(t.begin(), t.end(), [](const Triplet& a, const Triplet& b) { return a.src != b.src ? a.src < b.src : a.dst < b.dst; });
+                return;
+            }
+            const auto by_src   = [](const Triplet& a, const Triplet& b) { return a.src < b.src; };
+            const auto [lo, hi] = std::minmax_element(t.begin(), t.end(), by_src);
+            const int64_t first = lo->src;
+            std::vector<size_t> at(size_t(hi->src - first) + 2, 0);
+            for (const Triplet& e : t)
+            {
+                ++at[size_t(e.src - first) + 1];
+            }
+            for (size_t k = 1; k < at.size(); ++k)
+            {
+                at[k] += at[k - 1];
+            }
+            std::vector<Triplet> out(t.size());
+            for (const Triplet& e : t)
+            {
+                out[at[size_t(e.src - first)]++] = e;
+            }
+            t.swap(out);
+        }
+
         LinearStage make_stage(std::vector<int64_t>&& dst, std::vector<Triplet>& t, int64_t nref)
         {
             for (int64_t d : dst)
@@ -35,7 +64,7 @@ namespace smr
             }
             LinearStage st;
             st.dst = std::move(dst);
-            std::sort(t.begin(), t.end(), [](const Triplet& a, const Triplet& b) { return a.src != b.src ? a.src < b.src : a.dst < b.dst; });
+            sort_by_source(t);
             for (size_t i = 0; i < t.size();)
             {
                 size_t j = i;
@@ -381,13 +410,45 @@ namespace smr
         {
             throw std::invalid_argument("adjoint: two instances share a mesh");
         }
-        // transposed ghost stages and the ghost-neighbour scatter lists, built in parallel
+        // the ghost update as linear stages, built in parallel
+        parallel_for(int(inst_.size()),
+                     [&](int i)
+                     {
+                         Instance& in = inst_[size_t(i)];
+                         in.ghost     = ghost_linear_stages(in.mesh->host, *in.mesh->dev, in.has_bc);
+                     });
+        // the per-cell velocity-gradient terms of all instances, one array
+        ga_off_.assign(inst_.size() + 1, 0);
+        for (size_t i = 0; i < inst_.size(); ++i)
+        {
+            ga_off_[i + 1] = ga_off_[i] + inst_[i].ncells * inst_[i].mesh->host.cfg.dim;
+        }
+        ga_arena_ = static_cast<double*>(dev_alloc(size_t(std::max<int64_t>(ga_off_.back(), 1)) * 8, ctx_->stream));
+        for (size_t i = 0; i < inst_.size(); ++i)
+        {
+            inst_[i].ga = ga_arena_ + ga_off_[i];
+        }
+        flow_ = make_flow();
+        if (!flow_)
+        {
+            prepare_programs();
+        }
+    }
+
+    // the lists and arrays of the stage programs
+    void Adjoint::prepare_programs()
+    {
+        if (programs_built_)
+        {
+            return;
+        }
+        programs_built_ = true;
+        // the reverse stages and the ghost-neighbour scatter lists, built in parallel
         parallel_for(int(inst_.size()),
                      [&](int i)
                      {
                          Instance& in  = inst_[size_t(i)];
                          const auto& m = in.mesh->host;
-                         in.ghost      = ghost_linear_stages(m, *in.mesh->dev, in.has_bc);
                          in.adj_groups = group_reverse_stages(in.ghost);
                          const std::array<std::array<int, 3>, 6> offs = {
                              {{-1, 0, 0}, {1, 0, 0}, {0, -1, 0}, {0, 1, 0}, {0, 0, -1}, {0, 0, 1}}};
@@ -469,17 +530,6 @@ namespace smr
             // the first ghost update writes them only by the copies, never by operators)
             hip_check(hipMemsetAsync(in.states, 0, n * size_t(every_ + 1) * 8, st), "hipMemsetAsync(states)");
         }
-        // the per-cell velocity-gradient terms of all instances, one array
-        ga_off_.assign(inst_.size() + 1, 0);
-        for (size_t i = 0; i < inst_.size(); ++i)
-        {
-            ga_off_[i + 1] = ga_off_[i] + inst_[i].ncells * inst_[i].mesh->host.cfg.dim;
-        }
-        ga_arena_ = static_cast<double*>(dev_alloc(size_t(std::max<int64_t>(ga_off_.back(), 1)) * 8, st));
-        for (size_t i = 0; i < inst_.size(); ++i)
-        {
-            inst_[i].ga = ga_arena_ + ga_off_[i];
-        }
         ctx_->check_resolve();
     }
 
@@ -534,7 +584,19 @@ namespace smr
                 inst_[i].a[d] = a[3 * i + size_t(d)];
             }
         }
-        programs_ready_ = false;
+        programs_ready_ = forward_done_ = false;
+        if (flow_)
+        {
+            std::vector<dev::FlowParam> p(inst_.size());
+            for (size_t i = 0; i < inst_.size(); ++i)
+            {
+                const Instance& in = inst_[i];
+                p[i]               = {{in.a[0], in.a[1], in.mesh->host.cfg.dim == 3 ? in.a[2] : 0.0}, in.dt, in.bc};
+            }
+            hip_check(hipMemcpyAsync(flow_->params.p, p.data(), p.size() * sizeof(p[0]), hipMemcpyHostToDevice, ctx_->stream),
+                      "hipMemcpyAsync(velocity)");
+            ctx_->sync(); // p leaves
+        }
     }
 
     std::unique_ptr<ProgramBuf> Adjoint::make_program(const std::vector<Chain>& chains)
@@ -548,6 +610,7 @@ namespace smr
     void Adjoint::build_programs()
     {
         const size_t n = inst_.size();
+        prepare_programs();
         fseg_.clear();
         bseg_.clear();
         // the chains of every piece (one forward step, one adjoint step of each
@@ -790,6 +853,14 @@ namespace smr
     void Adjoint::forward(const double* u0, double* uT)
     {
         check_meshes();
+        if (flow_)
+        {
+            ScopedTimer t(ctx_, "adjoint forward");
+            flow_forward(u0, uT);
+            ctx_->sync();
+            forward_done_ = true;
+            return;
+        }
         if (!programs_ready_)
         {
             build_programs();
@@ -808,9 +879,16 @@ namespace smr
     void Adjoint::backward(const double* gT, double* g0, double* ga)
     {
         check_meshes();
-        if (!programs_ready_)
+        if (flow_ ? !forward_done_ : !programs_ready_)
         {
             throw std::logic_error("adjoint: backward before forward");
+        }
+        if (flow_)
+        {
+            ScopedTimer t(ctx_, "adjoint backward");
+            flow_backward(gT, g0);
+            sum_velocity_gradient(ga);
+            return;
         }
         bind_io(nullptr, nullptr, gT, g0);
         ScopedTimer t(ctx_, "adjoint backward");
@@ -820,6 +898,11 @@ namespace smr
             bseg_[size_t(sg)]->run(tuning_);
         }
         grad_out_->run(tuning_);
+        sum_velocity_gradient(ga);
+    }
+
+    void Adjoint::sum_velocity_gradient(double* ga)
+    {
         // velocity gradient: per-cell terms of all instances in one copy, summed
         // on the host per instance in cell order
         const size_t total = size_t(ga_off_.back());
@@ -850,5 +933,513 @@ namespace smr
                              ga[3 * i + size_t(d)] = d < dim ? acc[d] : 0.0;
                          }
                      });
+    }
+
+    // ------------------------------------------------------------------
+    // the dataflow form
+    // ------------------------------------------------------------------
+    namespace
+    {
+        // the operations of one instance; slots local to its storage
+        struct FlowTables
+        {
+            bool ok = false;
+            std::vector<uint8_t> kind;
+            RecipeFlow recipes;
+            std::array<std::vector<int32_t>, MAXL> proj, pred; // per level of the ghosts
+            std::vector<int32_t> cell;
+            // the adjoint's ghosts by the number of stages after theirs
+            std::vector<std::vector<int32_t>> ghosts;
+            std::vector<std::array<int32_t, 6>> beside; // per slot of a ghost beside cells: those cells
+            std::vector<int32_t> beside_at;             // per slot: its entry in beside, or -1
+            std::vector<int8_t> slot_level;
+            // entries of slot s: [start[s], start[s + 1]) of (source, sign bit: last of its stage) and weight
+            std::vector<int32_t> start, esrc;
+            std::vector<double> ew;
+        };
+
+        FlowTables flow_tables(const MRMeshData& m, const DevMesh& dm, const std::vector<LinearStage>& stages)
+        {
+            const int dim = m.cfg.dim, s = m.cfg.pred_s;
+            FlowTables t;
+            std::vector<const Recipes*> outer;
+            for (const DevRecipes& r : dm.outer)
+            {
+                outer.push_back(&r.host);
+            }
+            t.recipes = build_recipe_flow(outer, m.nref);
+            if (!t.recipes.ok)
+            {
+                return t;
+            }
+            const size_t n = size_t(m.nref);
+            t.kind.assign(n, 0);
+            t.slot_level.assign(n, 0);
+            auto runs_of = [](const WorkList& w, int level, auto&& f)
+            {
+                int64_t r0       = 0;
+                const int64_t nr = w.runs_of_levels(level, level + 1, r0);
+                for (int64_t k = r0; k < r0 + nr; ++k)
+                {
+                    f(&w.iv[size_t(5 * k)]);
+                }
+            };
+            for (int level = 0; level < MAXL; ++level)
+            {
+                auto& pj = t.proj[size_t(level)];
+                runs_of(dm.projection.host,
+                        level,
+                        [&](const int32_t* iv)
+                        {
+                            const int32_t x0 = iv[0], x1 = iv[1], y = iv[2], z = iv[3];
+                            const int nrows  = 1 << (dim - 1);
+                            const int64_t bd = row_base(m, level, x0, y, z);
+                            int64_t bf[4]    = {};
+                            for (int q = 0; q < nrows; ++q)
+                            {
+                                bf[q] = row_base(m, level + 1, 2 * x0, 2 * y + (q & 1), 2 * z + (q >> 1));
+                            }
+                            for (int32_t x = x0; x < x1; ++x)
+                            {
+                                const size_t at = pj.size();
+                                pj.resize(at + (dim == 2 ? 4 : 8), 0);
+                                pj[at] = int32_t(bd + x);
+                                for (int q = 0; q < nrows; ++q)
+                                {
+                                    pj[at + 1 + size_t(q)] = int32_t(bf[q] + 2 * x);
+                                }
+                            }
+                        });
+                auto& pr = t.pred[size_t(level)];
+                runs_of(dm.prediction.host,
+                        level,
+                        [&](const int32_t* iv)
+                        {
+                            const int32_t x0 = iv[0], x1 = iv[1], y = iv[2], z = iv[3];
+                            const int ny = 2 * s + 1, nz = dim == 3 ? ny : 1;
+                            const size_t words = s == 0 ? 2 : (dim == 2 ? 4 : 12);
+                            const int64_t bd   = row_base(m, level, x0, y, z);
+                            int64_t bc[9]      = {};
+                            for (int q = 0; q < nz * ny; ++q)
+                            {
+                                bc[q] = row_base(m, level - 1, (x0 >> 1) - s, (y >> 1) + q % ny - s, dim == 3 ? (z >> 1) + q / ny - s : 0);
+                            }
+                            for (int32_t x = x0; x < x1; ++x)
+                            {
+                                const size_t at = pr.size();
+                                pr.resize(at + words, 0);
+                                pr[at] = int32_t(bd + x) | (x & 1) << 28 | (y & 1) << 29 | (z & 1) << 30;
+                                for (int q = 0; q < nz * ny; ++q)
+                                {
+                                    pr[at + 1 + size_t(q)] = int32_t(bc[q] + (x >> 1) - s);
+                                }
+                            }
+                        });
+            }
+            // the ghosts by their last stage (an earlier write is overwritten unread)
+            const int nst = int(stages.size());
+            std::vector<int32_t> stage_of(n, -1);
+            for (int k = 0; k < nst; ++k)
+            {
+                for (int64_t d : stages[size_t(k)].dst)
+                {
+                    stage_of[size_t(d)] = k;
+                    t.kind[size_t(d)]   = 2;
+                }
+            }
+            t.ghosts.resize(size_t(nst));
+            for (size_t d = 0; d < n; ++d)
+            {
+                if (stage_of[d] >= 0)
+                {
+                    t.ghosts[size_t(nst - 1 - stage_of[d])].push_back(int32_t(d));
+                }
+            }
+            // the cells
+            const WorkList& cells = dm.cells.host;
+            for (int64_t k = 0; k < cells.nruns(); ++k)
+            {
+                const int32_t* iv = &cells.iv[size_t(5 * k)];
+                const int64_t b   = row_base(m, iv[4], iv[0], iv[2], iv[3]);
+                std::fill(t.kind.begin() + b + iv[0], t.kind.begin() + b + iv[1], uint8_t(1));
+            }
+            t.beside_at.assign(n, -1);
+            const size_t words = dim == 2 ? 4 : 8;
+            t.cell.reserve(words * size_t(cells.ncells()));
+            for (int64_t k = 0; k < cells.nruns(); ++k)
+            {
+                const int32_t* iv = &cells.iv[size_t(5 * k)];
+                const int32_t x0 = iv[0], x1 = iv[1], y = iv[2], z = iv[3];
+                const int level  = iv[4];
+                const int64_t b  = row_base(m, level, x0, y, z);
+                int64_t rows[4]  = {row_base(m, level, x0, y - 1, z), row_base(m, level, x0, y + 1, z), 0, 0};
+                if (dim == 3)
+                {
+                    rows[2] = row_base(m, level, x0, y, z - 1);
+                    rows[3] = row_base(m, level, x0, y, z + 1);
+                }
+                for (int32_t x = x0; x < x1; ++x)
+                {
+                    const int64_t own = b + x;
+                    int32_t word      = level;
+                    for (int d = 0; d < 2 * dim; ++d)
+                    {
+                        const size_t nb = size_t(d < 2 ? own + 2 * d - 1 : rows[d - 2] + x);
+                        if (t.kind[nb] != 1)
+                        {
+                            word |= 1 << (5 + d);
+                            if (t.kind[nb] == 2)
+                            {
+                                if (t.beside_at[nb] < 0)
+                                {
+                                    t.beside_at[nb] = int32_t(t.beside.size());
+                                    t.beside.push_back({-1, -1, -1, -1, -1, -1});
+                                }
+                                t.beside[size_t(t.beside_at[nb])][size_t(d)] = int32_t(own);
+                                t.slot_level[nb]                             = int8_t(level);
+                            }
+                        }
+                    }
+                    const size_t at = t.cell.size();
+                    t.cell.resize(at + words, 0);
+                    t.cell[at] = int32_t(own);
+                    for (int q = 0; q < 2 * dim - 2; ++q)
+                    {
+                        t.cell[at + 1 + size_t(q)] = int32_t(rows[q] + x);
+                    }
+                    t.cell[at + (dim == 2 ? 3 : 5)] = word;
+                }
+            }
+            // the transposed stages, last first, without the overwritten writes
+            t.start.assign(n + 1, 0);
+            auto each = [&](auto&& f)
+            {
+                for (int k = nst - 1; k >= 0; --k)
+                {
+                    const LinearStage& g = stages[size_t(k)];
+                    for (size_t r = 0; r < g.tgt.size(); ++r)
+                    {
+                        int64_t last = -1;
+                        for (int64_t e = g.ptr[r]; e < g.ptr[r + 1]; ++e)
+                        {
+                            last = stage_of[size_t(g.src[size_t(e)])] == k ? e : last;
+                        }
+                        for (int64_t e = g.ptr[r]; e <= last; ++e)
+                        {
+                            if (stage_of[size_t(g.src[size_t(e)])] == k)
+                            {
+                                f(size_t(g.tgt[r]), int32_t(g.src[size_t(e)]), g.w[size_t(e)], e == last);
+                            }
+                        }
+                    }
+                }
+            };
+            each([&](size_t slot, int32_t, double, bool) { ++t.start[slot + 1]; });
+            for (size_t i = 0; i < n; ++i)
+            {
+                t.start[i + 1] += t.start[i];
+            }
+            std::vector<int32_t> at(t.start.begin(), t.start.end() - 1);
+            t.esrc.resize(size_t(t.start[n]));
+            t.ew.resize(size_t(t.start[n]));
+            each(
+                [&](size_t slot, int32_t src, double w, bool last)
+                {
+                    const size_t e = size_t(at[slot]++);
+                    t.esrc[e]      = last ? int32_t(uint32_t(src) | 0x80000000u) : src;
+                    t.ew[e]        = w;
+                });
+            t.ok = true;
+            return t;
+        }
+    } // namespace
+
+    std::unique_ptr<Adjoint::Flow> Adjoint::make_flow()
+    {
+        if (inst_.empty() || inst_.size() >= (size_t(1) << 20))
+        {
+            return nullptr;
+        }
+        const MeshConfig& c0 = inst_[0].mesh->host.cfg;
+        int64_t n = 0, ncells = 0;
+        for (const Instance& in : inst_)
+        {
+            const MeshConfig& c = in.mesh->host.cfg;
+            if (!in.has_bc || c.dim != c0.dim || c.pred_s != c0.pred_s)
+            {
+                return nullptr;
+            }
+            n += in.nref;
+            ncells += in.ncells;
+        }
+        if (n > dev::kFlowSlotMask || ncells == 0)
+        {
+            return nullptr;
+        }
+        std::vector<FlowTables> ts(inst_.size());
+        parallel_for(int(inst_.size()),
+                     [&](int i)
+                     {
+                         const Instance& in = inst_[size_t(i)];
+                         ts[size_t(i)]      = flow_tables(in.mesh->host, *in.mesh->dev, in.ghost);
+                     });
+        std::vector<int64_t> slot0(inst_.size() + 1, 0);
+        size_t nent = 0, nranks = 0;
+        for (size_t i = 0; i < ts.size(); ++i)
+        {
+            if (!ts[i].ok)
+            {
+                return nullptr;
+            }
+            slot0[i + 1] = slot0[i] + inst_[i].nref;
+            nent += ts[i].esrc.size();
+            nranks = std::max(nranks, ts[i].ghosts.size());
+        }
+        if (nent > size_t(INT32_MAX))
+        {
+            return nullptr;
+        }
+        auto flow          = std::make_unique<Flow>();
+        dev::AdjointFlow& f = flow->f;
+        f.dim              = c0.dim;
+        f.ps               = c0.pred_s;
+        f.n                = n;
+        f.ncells           = ncells;
+        std::vector<uint8_t> kind;
+        std::vector<int32_t> rec, rsrc, proj, pred, cell, aghost, rowptr{0}, esrc;
+        std::vector<double> ew;
+        kind.reserve(size_t(n));
+        // one step's items: per level the recipes and the projection of all
+        // instances, then the predictions, then the cells
+        int64_t waves = 0;
+        auto item     = [&](int op, size_t words, const std::vector<int32_t>& all, size_t from)
+        {
+            if (all.size() > from)
+            {
+                const int k = f.nitems++;
+                f.op[k]     = op;
+                f.c0[k]     = int32_t(from / words);
+                f.c1[k]     = int32_t(all.size() / words);
+                f.wave0[k]  = int32_t(waves);
+                waves += int64_t(f.c1[k] - f.c0[k] + 63) / 64;
+            }
+        };
+        // appends the records, their slot words (all but `keep` at the end) moved to the instance's storage
+        auto append = [&](std::vector<int32_t>& all, const std::vector<int32_t>& one, size_t words, size_t nslots, int32_t by)
+        {
+            const size_t at = all.size();
+            all.insert(all.end(), one.begin(), one.end());
+            for (size_t q = at; q < all.size(); q += words)
+            {
+                for (size_t k = 0; k < nslots; ++k)
+                {
+                    all[q + k] += by;
+                }
+            }
+        };
+        const size_t jw = c0.dim == 2 ? 4 : 8, pw = c0.pred_s == 0 ? 2 : (c0.dim == 2 ? 4 : 12), cw = c0.dim == 2 ? 4 : 8;
+        const size_t nrow = c0.dim == 2 ? 2 : 4, npred = c0.pred_s == 0 ? 1 : (c0.dim == 2 ? 3 : 9);
+        std::vector<int32_t> src_at(ts.size());
+        for (size_t i = 0; i < ts.size(); ++i)
+        {
+            kind.insert(kind.end(), ts[i].kind.begin(), ts[i].kind.end());
+            src_at[i] = int32_t(rsrc.size());
+            for (int32_t v : ts[i].recipes.src)
+            {
+                rsrc.push_back(v + int32_t(slot0[i]));
+            }
+        }
+        for (int level = MAXL - 1; level >= 0; --level)
+        {
+            size_t from = rec.size();
+            for (size_t i = 0; i < ts.size(); ++i)
+            {
+                const RecipeFlow& r = ts[i].recipes;
+                for (int32_t q = r.level[size_t(level) + 1]; q < r.level[size_t(level)]; ++q)
+                {
+                    const int32_t* v = &r.rec[size_t(4 * q)];
+                    const bool one   = (v[1] & 255) == RECIPE_DIRICHLET;
+                    rec.insert(rec.end(), {v[0] + int32_t(slot0[i]), v[1], v[2] + int32_t(slot0[i]), one ? int32_t(i) : v[3] + src_at[i]});
+                }
+            }
+            item(dev::FLOW_RECIPES, 4, rec, from);
+            if (level > 0)
+            {
+                from = proj.size();
+                for (size_t i = 0; i < ts.size(); ++i)
+                {
+                    append(proj, ts[i].proj[size_t(level) - 1], jw, 1 + nrow, int32_t(slot0[i]));
+                }
+                item(dev::FLOW_PROJECT, jw, proj, from);
+            }
+        }
+        for (int level = 1; level < MAXL; ++level)
+        {
+            const size_t from = pred.size();
+            for (size_t i = 0; i < ts.size(); ++i)
+            {
+                append(pred, ts[i].pred[size_t(level)], pw, 1 + npred, int32_t(slot0[i]));
+            }
+            item(dev::FLOW_PREDICT, pw, pred, from);
+        }
+        for (size_t i = 0; i < ts.size(); ++i)
+        {
+            const size_t at = cell.size();
+            append(cell, ts[i].cell, cw, 1 + nrow, int32_t(slot0[i]));
+            for (size_t q = at + (c0.dim == 2 ? 3 : 5); q < cell.size(); q += cw)
+            {
+                cell[q] |= int32_t(i) << 11;
+            }
+        }
+        item(dev::FLOW_UPWIND, cw, cell, 0);
+        f.nwaves = int(waves);
+        // the adjoint's operations: the ghosts, last stage first, then the
+        // cells; first their places, then their records and entries
+        struct Place
+        {
+            int32_t inst, slot;
+        };
+        std::vector<Place> ghosts;
+        for (size_t rank = 0; rank < nranks; ++rank)
+        {
+            for (size_t i = 0; i < ts.size(); ++i)
+            {
+                if (rank < ts[i].ghosts.size())
+                {
+                    for (int32_t d : ts[i].ghosts[rank])
+                    {
+                        ghosts.push_back({int32_t(i), d});
+                    }
+                }
+            }
+        }
+        f.naghost = int64_t(ghosts.size());
+        rowptr.resize(ghosts.size() + size_t(ncells) + 1);
+        auto count = [&](size_t q, size_t i, size_t slot) { rowptr[q + 1] = rowptr[q] + ts[i].start[slot + 1] - ts[i].start[slot]; };
+        for (size_t q = 0; q < ghosts.size(); ++q)
+        {
+            count(q, size_t(ghosts[q].inst), size_t(ghosts[q].slot));
+        }
+        size_t row = ghosts.size();
+        for (size_t i = 0; i < ts.size(); ++i)
+        {
+            for (size_t q = 0; q < ts[i].cell.size(); q += cw)
+            {
+                count(row++, i, size_t(ts[i].cell[q]));
+            }
+        }
+        aghost.resize(8 * ghosts.size());
+        esrc.resize(size_t(rowptr.back()));
+        ew.resize(size_t(rowptr.back()));
+        auto entries = [&](size_t q, size_t i, size_t slot)
+        {
+            size_t to = size_t(rowptr[q]);
+            for (int32_t e = ts[i].start[slot]; e < ts[i].start[slot + 1]; ++e, ++to)
+            {
+                esrc[to] = ts[i].esrc[size_t(e)] + int32_t(slot0[i]);
+                ew[to]   = ts[i].ew[size_t(e)];
+            }
+        };
+        constexpr size_t kChunk = 4096;
+        const int ngc           = int((ghosts.size() + kChunk - 1) / kChunk);
+        parallel_for(ngc + int(ts.size()),
+                     [&](int job)
+                     {
+                         if (job >= ngc)
+                         {
+                             const size_t i = size_t(job - ngc);
+                             size_t q       = ghosts.size() + size_t(inst_[i].off);
+                             for (size_t k = 0; k < ts[i].cell.size(); k += cw)
+                             {
+                                 entries(q++, i, size_t(ts[i].cell[k]));
+                             }
+                             return;
+                         }
+                         for (size_t q = size_t(job) * kChunk; q < std::min(ghosts.size(), size_t(job + 1) * kChunk); ++q)
+                         {
+                             const size_t i = size_t(ghosts[q].inst), d = size_t(ghosts[q].slot);
+                             const int32_t b = ts[i].beside_at[d];
+                             int32_t* v      = &aghost[8 * q];
+                             v[0]            = int32_t(d) + int32_t(slot0[i]);
+                             v[1]            = int32_t(ts[i].slot_level[d]) | int32_t(i) << 5;
+                             for (size_t k = 0; k < 6; ++k)
+                             {
+                                 const int32_t c = b < 0 ? -1 : ts[i].beside[size_t(b)][k];
+                                 v[2 + k]        = c < 0 ? -1 : c + int32_t(slot0[i]);
+                             }
+                             entries(q, i, d);
+                         }
+                     });
+        ts.clear();
+        hipStream_t st      = ctx_->stream;
+        Blob& b             = flow->tables;
+        const size_t o_kind = b.add(std::move(kind)), o_rec = b.add(std::move(rec)), o_rsrc = b.add(std::move(rsrc)), o_proj = b.add(std::move(proj)),
+                     o_pred = b.add(std::move(pred)), o_cell = b.add(std::move(cell)), o_gh = b.add(std::move(aghost)), o_rp = b.add(std::move(rowptr)),
+                     o_es = b.add(std::move(esrc)), o_ew = b.add(std::move(ew));
+        b.upload(st);
+        auto i32 = [&](size_t o) { return reinterpret_cast<const int32_t*>(b.dptr(o)); };
+        f.kind   = reinterpret_cast<const uint8_t*>(b.dptr(o_kind));
+        f.rec    = i32(o_rec);
+        f.rsrc   = i32(o_rsrc);
+        f.proj   = i32(o_proj);
+        f.pred   = i32(o_pred);
+        f.cell   = i32(o_cell);
+        f.aghost = i32(o_gh);
+        f.rowptr = i32(o_rp);
+        f.esrc   = i32(o_es);
+        f.ew     = reinterpret_cast<const double*>(b.dptr(o_ew));
+        f.par    = static_cast<const dev::FlowParam*>(flow->params.get(inst_.size() * sizeof(dev::FlowParam), st));
+        flow->ticket.get(256, st);
+        const int between   = std::min(every_, kFlowSteps) - 1;
+        const size_t narr   = size_t(nseg_ + 1 + every_ - 1 + 2 + between);
+        flow->ckpt          = static_cast<double*>(flow->arrays.get(narr * size_t(n) * 8, st));
+        flow->states        = flow->ckpt + int64_t(nseg_ + 1) * n;
+        flow->ends          = flow->states + int64_t(every_ - 1) * n;
+        flow->between       = flow->ends + 2 * n;
+        // slots that no cell and no update writes are read as zero
+        hip_check(hipMemsetAsync(flow->ckpt, 0, narr * size_t(n) * 8, st), "hipMemsetAsync(adjoint arrays)");
+        hip_check(hipMemsetAsync(flow->params.p, 0, inst_.size() * sizeof(dev::FlowParam), st), "hipMemsetAsync(adjoint parameters)");
+        return flow;
+    }
+
+    void Adjoint::flow_forward(const double* u0, double* uT)
+    {
+        Flow& w       = *flow_;
+        hipStream_t s = ctx_->stream;
+        auto* ticket  = static_cast<unsigned*>(w.ticket.p);
+        dev::adjoint_flow_cells(w.f, w.ckpt, const_cast<double*>(u0), false, s);
+        for (int sg = 0; sg < nseg_; ++sg)
+        {
+            double* at = w.ckpt + int64_t(sg) * w.f.n;
+            dev::adjoint_flow_forward(w.f, {at, w.states, at + w.f.n, every_}, true, ticket, s);
+        }
+        dev::adjoint_flow_cells(w.f, w.ckpt + int64_t(nseg_) * w.f.n, uT, true, s);
+    }
+
+    void Adjoint::flow_backward(const double* gT, double* g0)
+    {
+        Flow& w       = *flow_;
+        hipStream_t s = ctx_->stream;
+        auto* ticket  = static_cast<unsigned*>(w.ticket.p);
+        double* end[2] = {w.ends, w.ends + w.f.n};
+        int cur        = 0;
+        dev::adjoint_flow_cells(w.f, end[cur], const_cast<double*>(gT), false, s);
+        dev::zero_f64(ga_arena_, ga_off_.back(), s);
+        for (int sg = nseg_ - 1; sg >= 0; --sg)
+        {
+            double* at = w.ckpt + int64_t(sg) * w.f.n;
+            const dev::FlowArrays states{at, w.states, at + w.f.n, every_};
+            dev::adjoint_flow_forward(w.f, states, false, ticket, s);
+            for (int done = 0; done < every_;)
+            {
+                const int k = std::min(kFlowSteps, every_ - done);
+                const dev::FlowArrays lam{end[cur], w.between, end[1 - cur], k};
+                dev::adjoint_flow_backward(w.f, lam, ticket, s);
+                dev::adjoint_flow_velocity(w.f, lam, states, every_ - 1 - done, ga_arena_, s);
+                done += k;
+                cur = 1 - cur;
+            }
+        }
+        dev::adjoint_flow_cells(w.f, end[cur], g0, true, s);
     }
 } // namespace smr

@@ -10,9 +10,12 @@
 // transposed (target <- sources) lists followed by zeroing its outputs.  The
 // velocity gradient accumulates lam_{n+1} . dU/da (u_n) per cell.
 //
-// Many instances are advanced together with the batched stage programs; the
-// forward pass keeps a checkpoint every `every` steps and the backward pass
-// recomputes each segment from its checkpoint before running it backwards.
+// Many instances are advanced together; the forward pass keeps a checkpoint
+// every `every` steps and the backward pass recomputes each segment from its
+// checkpoint before running it backwards.  A segment is one dataflow launch
+// (dev::AdjointFlow) where every instance has a B.C. and a recipe flow and all
+// share the dimension and the prediction radius; the others, and problems
+// given a launch shape by set_tuning, run the batched stage programs.
 #pragma once
 
 #include "batch.hpp"
@@ -63,7 +66,12 @@ namespace smr
         void forward(const double* u0, double* uT);
         // gT = dL/duT -> g0 = dL/du0 (device), ga = dL/da (host, n*3)
         void backward(const double* gT, double* g0, double* ga);
-        void set_tuning(const Tuning& t) { tuning_ = t; }
+        // selects the stage programs, in that launch shape
+        void set_tuning(const Tuning& t)
+        {
+            tuning_ = t;
+            flow_   = nullptr;
+        }
         const Tuning& tuning() const { return tuning_; }
         int steps() const { return steps_; }
         int every() const { return every_; }
@@ -124,6 +132,26 @@ namespace smr
         std::vector<int64_t> ga_off_;
         PinnedStaging ga_host_;
 
+        // the dataflow form: its tables and arrays, null when it does not apply
+        struct Flow
+        {
+            dev::AdjointFlow f{};
+            Blob tables;
+            DevBuffer arrays, params, ticket;
+            // nseg + 1 checkpoints, every - 1 states, two arrays at the ends of
+            // an adjoint launch and kFlowSteps - 1 between
+            double *ckpt = nullptr, *states = nullptr, *ends = nullptr, *between = nullptr;
+        };
+        // adjoint steps per launch (their arrays are all in memory)
+        static constexpr int kFlowSteps = 16;
+        std::unique_ptr<Flow> flow_;
+        bool forward_done_   = false; // with the velocity set last
+        bool programs_built_ = false; // the lists and arrays of the stage programs
+        std::unique_ptr<Flow> make_flow();
+        void prepare_programs();
+        void flow_forward(const double* u0, double* uT);
+        void flow_backward(const double* gT, double* g0);
+        void sum_velocity_gradient(double* ga);
         void check_meshes() const;
         void build_programs();
         void bind_io(const double* u0, double* uT, const double* gT, double* g0);

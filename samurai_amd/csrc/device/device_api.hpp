@@ -364,6 +364,64 @@ namespace smr::dev
     };
     void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s);
 
+    // Frozen-mesh steps of many instances and their adjoint as dataflow
+    // launches (adjoint_flow.hip).  Slots number the storages of all instances
+    // one after the other, n in all (below 2^28).
+    enum FlowOp : int32_t
+    {
+        FLOW_RECIPES = 0,
+        FLOW_PROJECT = 1,
+        FLOW_PREDICT = 2,
+        FLOW_UPWIND  = 3
+    };
+    constexpr int32_t kFlowSlotMask = (1 << 28) - 1;
+    struct FlowParam
+    {
+        double a[3], dt, bc;
+    };
+    struct AdjointFlow
+    {
+        int dim, ps;
+        int64_t n, ncells, naghost;
+        const uint8_t* kind; // per slot: 1 cell, 2 ghost that an update writes, else 0
+        // recipes as in GhostFlow (a Dirichlet recipe's last word is its instance)
+        const int32_t *rec, *rsrc;
+        // projections: dst, the fine rows at 2x (4 words in 2D, 8 in 3D)
+        const int32_t* proj;
+        // predictions: dst | parities << 28, the coarse rows at (x >> 1) - s
+        // (2 words for s = 0, 4 in 2D, 12 in 3D)
+        const int32_t* pred;
+        // cells: own slot, the neighbouring rows at x, level | ghost
+        // neighbours << 5 | instance << 11 (4 words in 2D, 8 in 3D)
+        const int32_t* cell;
+        // ghosts in an order of the adjoint: dst, level | instance << 5, then
+        // the cell whose x-1, x+1, y-1, ... neighbour the ghost is, or -1
+        const int32_t* aghost;
+        // entries of operation q (the ghosts, then the cells): source slot,
+        // the sign bit on the last of a stage; weight
+        const int32_t *rowptr, *esrc;
+        const double* ew;
+        const FlowParam* par; // per instance
+        // the items of one step, as in GhostFlow
+        int nitems, nwaves;
+        int32_t wave0[kFlowItems], c0[kFlowItems], c1[kFlowItems], op[kFlowItems];
+    };
+    // the steps + 1 arrays of n slots a launch works on
+    struct FlowArrays
+    {
+        double *first, *between, *last;
+        int steps;
+    };
+    void adjoint_flow_cells(const AdjointFlow& f, double* array, double* compact, bool to_compact, hipStream_t s);
+    // a.steps time steps from the cells of the first array; with `last` the
+    // cells of the last array are computed too
+    void adjoint_flow_forward(const AdjointFlow& f, const FlowArrays& a, bool last, unsigned* ticket, hipStream_t s);
+    // a.steps adjoint steps from the cells of the first array to the last's
+    void adjoint_flow_backward(const AdjointFlow& f, const FlowArrays& a, unsigned* ticket, hipStream_t s);
+    // adds the velocity-gradient terms of the adjoint steps of lam to ga (dim
+    // per cell): step j with state st0 - j of st
+    void adjoint_flow_velocity(const AdjointFlow& f, const FlowArrays& lam, const FlowArrays& st, int st0, double* ga, hipStream_t s);
+
     struct Segment
     {
         int32_t op, dim, pred_s, has_bc;

@@ -25,90 +25,12 @@
 // the lowest unfinished wave waits for nothing that is not done; and a wave
 // gives up after kMaxSpins rounds and uses what it has read (which is the
 // right value when a cell itself holds the bits of the mark).
-#include "cell_ops.hpp"
+#include "flow_ops.hpp"
 
 namespace smr::dev
 {
     namespace
     {
-        // a signalling NaN: arithmetic results are never signalling, and a
-        // copied value with these very bits is stored quiet
-        constexpr unsigned long long kMark = 0x7FF05A3C96E1D2B4ull;
-        constexpr unsigned long long kQuiet = 0x0008000000000000ull;
-        constexpr int kMaxSpins            = 1 << 17;
-
-        __device__ __forceinline__ bool marked(double v)
-        {
-            return (unsigned long long)__double_as_longlong(v) == kMark;
-        }
-
-        // the first look at a source: any cache may answer, since a line that
-        // is out of date holds the mark
-        __device__ __forceinline__ double look(const double* p)
-        {
-            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-
-        __device__ __forceinline__ double look_again(const double* p)
-        {
-            return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-
-        __device__ __forceinline__ void publish(double* p, double v)
-        {
-            if (marked(v))
-            {
-                v = __longlong_as_double((long long)(kMark | kQuiet));
-            }
-            __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-
-        // runs attempt(last) on the lanes not yet done until all of them are:
-        // it returns true once the lane has published (always when last)
-        template <class F>
-        __device__ __forceinline__ void until_done(bool active, F&& attempt)
-        {
-            bool done = !active;
-            for (int spin = 0; !__all(done); ++spin)
-            {
-                if (!done)
-                {
-                    done = attempt(spin >= kMaxSpins);
-                }
-            }
-        }
-
-        // N sources held in registers; true when none of them is marked
-        template <int N, class Addr>
-        struct Sources
-        {
-            double v[N];
-            bool fresh = true;
-            __device__ __forceinline__ bool ready(const Addr& at)
-            {
-                bool ok = true;
-#pragma unroll
-                for (int k = 0; k < N; ++k)
-                {
-                    if (fresh)
-                    {
-                        v[k] = look(at(k));
-                    }
-                    else if (marked(v[k]))
-                    {
-                        v[k] = look_again(at(k));
-                    }
-                }
-#pragma unroll
-                for (int k = 0; k < N; ++k)
-                {
-                    ok = ok && !marked(v[k]);
-                }
-                fresh = false;
-                return ok;
-            }
-        };
-
         // projection_op_ (op_project_at) on waited-for sources
         template <int DIM>
         __device__ __forceinline__ void flow_project(const List& l, int64_t c, bool active, double* u)
@@ -214,75 +136,6 @@ namespace smr::dev
                        });
         }
 
-        // op_recipe on waited-for sources; (dst, op | n << 8, first source,
-        // first of the n sources in src).  The sources are taken one after the
-        // other as they come, in the recipe's order.
-        __device__ __forceinline__ void flow_recipe(const int32_t* __restrict__ rec, const int32_t* __restrict__ src, int64_t c, bool active,
-                                                    double* u, double bc)
-        {
-            int4 r{};
-            if (active)
-            {
-                r = reinterpret_cast<const int4*>(rec)[c];
-            }
-            const int op = r.y & 255, n = r.y >> 8;
-            double acc = 0;
-            int k      = 0;
-            bool first = true;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           for (; k < n; ++k)
-                           {
-                               const double* p = u + (k == 0 ? r.z : src[r.w + k]);
-                               double x        = first ? look(p) : look_again(p);
-                               if (marked(x) && first)
-                               {
-                                   x = look_again(p);
-                               }
-                               if (marked(x) && !last)
-                               {
-                                   first = false;
-                                   return false;
-                               }
-                               first = true;
-                               if (op == 0)
-                               {
-                                   acc = x;
-                               }
-                               else if (op == 1)
-                               {
-                                   acc = 2 * bc - x;
-                               }
-                               else if (op == 2)
-                               {
-                                   acc += x;
-                               }
-                               else if (k == 0)
-                               {
-                                   acc = x;
-                               }
-                               else if (n == 3)
-                               {
-                                   // u0 - u1 * 3 + u2 * 3
-                                   acc = k == 1 ? acc - x * 3.0 : acc + x * 3.0;
-                               }
-                               else
-                               {
-                                   // u0 - u1 * 5 + u2 * 10 - u3 * 10 + u4 * 5
-                                   const double w = x * (k == 1 || k == 4 ? 5.0 : 10.0);
-                                   acc            = (k & 1) ? acc - w : acc + w;
-                               }
-                           }
-                           if (op == 2 && n > 0)
-                           {
-                               acc /= n;
-                           }
-                           publish(u + r.x, acc);
-                           return true;
-                       });
-        }
-
         // the item of wave w: the last one whose first wave is at most w
         // (at most 64 items, one per lane)
         __device__ __forceinline__ int item_of(const GhostFlow& f, int w)
@@ -325,8 +178,11 @@ namespace smr::dev
             u[dst] = __longlong_as_double((long long)kMark);
         }
 
+        // at most this many threads in a block (one ticket each)
+        constexpr int FLOW_BLOCK = 512;
+
         template <int DIM, int S>
-        __global__ __launch_bounds__(256) void k_ghost_flow(GhostFlow f, double* u, int64_t nref, double bc)
+        __global__ __launch_bounds__(FLOW_BLOCK) void k_ghost_flow(GhostFlow f, double* u, int64_t nref, double bc)
         {
             __shared__ unsigned ticket;
             if (threadIdx.x == 0)
@@ -334,7 +190,7 @@ namespace smr::dev
                 ticket = atomicAdd(reinterpret_cast<unsigned*>(u + nref), 1u);
             }
             __syncthreads();
-            const int w = __builtin_amdgcn_readfirstlane(int(ticket) * 4 + int(threadIdx.x >> 6));
+            const int w = __builtin_amdgcn_readfirstlane(int(ticket * (blockDim.x >> 6) + (threadIdx.x >> 6)));
             if (w >= f.nwaves)
             {
                 return;
@@ -357,8 +213,13 @@ namespace smr::dev
         {
             return;
         }
-        const dim3 g(unsigned((f.nwaves + 3) / 4)), b(256);
-        hipLaunchKernelGGL(k_ghost_reset, g, b, 0, s, f, u, nref);
+        // blocks queue about 10 ns each for their tickets, and small grids
+        // spread better in small blocks (update + upwind, 256 / 512 / 1024
+        // threads: 170 waves 19.0 / 19.9 / 20.8 us, 1.4 K waves 27.6 / 26.8 /
+        // 27.7, 3D 1.8 K waves 37.6 / 36.0 / 37.0)
+        const unsigned W = f.nwaves <= 512 ? 4 : FLOW_BLOCK / 64;
+        const dim3 g((unsigned(f.nwaves) + W - 1) / W), b(W * 64);
+        hipLaunchKernelGGL(k_ghost_reset, dim3(unsigned((f.nwaves + 3) / 4)), dim3(256), 0, s, f, u, nref);
         if (dim == 2 && ps == 0)
         {
             hipLaunchKernelGGL((k_ghost_flow<2, 0>), g, b, 0, s, f, u, nref, bc);

@@ -1,0 +1,56 @@
+"""The dataflow form of the frozen steps and their adjoint against the staged
+programs (which set_tuning selects): the same bits for both prediction radii,
+2D and 3D, one to many instances, and checkpoint intervals around the number of
+adjoint steps of a launch."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def frozen(sa, ctx, dim, lmax, s, seed):
+    mesh = sa.make_mesh(ctx, sa.mesh_config(dim, 1, lmax, s))
+    u = sa.make_scalar_field("u", mesh)
+    sa.make_bc_dirichlet(u, 0.5)
+    rng = np.random.default_rng(seed)
+    x = (mesh.cells()[:, 1:1 + dim] + 0.5) * 2.0 ** -lmax
+    c = rng.uniform(0.0, 1.0, dim)  # up to the boundary
+    u.set_cells(np.where(np.abs(x - c).max(axis=1) < 0.15, 1.0, 0.2) + 0.3 * np.exp(-((x - 0.4) ** 2).sum(axis=1) / 0.02))
+    sa.make_MRAdapt(u)(1e-2, 1.0)
+    return mesh, u.cells()
+
+
+@pytest.mark.parametrize("dim,lmax,s,n,steps,every", [(2, 4, 1, 1, 1, 1), (2, 6, 0, 3, 6, 3), (2, 6, 1, 2, 18, 18), (2, 5, 1, 2, 34, 17),
+                                                      (3, 3, 1, 2, 4, 2), (3, 4, 0, 1, 3, 1), (3, 5, 1, 2, 4, 4)])
+def test_flow_matches_stage_programs(gpu_ctx, dim, lmax, s, n, steps, every):
+    import samurai_amd as sa
+    import torch
+    print("flow", dim, lmax, s, n, steps, every, flush=True)
+    inst = [frozen(sa, gpu_ctx, dim, lmax, s, 10 + k) for k in range(n)]
+    rng = np.random.default_rng(2)
+    a = rng.uniform(-1.0, 1.0, (n, dim))
+    p = sa.AdjointProblem(gpu_ctx, [m for m, _ in inst], [0.2 * 2.0 ** -lmax] * n, bc=list(rng.uniform(0, 1, n)), steps=steps, checkpoint_every=every)
+    u0 = torch.tensor(np.concatenate([u for _, u in inst]), device="cuda")
+    gT = torch.tensor(rng.standard_normal(u0.numel()), device="cuda")
+
+    def both_ways():
+        uT, g0 = torch.empty_like(u0), torch.empty_like(u0)
+        torch.cuda.synchronize()
+        p.forward_ptr(u0.data_ptr(), uT.data_ptr())
+        ga = p.backward_ptr(gT.data_ptr(), g0.data_ptr())
+        return uT.cpu().numpy(), g0.cpu().numpy(), ga
+
+    p.set_velocity(a)
+    with pytest.raises(sa.SamuraiError):
+        p.backward_ptr(gT.data_ptr(), torch.empty_like(u0).data_ptr())
+    flow = [both_ways()]
+    p.set_velocity(-a)
+    flow.append(both_ways())
+    p.set_tuning(256, 0, 1)
+    staged = []
+    for v in (a, -a):
+        p.set_velocity(v)
+        staged.append(both_ways())
+    for got, want in zip(flow, staged):
+        for g, w in zip(got, want):
+            assert np.array_equal(g, w)
