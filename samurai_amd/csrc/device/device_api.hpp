@@ -512,6 +512,33 @@ namespace smr::dev
     void resolve_batch(const ResolveBatch& b, int* err, hipStream_t s);
     // fills l.walk_rows from the resolved bases (after resolve; no-op without walks)
     void walk_rows(const List& l, hipStream_t s);
+    // The flux-based convection operators without term lists (convection.hip),
+    // on graduated meshes: per cell the kinds of its sides (3 bits each, x-1,
+    // x+1, y-1, ...) and where its entries of fine (slots across its faces to
+    // finer cells) begin.
+    enum ConvOp : int
+    {
+        CONV_LINEAR  = 0,
+        CONV_BURGERS = 1,
+        CONV_FIELD   = 2
+    };
+    struct ConvSides
+    {
+        const int32_t *word, *fine_at, *fine;
+    };
+    struct ConvFields
+    {
+        const double* u;
+        const double* v[3]; // CONV_FIELD: the velocity components
+        double vel[3];      // CONV_LINEAR
+    };
+    // word, fine_at (one per cell) and fine (at most room entries) of the
+    // cells list l; leaf: nref scratch bytes, used: one scratch word; *err = 1
+    // when a stencil slot is missing
+    void conv_sides(int dim, const List& l, const Table& t, uint8_t* leaf, int64_t nref, int32_t* word, int32_t* fine_at, int32_t* fine, double* used,
+                    int64_t room, int* err, hipStream_t s);
+    // out[cell] = the operator on the cells of l
+    void convection(int dim, int op, const List& l, const ConvSides& sd, const ConvFields& a, double* out, hipStream_t s);
     // out[row[r]] = ordered sum of the terms of row r (flux-based convection)
     void conv_gather(const int64_t* row, const int64_t* ptr, const int64_t* src, const double* coef, int64_t nrows, const double* u,
                      double* out, hipStream_t s);

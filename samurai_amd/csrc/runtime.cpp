@@ -1345,10 +1345,12 @@ namespace smr
 
         // the dataflow launch of dm's update_ghost_mr for a field with a B.C.:
         // the stages of ghost_plan in order, the recipes of a level as one
-        // item; null when the recipes have no such form, and for one or two
-        // stages (uniform meshes), whose launches cost less than the reset
-        // and the flow (2D L9 uniform: 3 us against 8; from three stages on
-        // the flow wins: 12 us against 21 on 2D L2..7, 17 against 80 on L4..12)
+        // item; null when the recipes have no such form, and where the stages
+        // cost less than the reset and the flow (8 us): one or two stages
+        // (uniform meshes: 3 us), and up to ten stages of at most 1024 ghosts
+        // in all, which one block runs in a round each (update + upwind: 348
+        // ghosts in 9 stages 10.8 us against 14.1, 570 in 10 13.8 against 14.6;
+        // but 1177 in 10 15.8 against 14.9, 324 in 12 15.2 against 13.6)
         const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
         {
             const RecipeFlow& rf = dm.recipe_flow;
@@ -1397,11 +1399,13 @@ namespace smr
                     dm.prediction.cells_of_levels(level, level + 1, c0, c1);
                     add(dev::SEQ_PREDICT, c0, c1);
                 }
+                int64_t ghosts = 0;
                 for (int k = 0; k < f->nitems; ++k)
                 {
                     stages += f->op[k] != dev::SEQ_RECIPES;
+                    ghosts += f->c1[k] - f->c0[k];
                 }
-                f->nwaves     = stages < 3 ? 0 : int(waves);
+                f->nwaves     = stages < 3 || (stages <= 10 && ghosts <= 1024) ? 0 : int(waves);
                 dm.ghost_flow = std::move(f);
             }
             return dm.ghost_flow->nwaves > 0 ? dm.ghost_flow.get() : nullptr;
@@ -1529,6 +1533,54 @@ namespace smr
         dev::hand_loop(dm.cells.d, 0, dm.cells.d.ncells, u.d, unp1.d, dt, m.ctx->stream);
     }
 
+    namespace
+    {
+        // the cells fill the unit box
+        bool fills_box(const MRMeshData& m)
+        {
+            const CellArray& cells = m.ids[CELLS];
+            double volume          = 0; // sums of powers of two, exact
+            for (int l = 0; l < MAXL; ++l)
+            {
+                volume += std::ldexp(double(cells[size_t(l)].count()), -m.cfg.dim * l);
+            }
+            return volume == 1.0;
+        }
+
+        // the side table of m's cells, or null where the operators run on term
+        // lists: a mesh that is not graduated or has holes (jumps of several
+        // levels, part-refined faces), or more table entries than an int32 counts
+        const dev::ConvSides* conv_sides(Mesh& m, DevMesh& dm)
+        {
+            const int dim     = m.host.cfg.dim;
+            const int64_t n   = dm.cells.d.ncells;
+            const auto& cells = m.host.ids[CELLS];
+            const int64_t room = ca_min_level(cells) == ca_max_level(cells) ? 0 : 2 * dim * n;
+            if (!dm.sides)
+            {
+                if (!m.host.graduated || room > INT32_MAX || m.host.nref > INT32_MAX || !fills_box(m.host))
+                {
+                    return nullptr;
+                }
+                hipStream_t s = m.ctx->stream;
+                auto sides    = std::make_unique<DevMesh::Sides>();
+                const auto up = [](size_t b) { return (b + 255) & ~size_t(255); };
+                const size_t wb = up(size_t(n) * 4), fb = up(size_t(room) * 4);
+                char* p       = static_cast<char*>(sides->mem.get(2 * wb + fb + 256, s));
+                auto* word    = reinterpret_cast<int32_t*>(p);
+                auto* fine_at = reinterpret_cast<int32_t*>(p + wb);
+                auto* fine    = reinterpret_cast<int32_t*>(p + 2 * wb);
+                auto* used    = reinterpret_cast<double*>(p + 2 * wb + fb);
+                DevBuffer leaf;
+                dev::conv_sides(dim, dm.cells.d, dm.table, static_cast<uint8_t*>(leaf.get(size_t(m.host.nref), s)), m.host.nref, word, fine_at, fine,
+                                used, room, m.ctx->d_err, s);
+                sides->d = {word, fine_at, fine};
+                dm.sides = std::move(sides);
+            }
+            return &dm.sides->d;
+        }
+    } // namespace
+
     void convection_upwind(const double* v, Field& u, Field& out)
     {
         u.check_current();
@@ -1542,6 +1594,12 @@ namespace smr
         update_ghost_mr(u);
         DevMesh& dm = m.device();
         ScopedTimer timer(m.ctx, "convection operator");
+        if (const dev::ConvSides* sides = conv_sides(m, dm))
+        {
+            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, m.ctx->stream), "hipMemsetAsync(convection)");
+            dev::convection(dim, dev::CONV_LINEAR, dm.cells.d, *sides, {u.d, {}, {v[0], v[1], dim == 3 ? v[2] : 0.0}}, out.d, m.ctx->stream);
+            return;
+        }
         bool same = dm.conv != nullptr;
         for (int d = 0; same && d < dim; ++d)
         {
@@ -1608,6 +1666,12 @@ namespace smr
         DevMesh& dm = m.device();
         ScopedTimer timer(m.ctx, "convection operator");
         hipStream_t s = m.ctx->stream;
+        if (const dev::ConvSides* sides = conv_sides(m, dm))
+        {
+            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, s), "hipMemsetAsync(convection)");
+            dev::convection(m.host.cfg.dim, dev::CONV_BURGERS, dm.cells.d, *sides, {u.d, {}, {}}, out.d, s);
+            return;
+        }
         if (!dm.burgers)
         {
             dm.burgers = upload_terms(build_burgers_terms(m.host), s);
@@ -1686,6 +1750,12 @@ namespace smr
         DevMesh& dm = m.device();
         ScopedTimer timer(m.ctx, "convection operator");
         hipStream_t s = m.ctx->stream;
+        if (const dev::ConvSides* sides = conv_sides(m, dm))
+        {
+            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, s), "hipMemsetAsync(convection)");
+            dev::convection(dim, dev::CONV_FIELD, dm.cells.d, *sides, {u.d, {vel[0], vel[1], vel[2]}, {}}, out.d, s);
+            return;
+        }
         if (!dm.heterogeneous)
         {
             dm.heterogeneous = upload_terms(build_heterogeneous_terms(m.host), s);

@@ -200,7 +200,16 @@ namespace smr
         std::vector<DevRecipes> outer;
         DevWorkList projection, prediction;
         DevWorkList detail, criteria, maximum;
+        // what lies across the cells' faces, for the flux-based convection
+        // operators on graduated meshes (built on first use)
+        struct Sides
+        {
+            DevBuffer mem;
+            dev::ConvSides d{};
+        };
+        std::unique_ptr<Sides> sides;
         // flux-based convection terms of the last velocity used on this image
+        // (meshes that are not graduated)
         struct Conv
         {
             double v[3] = {0, 0, 0};

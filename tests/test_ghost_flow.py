@@ -17,10 +17,10 @@ def random_mesh(ctx, dim, lmin, lmax, s, r, seed):
     rng = np.random.default_rng(seed)
     for _ in range(lmax - lmin):
         cells, tags = m.cells(), np.zeros(m.nb_cells(sa.REFERENCE), dtype=np.uint8)
-        side = 1 << cells[:, 0]
-        parent = cells[:, 1] // 2 + side * (cells[:, 2] // 2 + side * (cells[:, 3] // 2)) + cells[:, 0] * 7919
-        coarsen = rng.random(parent.max() + 1) < 0.7  # whole sibling groups
-        tags[cells[:, 4]] = np.where(coarsen[parent], sa.COARSEN, sa.KEEP)
+        keys = np.column_stack([cells[:, 0], cells[:, 1:4] // 2])
+        _, group, size = np.unique(keys, axis=0, return_inverse=True, return_counts=True)
+        coarsen = (rng.random(len(size)) < 0.7) & (size == 1 << dim)  # whole sibling groups
+        tags[cells[:, 4]] = np.where(coarsen[group.ravel()], sa.COARSEN, sa.KEEP)
         m.rebuild_from_tags(tags)
     return m
 
