@@ -218,6 +218,25 @@ namespace smr::dev
             out[row[r]] = acc;
         }
 
+        // 1 / b to the last bit or so, by Newton's iteration from the hardware's
+        // estimate, for b far from the ends of the exponent range
+        __device__ __forceinline__ double newton_rcp(double b)
+        {
+            double y = __builtin_amdgcn_rcp(b);
+            y        = fma(y, fma(-b, y, 1.0), y);
+            return fma(y, fma(-b, y, 1.0), y);
+        }
+
+        // a / b correctly rounded, from y = newton_rcp(b): the quotient corrected
+        // by its exact remainder (Markstein, Computation of elementary functions
+        // on the IBM RISC System/6000 processor, 1990).  Without the scaling a
+        // division needs at the ends of the exponent range.
+        __device__ __forceinline__ double markstein_div(double a, double b, double y)
+        {
+            const double q = a * y;
+            return fma(fma(-b, q, a), y, q);
+        }
+
         // The WENO5 flux of Jiang & Shu (1996) on five flux values centred on
         // f[2] (schemes/fv/operators/weno_impl.hpp:26-66): third-order
         // candidates (eq. 2.8), smoothness indicators (3.2-3.4), non-linear
@@ -237,9 +256,26 @@ namespace smr::dev
             const double is1 = 13. / 12 * (b1 * b1) + 1. / 4 * (c1 * c1);
             const double is2 = 13. / 12 * (b2 * b2) + 1. / 4 * (c2 * c2);
             const double e0 = eps + is0, e1 = eps + is1, e2 = eps + is2;
-            const double a0  = 0.1 / (e0 * e0);
-            const double a1  = 0.6 / (e1 * e1);
-            const double a2  = 0.3 / (e2 * e2);
+            const double g0 = e0 * e0, g1 = e1 * e1, g2 = e2 * e2;
+            // The divisions were most of the kernels' FP64 work (with them as
+            // below L11 took 73.1 us instead of 83.7, 3D L7 75.6 instead of
+            // 84.2).  g is at least 1e-12; below 2^300
+            // no quotient, remainder or sum comes near the ends of the exponent
+            // range, and the three divisions by the sum share one reciprocal
+            // (larger values, infinities and NaN take the plain divisions).
+            const double limit = 0x1p300;
+            if (g0 < limit && g1 < limit && g2 < limit)
+            {
+                const double a0  = markstein_div(0.1, g0, newton_rcp(g0));
+                const double a1  = markstein_div(0.6, g1, newton_rcp(g1));
+                const double a2  = markstein_div(0.3, g2, newton_rcp(g2));
+                const double sum = a0 + a1 + a2;
+                const double y   = newton_rcp(sum);
+                return markstein_div(a0, sum, y) * q0 + markstein_div(a1, sum, y) * q1 + markstein_div(a2, sum, y) * q2;
+            }
+            const double a0  = 0.1 / g0;
+            const double a1  = 0.6 / g1;
+            const double a2  = 0.3 / g2;
             const double sum = a0 + a1 + a2;
             return a0 / sum * q0 + a1 / sum * q1 + a2 / sum * q2;
         }
@@ -404,6 +440,71 @@ namespace smr::dev
             const int lo     = __builtin_amdgcn_update_dpp(0, int(uint32_t(w)), CTRL, 0xF, 0xF, false);
             const int hi     = __builtin_amdgcn_update_dpp(0, int(uint32_t(w >> 32)), CTRL, 0xF, 0xF, false);
             return __longlong_as_double(int64_t((uint64_t(uint32_t(hi)) << 32) | uint32_t(lo)));
+        }
+
+        // The dense kernel by strips of 64 columns: a wavefront walks R rows up,
+        // so that most interface fluxes are evaluated once instead of by both of
+        // their cells.  Along x a cell evaluates its right interface and takes
+        // the left one from the lane beside it (the strip's first column from
+        // one extra evaluation, lane r for row r); along y the upper interface
+        // stays in its register as the next row's lower one; in 3D the two z
+        // interfaces are evaluated per cell.  The fluxes and the order of the
+        // sums are those of k_weno5_dense, so the results are the same bits.
+        // n >= 64.  Bound by the FP64 work of the fluxes: 2 R + 2 evaluations
+        // for R rows in 2D, against 3.25 per row on the 64 x 4 tiles.
+        template <int DIM, int R>
+        __global__ __launch_bounds__(BLOCK) void k_weno5_strips(const double* __restrict__ u, double* __restrict__ out, int n, int64_t W,
+                                                                double v0, double v1, double v2, double fa)
+        {
+            const int lane    = int(threadIdx.x & 63);
+            const int64_t w   = int64_t(blockIdx.x) * (BLOCK / 64) + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+            const int strips  = n / 64, bands = n / R;
+            const int64_t all = int64_t(strips) * bands * (DIM == 3 ? n : 1);
+            if (w >= all)
+            {
+                return;
+            }
+            const int x  = int(w % strips) * 64 + lane, y0 = int((w / strips) % bands) * R, z = DIM == 3 ? int(w / (int64_t(strips) * bands)) : 0;
+            const int g  = 3;
+            int64_t c    = (DIM == 3 ? int64_t(z + g) * W * W : 0) + int64_t(y0 + g) * W + (x + g);
+            double left0 = 0;
+            if (lane < R)
+            {
+                left0 = weno5_at(u + c - lane + lane * W - 3, 1, v0);
+            }
+            double below = weno5_at(u + c - 3 * W, W, v1);
+#pragma unroll 1
+            for (int r = 0; r < R; ++r, c += W)
+            {
+                const double frx   = weno5_at(u + c - 2, 1, v0);
+                const double above = weno5_at(u + c - 2 * W, W, v1);
+                const double first = __longlong_as_double(readlane64(__double_as_longlong(left0), r));
+                const double shift = wave_shift<0x138>(frx);
+                const double flx   = lane == 0 ? first : shift;
+                double acc         = 0;
+                auto add           = [&](bool low, double fl, double fr)
+                {
+                    if (low)
+                    {
+                        acc += fr * fa;
+                        acc += fl * -fa;
+                    }
+                    else
+                    {
+                        acc += fl * -fa;
+                        acc += fr * fa;
+                    }
+                };
+                add(x == 0, flx, frx);
+                add(y0 + r == 0, below, above);
+                if constexpr (DIM == 3)
+                {
+                    const double flz = weno5_at(u + c - 3 * W * W, W * W, v2), frz = weno5_at(u + c - 2 * W * W, W * W, v2);
+                    add(z == 0, flz, frz);
+                }
+                out[c] = acc;
+                below  = above;
+            }
         }
 
         // Upwind (2D) by column walks: a wavefront owns 64 columns of a stack of
@@ -1005,17 +1106,33 @@ namespace smr::dev
     {
         const int64_t W     = int64_t(n) + 6;
         const int64_t total = dim == 3 ? int64_t(n) * n * n : int64_t(n) * n;
-        if (dim == 3)
+        // Strips walk R rows one after the other, so they need enough of them
+        // to fill the chip.  Whole call, ghosts included (one thread per cell or
+        // tiles / strips of 4 rows): 2D L9 19.1 / 21.6 us, L10 30.8 / 30.3, L11
+        // 73.1 / 64.4; 3D L6 26.2 / 29.6, L7 75.6 / 64.4 (2 rows: L10 30.7, L11
+        // 73.6; 8 rows: 32.4, 62.1; 16 rows: 38.0, 66.3).
+        const bool untiled = std::getenv("SMR_WENO5_UNTILED") != nullptr;
+        const bool strips  = !untiled && n >= (dim == 3 ? 128 : 1024);
+        auto waves        = [&](int rows) { return dim3(unsigned((total / 64 / rows + BLOCK / 64 - 1) / (BLOCK / 64))); };
+        if (!strips && dim == 3)
         {
             hipLaunchKernelGGL(k_weno5_dense<3>, dim3(nblocks(total)), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
         }
-        else if (n >= 64 && !std::getenv("SMR_WENO5_UNTILED"))
+        else if (!strips && n >= 64 && !untiled)
         {
             hipLaunchKernelGGL(k_weno5_dense2d_tiled, dim3(unsigned(n / 64), unsigned(n / 4)), dim3(256), 0, s, u, out, n, W, v[0], v[1], fa);
         }
-        else
+        else if (!strips)
         {
             hipLaunchKernelGGL(k_weno5_dense<2>, dim3(nblocks(total)), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
+        }
+        else if (dim == 3)
+        {
+            hipLaunchKernelGGL((k_weno5_strips<3, 4>), waves(4), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
+        }
+        else
+        {
+            hipLaunchKernelGGL((k_weno5_strips<2, 4>), waves(4), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
         }
     }
 

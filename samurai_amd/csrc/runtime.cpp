@@ -1345,12 +1345,14 @@ namespace smr
 
         // the dataflow launch of dm's update_ghost_mr for a field with a B.C.:
         // the stages of ghost_plan in order, the recipes of a level as one
-        // item; null when the recipes have no such form, and where the stages
-        // cost less than the reset and the flow (8 us): one or two stages
-        // (uniform meshes: 3 us), and up to ten stages of at most 1024 ghosts
-        // in all, which one block runs in a round each (update + upwind: 348
-        // ghosts in 9 stages 10.8 us against 14.1, 570 in 10 13.8 against 14.6;
-        // but 1177 in 10 15.8 against 14.9, 324 in 12 15.2 against 13.6)
+        // item; null when the recipes have no such form, and where the staged
+        // launches cost at most 11 us by the count below (the reset and the flow
+        // take 9 to 17): a run of stages in one block 2 us and 0.9 us per 1024
+        // ghosts of each, a grid-wide stage 3.5 us.  Measured, the stages
+        // against the flow, with the operator that follows: WENO5 2D L7 13.4 /
+        // 17.3 us, L8 16.2 / 17.1, L9 22.0 / 19.2 (uniform meshes, 3 to 4 wide
+        // ghost stages); upwind, 348 ghosts in 9 stages 10.8 / 14.1, 570 in 10
+        // 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7.
         const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
         {
             const RecipeFlow& rf = dm.recipe_flow;
@@ -1360,8 +1362,22 @@ namespace smr
             }
             if (!dm.ghost_flow)
             {
-                int stages = 0;
-                auto f     = std::make_unique<dev::GhostFlow>();
+                double staged_us = 0;
+                bool in_block    = false;
+                auto stage       = [&](int64_t n)
+                {
+                    if (n > kSeqSmall)
+                    {
+                        staged_us += 3.5;
+                        in_block = false;
+                    }
+                    else if (n > 0)
+                    {
+                        staged_us += (in_block ? 0.0 : 2.0) + 0.9 * double((n + 1023) / 1024);
+                        in_block = true;
+                    }
+                };
+                auto f = std::make_unique<dev::GhostFlow>();
                 f->proj = dm.projection.d;
                 f->pred = dm.prediction.d;
                 f->rec  = dm.flow_rec;
@@ -1386,26 +1402,22 @@ namespace smr
                     const Recipes& r = dm.outer[size_t(level)].host;
                     for (size_t k = 0; k + 1 < r.stage_ptr.size(); ++k)
                     {
-                        stages += r.stage_ptr[k + 1] > r.stage_ptr[k] && !r.stage_without_bc_only(k);
+                        stage(r.stage_without_bc_only(k) ? 0 : r.stage_ptr[k + 1] - r.stage_ptr[k]);
                     }
                     if (level > 0)
                     {
                         dm.projection.cells_of_levels(level - 1, level, c0, c1);
+                        stage(c1 - c0);
                         add(dev::SEQ_PROJECT, c0, c1);
                     }
                 }
                 for (int level = 1; level <= cfg.max_level; ++level)
                 {
                     dm.prediction.cells_of_levels(level, level + 1, c0, c1);
+                    stage(c1 - c0);
                     add(dev::SEQ_PREDICT, c0, c1);
                 }
-                int64_t ghosts = 0;
-                for (int k = 0; k < f->nitems; ++k)
-                {
-                    stages += f->op[k] != dev::SEQ_RECIPES;
-                    ghosts += f->c1[k] - f->c0[k];
-                }
-                f->nwaves     = stages < 3 || (stages <= 10 && ghosts <= 1024) ? 0 : int(waves);
+                f->nwaves     = staged_us < 11.05 ? 0 : int(waves);
                 dm.ghost_flow = std::move(f);
             }
             return dm.ghost_flow->nwaves > 0 ? dm.ghost_flow.get() : nullptr;
