@@ -90,11 +90,12 @@ namespace smr::dev::bitops
             WordPos p;
             p.l             = level_of_word(b, w);
             const int64_t r = w - b.off[p.l];
-            const int64_t n = int64_t(1) << p.l;
-            p.wx            = r % b.wpr[p.l];
-            const int64_t row = r / b.wpr[p.l];
-            p.y             = int32_t(dim == 3 ? row % n : row);
-            p.z             = int32_t(dim == 3 ? row / n : 0);
+            // max(1, 2^l / 64) words per row and 2^l rows per plane
+            const int sw      = p.l > 6 ? p.l - 6 : 0;
+            const int64_t row = r >> sw;
+            p.wx              = r & ((int64_t(1) << sw) - 1);
+            p.y               = int32_t(dim == 3 ? row & ((int64_t(1) << p.l) - 1) : row);
+            p.z               = int32_t(dim == 3 ? row >> p.l : 0);
             return p;
         }
 

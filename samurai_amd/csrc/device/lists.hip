@@ -48,93 +48,128 @@ namespace smr::dev
             }
         }
 
-        // the lists of one mesh laid out one after the other, each over the
-        // words of its own levels only: list k holds the words [off[lo[k]],
-        // off[hi[k]]) of the padded layout, from index base[k] on
-        struct ListLayout
+        // The lists of one mesh are laid out one after the other, each over the
+        // words of its own levels only: list k holds the words [off[lo], off[hi])
+        // of the padded layout.  The list of an index comes from a chain of
+        // compares over values that all threads share (an array of them indexed
+        // per thread lived in scratch memory).
+        struct ListWord
         {
-            int64_t base[DL_N + 1];
-            int lo[DL_N], hi[DL_N];
+            int k;
+            int64_t gw;  // word of the padded layout
+            int64_t set; // the list's words of the layout start at bits + set when addressed by padded word
         };
 
-        __device__ __forceinline__ ListLayout list_layout(const PBits& p, int minl, int maxl, int nlists)
+        __device__ __forceinline__ ListWord list_of(const PBits& p, int minl, int maxl, int nlists, int64_t j)
         {
-            ListLayout L;
-            L.base[0] = 0;
+            ListWord w{0, 0, 0};
+            int64_t base = 0;
+#pragma unroll
             for (int k = 0; k < DL_N; ++k)
             {
-                int lo = 0, hi = 0;
                 if (k < nlists)
                 {
+                    int lo, hi;
                     list_levels(k, minl, maxl, lo, hi);
+                    const int64_t o = p.off[lo], n = p.off[hi] - o;
+                    if (j >= base)
+                    {
+                        w.k   = k;
+                        w.set = base - o;
+                        w.gw  = o + (j - base);
+                    }
+                    base += n;
                 }
-                L.lo[k]       = lo;
-                L.hi[k]       = hi;
-                L.base[k + 1] = L.base[k] + (p.off[hi] - p.off[lo]);
             }
-            return L;
+            return w;
         }
 
-        // the list holding layout index j, and its word of the padded layout
-        __device__ __forceinline__ int list_of(const ListLayout& L, const PBits& p, int64_t j, int64_t& gw)
+        // the words of all lists
+        __device__ __forceinline__ int64_t list_total(const PBits& p, int minl, int maxl, int nlists)
         {
-            int k = 0;
-            while (k + 1 < DL_N && L.base[k + 1] <= j)
+            int64_t n = 0;
+#pragma unroll
+            for (int k = 0; k < DL_N; ++k)
             {
-                ++k;
+                if (k < nlists)
+                {
+                    int lo, hi;
+                    list_levels(k, minl, maxl, lo, hi);
+                    n += p.off[hi] - p.off[lo];
+                }
             }
-            gw = p.off[L.lo[k]] + (j - L.base[k]);
-            return k;
+            return n;
         }
 
-        // the bitmap of list k addressed by padded word (only its levels' words exist)
-        __device__ __forceinline__ const uint64_t* list_set(const ListLayout& L, const PBits& p, const uint64_t* bits, int k)
+        // the layout index of the first word of level l of list k (levels
+        // outside the list's range: its start or its end)
+        __device__ __forceinline__ int64_t list_level_index(const PBits& p, int minl, int maxl, int nlists, int k, int l)
         {
-            return bits + L.base[k] - p.off[L.lo[k]];
+            int64_t base = 0;
+            for (int q = 0; q < k; ++q)
+            {
+                int lo, hi;
+                list_levels(q, minl, maxl, lo, hi);
+                base += p.off[hi] - p.off[lo];
+            }
+            int lo, hi;
+            list_levels(k, minl, maxl, lo, hi);
+            return base + p.off[l < lo ? lo : (l > hi ? hi : l)] - p.off[lo];
         }
 
-        // the scan at the first word of level l of list k (levels outside the
-        // list's range: its start or its end); n: the scanned words
-        __device__ __forceinline__ uint64_t list_level_start(const ListLayout& L, const PBits& p, int k, int l, const uint64_t* counts,
-                                                             const uint64_t* scan, int64_t n)
-        {
-            const int c     = l < L.lo[k] ? L.lo[k] : (l > L.hi[k] ? L.hi[k] : l);
-            const int64_t w = L.base[k] + (p.off[c] - p.off[L.lo[k]]);
-            return w < n ? scan[w] : (n > 0 ? scan[n - 1] + counts[n - 1] : 0ull);
-        }
-
-        // word gw (of a level of the list) of list k
+        // word gw (of a level of the list) of list k.  Most words are empty: the
+        // one set that costs a single load is looked at first.
         __device__ __forceinline__ uint64_t list_word(const PBits& p, const uint64_t* sets, const uint64_t* old_sets, int k, int64_t gw)
         {
-            const PWord q = pword(p, gw);
-            const int t   = q.l;
             const int64_t total = p.off[p.hi + 1];
             const uint64_t* C   = sets + SM_CELLS * total;
             const uint64_t* J   = sets + SM_PROJ_CELLS * total;
             const uint64_t* R   = sets + SM_REFERENCE * total;
-            const int64_t X0    = 64 * q.wx;
-            uint64_t v          = 0;
+            const uint64_t* OC  = old_sets + SM_CELLS * total;
+            uint64_t v;
             switch (k)
             {
-                case DL_PROJECTION: v = coarse_word(p, R, t, 1, q.Y, q.Z, X0) & J[gw]; break;
-                case DL_PREDICTION:
-                {
-                    // clip to the domain [0, 2^t) on every axis
-                    const int64_t n = int64_t(1) << t;
-                    const int64_t y = q.Y - p.pad, z = q.Z - p.pad;
-                    if (y < 0 || y >= n || (p.dim == 3 && (z < 0 || z >= n)))
-                    {
-                        return 0ull;
-                    }
-                    v = R[gw] & ~(C[gw] | J[gw]) & range_mask(p.pad, q.wx, 0, n) & refine_word(p, R, t, q.Y, q.Z, q.wx);
-                    break;
-                }
-                case DL_DETAIL: v = R[gw] & (coarse_word(p, C, t, 1, q.Y, q.Z, X0) | coarse_word(p, C, t, 2, q.Y, q.Z, X0)); break;
+                case DL_PROJECTION: v = J[gw]; break;
+                case DL_PREDICTION: v = R[gw] & ~(C[gw] | J[gw]); break;
+                case DL_DETAIL:
                 case DL_CRITERIA:
-                case DL_MAXIMUM: v = coarse_word(p, C, t, 1, q.Y, q.Z, X0) & R[gw]; break;
-                case DL_UF_COPY: v = old_sets[SM_REFERENCE * total + gw] & C[gw]; break;
-                case DL_UF_COARSEN: v = coarse_word(p, old_sets + SM_CELLS * total, t, 1, q.Y, q.Z, X0) & C[gw]; break;
-                default: v = coarse_word(p, C, t, 1, q.Y, q.Z, X0) & old_sets[SM_CELLS * total + gw]; break;
+                case DL_MAXIMUM: v = R[gw]; break;
+                case DL_UF_COPY: v = C[gw]; break;
+                case DL_UF_COARSEN: v = C[gw]; break;
+                default: v = OC[gw]; break;
+            }
+            if (v == 0)
+            {
+                return 0ull;
+            }
+            if (k == DL_UF_COPY)
+            {
+                // both sets are clear past the row
+                return v & old_sets[SM_REFERENCE * total + gw];
+            }
+            const PWord q    = pword(p, gw);
+            const int t      = q.l;
+            const int64_t X0 = 64 * q.wx;
+            if (k == DL_PREDICTION)
+            {
+                // clip to the domain [0, 2^t) on every axis
+                const int64_t n = int64_t(1) << t;
+                const int64_t y = q.Y - p.pad, z = q.Z - p.pad;
+                if (y < 0 || y >= n || (p.dim == 3 && (z < 0 || z >= n)))
+                {
+                    return 0ull;
+                }
+                v &= range_mask(p.pad, q.wx, 0, n) & refine_word(p, R, t, q.Y, q.Z, q.wx);
+            }
+            else
+            {
+                const uint64_t* fine = k == DL_PROJECTION ? R : (k == DL_UF_COARSEN ? OC : C);
+                uint64_t on          = coarse_word(p, fine, t, 1, q.Y, q.Z, X0);
+                if (k == DL_DETAIL)
+                {
+                    on |= coarse_word(p, C, t, 2, q.Y, q.Z, X0);
+                }
+                v &= on;
             }
             return v & tail_mask(p, t, q.wx);
         }
@@ -142,27 +177,28 @@ namespace smr::dev
         __global__ __launch_bounds__(SB) void k_list_words(PBits p, int minl, int maxl, const uint64_t* sets, const uint64_t* old_sets, int nlists,
                                                            uint64_t* bits)
         {
-            const ListLayout L = list_layout(p, minl, maxl, nlists);
-            const int64_t i    = int64_t(blockIdx.x) * SB + threadIdx.x;
-            if (i < L.base[DL_N])
+            const int64_t i = int64_t(blockIdx.x) * SB + threadIdx.x;
+            if (i < list_total(p, minl, maxl, nlists))
             {
-                int64_t gw;
-                const int k = list_of(L, p, i, gw);
-                bits[i]     = list_word(p, sets, old_sets, k, gw);
+                const ListWord w = list_of(p, minl, maxl, nlists, i);
+                bits[i]          = list_word(p, sets, old_sets, w.k, w.gw);
             }
         }
 
         // runs starting in the word << 32 | cells of the word
+        __device__ __forceinline__ uint64_t list_count(const PBits& p, const uint64_t* bits, const ListWord& w)
+        {
+            const uint64_t* set = bits + w.set;
+            const uint64_t v    = set[w.gw];
+            return v ? (uint64_t(run_count_word(p, set, w.gw)) << 32) | uint64_t(__popcll(v)) : 0ull;
+        }
+
         __global__ __launch_bounds__(SB) void k_list_counts(PBits p, int minl, int maxl, int nlists, const uint64_t* bits, uint64_t* counts)
         {
-            const ListLayout L = list_layout(p, minl, maxl, nlists);
-            const int64_t i    = int64_t(blockIdx.x) * SB + threadIdx.x;
-            if (i < L.base[DL_N])
+            const int64_t i = int64_t(blockIdx.x) * SB + threadIdx.x;
+            if (i < list_total(p, minl, maxl, nlists))
             {
-                int64_t gw;
-                const int k         = list_of(L, p, i, gw);
-                const uint64_t* set = list_set(L, p, bits, k);
-                counts[i]           = (uint64_t(run_count_word(p, set, gw)) << 32) | uint64_t(__popcll(set[gw]));
+                counts[i] = list_count(p, bits, list_of(p, minl, maxl, nlists, i));
             }
         }
 
@@ -172,8 +208,9 @@ namespace smr::dev
             const int i = int(blockIdx.x) * SB + threadIdx.x;
             if (i < nlists * SM_SEG)
             {
-                const ListLayout L = list_layout(p, minl, maxl, nlists);
-                table[i]           = list_level_start(L, p, i / SM_SEG, i % SM_SEG, counts, scan, L.base[DL_N]);
+                const int64_t n = list_total(p, minl, maxl, nlists);
+                const int64_t w = list_level_index(p, minl, maxl, nlists, i / SM_SEG, i % SM_SEG);
+                table[i]        = w < n ? scan[w] : (n > 0 ? scan[n - 1] + counts[n - 1] : 0ull);
             }
         }
 
@@ -250,14 +287,15 @@ namespace smr::dev
         __global__ __launch_bounds__(SB) void k_list_emit(PBits p, int minl, int maxl, int nlists, const uint64_t* bits, const uint64_t* scan,
                                                           ListOuts outs)
         {
-            const ListLayout L = list_layout(p, minl, maxl, nlists);
-            const int64_t i    = int64_t(blockIdx.x) * SB + threadIdx.x;
-            const int64_t n    = L.base[DL_N];
+            const int64_t i = int64_t(blockIdx.x) * SB + threadIdx.x;
+            const int64_t n = list_total(p, minl, maxl, nlists);
             if (i < n)
             {
-                int64_t gw;
-                const int k = list_of(L, p, i, gw);
-                emit_list_word(p, list_set(L, p, bits, k), gw, scan[i], outs.l[k]);
+                const ListWord w = list_of(p, minl, maxl, nlists, i);
+                if (bits[i])
+                {
+                    emit_list_word(p, bits + w.set, w.gw, scan[i], outs.l[w.k]);
+                }
             }
             else if (i < n + nlists)
             {
@@ -269,21 +307,14 @@ namespace smr::dev
         // layout) from index cp[k] of the concatenated bitmaps, its ids and old
         // ids from word SM_NSETS * pw0 ----
 
-        __device__ __forceinline__ ListLayout item_layout(const SubmeshItem& it)
-        {
-            return list_layout(it.p, it.minl, it.p.hi, DL_N);
-        }
-
         __global__ __launch_bounds__(SB) void k_blist_words(const SubmeshItem* items, const int64_t* cp, int n, const uint64_t* sets,
                                                             const uint64_t* old_sets, uint64_t* bits)
         {
             for_word(items, cp, n, 1,
                      [&](const SubmeshItem& it, int k, int64_t j)
                      {
-                         const ListLayout L = item_layout(it);
-                         int64_t gw;
-                         const int list  = list_of(L, it.p, j, gw);
-                         bits[cp[k] + j] = list_word(it.p, sets + SM_NSETS * it.pw0, old_sets + SM_NSETS * it.pw0, list, gw);
+                         const ListWord w = list_of(it.p, it.minl, it.p.hi, DL_N, j);
+                         bits[cp[k] + j]  = list_word(it.p, sets + SM_NSETS * it.pw0, old_sets + SM_NSETS * it.pw0, w.k, w.gw);
                      });
         }
 
@@ -293,11 +324,7 @@ namespace smr::dev
             for_word(items, cp, n, 1,
                      [&](const SubmeshItem& it, int k, int64_t j)
                      {
-                         const ListLayout L = item_layout(it);
-                         int64_t gw;
-                         const int list      = list_of(L, it.p, j, gw);
-                         const uint64_t* set = list_set(L, it.p, bits + cp[k], list);
-                         counts[cp[k] + j]   = (uint64_t(run_count_word(it.p, set, gw)) << 32) | uint64_t(__popcll(set[gw]));
+                         counts[cp[k] + j] = list_count(it.p, bits + cp[k], list_of(it.p, it.minl, it.p.hi, DL_N, j));
                      });
         }
 
@@ -312,14 +339,11 @@ namespace smr::dev
             }
             const int k           = int(i / (DL_N * SM_SEG));
             const SubmeshItem& it = items[k];
-            const ListLayout L    = item_layout(it);
             // the item's counts and scan, read through its first index (the
             // scan keeps counting over the items before it)
             const int64_t N = cp[n];
             const int list  = int(i / SM_SEG % DL_N);
-            const int l     = int(i % SM_SEG);
-            const int c     = l < L.lo[list] ? L.lo[list] : (l > L.hi[list] ? L.hi[list] : l);
-            const int64_t w = cp[k] + L.base[list] + (it.p.off[c] - it.p.off[L.lo[list]]);
+            const int64_t w = cp[k] + list_level_index(it.p, it.minl, it.p.hi, DL_N, list, int(i % SM_SEG));
             table[i]        = w < N ? scan[w] : (N > 0 ? scan[N - 1] + counts[N - 1] : 0ull);
         }
 
@@ -329,10 +353,11 @@ namespace smr::dev
             for_word(items, cp, n, 1,
                      [&](const SubmeshItem& it, int k, int64_t j)
                      {
-                         const ListLayout L = item_layout(it);
-                         int64_t gw;
-                         const int list = list_of(L, it.p, j, gw);
-                         emit_list_word(it.p, list_set(L, it.p, bits + cp[k], list), gw, scan[cp[k] + j], outs[k * DL_N + list]);
+                         const ListWord w = list_of(it.p, it.minl, it.p.hi, DL_N, j);
+                         if (bits[cp[k] + j])
+                         {
+                             emit_list_word(it.p, bits + cp[k] + w.set, w.gw, scan[cp[k] + j], outs[k * DL_N + w.k]);
+                         }
                      });
         }
 

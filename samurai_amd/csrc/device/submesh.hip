@@ -102,13 +102,25 @@ namespace smr::dev
             project_chain(p, R, U, J, t1);
         }
 
+        // the first word of the set that holds word i of consecutive sets (a few)
+        __device__ __forceinline__ int64_t set_start(int64_t total, int64_t i)
+        {
+            int64_t s = 0;
+            while (i >= s + total)
+            {
+                s += total;
+            }
+            return s;
+        }
+
         __global__ __launch_bounds__(SB) void k_sm_run_counts(PBits p, int nsets, const uint64_t* sets, int32_t* counts)
         {
             const int64_t total = p.off[p.hi + 1];
             const int64_t i     = int64_t(blockIdx.x) * SB + threadIdx.x;
             if (i < total * nsets)
             {
-                counts[i] = run_count_word(p, sets + (i / total) * total, i % total);
+                const int64_t set0 = set_start(total, i);
+                counts[i]          = run_count_word(p, sets + set0, i - set0);
             }
         }
 
@@ -120,7 +132,8 @@ namespace smr::dev
             const int64_t i     = int64_t(blockIdx.x) * SB + threadIdx.x;
             if (i < total * nsets)
             {
-                run_emit_word(p, sets + (i / total) * total, i % total, offsets[i], runs, cap);
+                const int64_t set0 = set_start(total, i);
+                run_emit_word(p, sets + set0, i - set0, offsets[i], runs, cap);
             }
         }
 

@@ -67,6 +67,22 @@ namespace smr::dev::smops
             return c;
         }
 
+        // a = q b + r for a, b >= 0; in 32 bits where both fit (a 64-bit
+        // division is over a hundred instructions, and the per-word kernels
+        // below were bound by two or three of them per word)
+        __device__ __forceinline__ void divmod(int64_t a, int64_t b, int64_t& q, int64_t& r)
+        {
+            if ((uint64_t(a) | uint64_t(b)) >> 32 == 0)
+            {
+                const uint32_t x = uint32_t(a), y = uint32_t(b), z = x / y;
+                q = z;
+                r = x - z * y;
+                return;
+            }
+            q = a / b;
+            r = a - q * b;
+        }
+
         struct PWord
         {
             int l;
@@ -81,12 +97,16 @@ namespace smr::dev::smops
             {
                 ++l;
             }
-            q.l               = l;
-            const int64_t r   = gw - p.off[l];
-            q.wx              = r % p.wpr[l];
-            const int64_t row = r / p.wpr[l];
-            q.Y               = p.dim == 3 ? row % p.n[l] : row;
-            q.Z               = p.dim == 3 ? row / p.n[l] : 0;
+            q.l             = l;
+            const int64_t r = gw - p.off[l];
+            int64_t row;
+            divmod(r, p.wpr[l], row, q.wx);
+            q.Y = row;
+            q.Z = 0;
+            if (p.dim == 3)
+            {
+                divmod(row, p.n[l], q.Z, q.Y);
+            }
             return q;
         }
 
