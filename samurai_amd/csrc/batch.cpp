@@ -11,6 +11,7 @@
 #include <cstring>
 #include <fstream>
 #include <map>
+#include <numeric>
 #include <optional>
 #include <sstream>
 #include <stdexcept>
@@ -1334,6 +1335,7 @@ namespace smr
                 std::optional<ScopedTimer> tb(std::in_place, nullptr, "harten program build");
                 adapt_prog_.clear();
                 std::vector<Chain> chains(na);
+                build_flow(adapt_flow_, act);
                 // the criteria thresholds of every instance (the program's aux
                 // data), then the instances' chains in parallel
                 std::vector<size_t> thr_at(na);
@@ -1367,7 +1369,10 @@ namespace smr
                     ti.tag          = tag;
                     pre[1]          = {ti};
                     Chain g;
-                    ghost_chain(g, dm, c, f.d, f.has_bc, f.bc_value);
+                    if (!adapt_flow_.ok)
+                    {
+                        ghost_chain(g, dm, c, f.d, f.has_bc, f.bc_value);
+                    }
                     Chain ch = zip(pre, g);
                     int64_t c0, c1;
                     dm.detail.cells_of_levels(c.min_level > 0 ? c.min_level - 1 : 0, c.max_level - ite, c0, c1);
@@ -1399,6 +1404,7 @@ namespace smr
                 adapt_prog_.append(chains);
                 adapt_prog_.upload_for(pass_tuning());
                 tb.reset();
+                run_flow(adapt_flow_);
                 adapt_prog_.run(pass_tuning());
                 calls += int(na);
                 // the versions the previous pass replaced, freed on the host
@@ -1726,13 +1732,19 @@ namespace smr
         {
             if (fv_key_[q] == key)
             {
+                fv_last_ = q;
                 return *fv_prog_[q];
             }
         }
         const int q   = fv_next_;
         fv_next_      = 1 - fv_next_;
+        fv_last_      = q;
         ProgramBuf& p = *fv_prog_[q];
         p.clear();
+        fv_key_[q].clear();
+        std::vector<int> all(inst_.size());
+        std::iota(all.begin(), all.end(), 0);
+        build_flow(fv_flow_[q], all);
         std::vector<Chain> chains(inst_.size());
         for (size_t i = 0; i < inst_.size(); ++i)
         {
@@ -1740,7 +1752,10 @@ namespace smr
             DevMesh& dm         = *b.u->mesh->dev;
             const MeshConfig& c = b.u->mesh->host.cfg;
             Chain ch;
-            ghost_chain(ch, dm, c, b.u->d, b.u->has_bc, b.u->bc_value);
+            if (!fv_flow_[q].ok)
+            {
+                ghost_chain(ch, dm, c, b.u->d, b.u->has_bc, b.u->bc_value);
+            }
             dev::Segment g = list_seg(dev::SEG_UPWIND, c, dm.cells, 0, dm.cells.d.ncells);
             g.u            = b.u->d;
             g.out          = b.unp1->d;
@@ -1755,6 +1770,58 @@ namespace smr
         p.upload();
         fv_key_[q] = std::move(key);
         return p;
+    }
+
+    void Batch::build_flow(FlowSet& fs, const std::vector<int>& ids)
+    {
+        fs.ok            = false;
+        const size_t n   = ids.size();
+        std::vector<int64_t> pref(n + 1, 0);
+        std::vector<const dev::GhostFlow*> form(n);
+        for (size_t k = 0; k < n; ++k)
+        {
+            const Field& u      = *inst_[size_t(ids[k])].u;
+            const MeshConfig& c = u.mesh->host.cfg;
+            const MeshConfig& d = inst_[size_t(ids[0])].u->mesh->host.cfg;
+            form[k]             = u.has_bc && c.dim == d.dim && c.pred_s == d.pred_s ? ghost_flow(*u.mesh->dev, c) : nullptr;
+            if (!form[k])
+            {
+                return;
+            }
+            pref[k + 1] = pref[k] + form[k]->nwaves;
+            fs.dim      = c.dim;
+            fs.ps       = c.pred_s;
+        }
+        fs.ok     = true;
+        fs.n      = int(n);
+        fs.nwaves = pref[n];
+        if (fs.nwaves == 0)
+        {
+            return;
+        }
+        const size_t ib = align_up(n * sizeof(dev::FlowInstance), 256), pb = align_up((n + 1) * 8, 256);
+        char* h         = ctx_->staging->acquire(ib + pb);
+        auto* inst      = reinterpret_cast<dev::FlowInstance*>(h);
+        for (size_t k = 0; k < n; ++k)
+        {
+            const Field& u = *inst_[size_t(ids[k])].u;
+            inst[k]        = {*form[k], u.d, u.bc_value};
+        }
+        std::memcpy(h + ib, pref.data(), (n + 1) * 8);
+        char* d = static_cast<char*>(fs.mem.get(ib + pb + 256, ctx_->stream));
+        hip_check(hipMemcpyAsync(d, h, ib + pb, hipMemcpyHostToDevice, ctx_->stream), "hipMemcpyAsync(ghost flows)");
+        ctx_->staging->release(ctx_->stream);
+        fs.inst   = reinterpret_cast<const dev::FlowInstance*>(d);
+        fs.pref   = reinterpret_cast<const int64_t*>(d + ib);
+        fs.ticket = reinterpret_cast<unsigned*>(d + ib + pb);
+    }
+
+    void Batch::run_flow(const FlowSet& fs)
+    {
+        if (fs.ok)
+        {
+            dev::ghost_flow_batch(fs.dim, fs.ps, fs.inst, fs.pref, fs.n, fs.nwaves, fs.ticket, ctx_->stream);
+        }
     }
 
     Tuning Batch::pass_tuning() const
@@ -1795,7 +1862,9 @@ namespace smr
         ensure_images(all);
         {
             ScopedTimer t(ctx_, "ghost update + field expressions");
-            fv_program().run(tuning_);
+            ProgramBuf& p = fv_program();
+            run_flow(fv_flow_[fv_last_]);
+            p.run(tuning_);
             // the versions the adaptation replaced, freed on the host while the
             // advance program runs
             release_replaced();

@@ -167,7 +167,7 @@ namespace smr
         // advance programs for the two u/unp1 parities, reused while the instances' storages are unchanged
         std::unique_ptr<ProgramBuf> fv_prog_[2];
         std::vector<const void*> fv_key_[2];
-        int fv_next_ = 0;
+        int fv_next_ = 0, fv_last_ = 0; // the slot replaced next, the one fv_program returned last
         // per-instance detail (f64) and tag (u8) storage, concatenated
         double* det_arena_ = nullptr;
         uint8_t* tag_arena_ = nullptr;
@@ -181,6 +181,23 @@ namespace smr
         // update_fields lists), freed while the next launches run
         std::vector<std::shared_ptr<void>> replaced_;
 
+        // the dataflow ghost update of several instances' u fields in one
+        // launch; ok is false when an instance has no such form (no B.C., see
+        // ghost_flow) or the instances differ in dimension or prediction radius:
+        // their programs then carry the staged chains
+        struct FlowSet
+        {
+            bool ok = false;
+            int dim = 2, ps = 1, n = 0;
+            int64_t nwaves = 0;
+            DevBuffer mem;
+            const dev::FlowInstance* inst = nullptr;
+            const int64_t* pref           = nullptr;
+            unsigned* ticket              = nullptr;
+        };
+        FlowSet adapt_flow_, fv_flow_[2];
+        void build_flow(FlowSet& fs, const std::vector<int>& ids);
+        void run_flow(const FlowSet& fs);
         void release_replaced();
         // the launch shape of the programs built for one adaptation pass
         Tuning pass_tuning() const;

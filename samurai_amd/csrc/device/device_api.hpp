@@ -363,6 +363,16 @@ namespace smr::dev
         int32_t op[kFlowItems]; // SeqOp
     };
     void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s);
+    // the same of many fields in one launch: instance k takes the waves
+    // [wpref[k], wpref[k + 1]) of wpref[n] = nwaves (device arrays; ticket: one
+    // scratch word)
+    struct FlowInstance
+    {
+        GhostFlow f;
+        double* u;
+        double bc;
+    };
+    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, hipStream_t s);
 
     // Frozen-mesh steps of many instances and their adjoint as dataflow
     // launches (adjoint_flow.hip).  Slots number the storages of all instances

@@ -146,18 +146,9 @@ namespace smr::dev
             return __builtin_amdgcn_readfirstlane(63 - __clzll(m));
         }
 
-        // stores the mark in every ghost of the update and clears its ticket
-        __global__ __launch_bounds__(256) void k_ghost_reset(GhostFlow f, double* u, int64_t nref)
+        // stores the mark in the ghosts of wave w of the update
+        __device__ __forceinline__ void reset_wave(const GhostFlow& f, int w, double* u)
         {
-            if (blockIdx.x == 0 && threadIdx.x == 0)
-            {
-                *reinterpret_cast<unsigned*>(u + nref) = 0;
-            }
-            const int w = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
-            if (w >= f.nwaves)
-            {
-                return;
-            }
             const int k     = item_of(f, w);
             const int64_t c = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
             if (c >= f.c1[k])
@@ -171,11 +162,40 @@ namespace smr::dev
             }
             else
             {
-                const List& l  = f.op[k] == SEQ_PROJECT ? f.proj : f.pred;
+                const List& l   = f.op[k] == SEQ_PROJECT ? f.proj : f.pred;
                 const int64_t r = l.cellrun[c];
                 dst             = l.base[r * l.ntaps] + l.iv[5 * r] + (c - l.pref[r]);
             }
             u[dst] = __longlong_as_double((long long)kMark);
+        }
+
+        // computes the ghosts of wave w
+        template <int DIM, int S>
+        __device__ __forceinline__ void flow_wave(const GhostFlow& f, int w, double* u, double bc)
+        {
+            const int k       = item_of(f, w);
+            const int64_t c   = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
+            const bool active = c < f.c1[k];
+            switch (f.op[k])
+            {
+                case SEQ_RECIPES: flow_recipe(f.rec, f.rsrc, c, active, u, bc); break;
+                case SEQ_PROJECT: flow_project<DIM>(f.proj, c, active, u); break;
+                default: flow_predict<DIM, S>(f.pred, c, active, u); break;
+            }
+        }
+
+        // marks every ghost of the update and clears its ticket
+        __global__ __launch_bounds__(256) void k_ghost_reset(GhostFlow f, double* u, int64_t nref)
+        {
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+            {
+                *reinterpret_cast<unsigned*>(u + nref) = 0;
+            }
+            const int w = int(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+            if (w < f.nwaves)
+            {
+                reset_wave(f, w, u);
+            }
         }
 
         // at most this many threads in a block (one ticket each)
@@ -191,18 +211,65 @@ namespace smr::dev
             }
             __syncthreads();
             const int w = __builtin_amdgcn_readfirstlane(int(ticket * (blockDim.x >> 6) + (threadIdx.x >> 6)));
-            if (w >= f.nwaves)
+            if (w < f.nwaves)
             {
-                return;
+                flow_wave<DIM, S>(f, w, u, bc);
             }
-            const int k       = item_of(f, w);
-            const int64_t c   = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
-            const bool active = c < f.c1[k];
-            switch (f.op[k])
+        }
+
+        // ---- many fields per launch: the waves of one after the other ----
+
+        // blocks of the batched launch: thousands of tickets, so the largest
+        constexpr int BATCH_BLOCK = 1024;
+
+        // the instance of wave w: the last one with pref[k] <= w, 64 looked at
+        // per step
+        __device__ __forceinline__ int instance_of(const int64_t* pref, int n, int64_t w)
+        {
+            const int lane = int(threadIdx.x & 63);
+            int lo = 0; // pref[lo] <= w throughout
+            while (n > 64)
             {
-                case SEQ_RECIPES: flow_recipe(f.rec, f.rsrc, c, active, u, bc); break;
-                case SEQ_PROJECT: flow_project<DIM>(f.proj, c, active, u); break;
-                default: flow_predict<DIM, S>(f.pred, c, active, u); break;
+                const int step   = (n + 63) >> 6;
+                const int k      = lo + lane * step;
+                const uint64_t m = __ballot(k < lo + n && pref[k] <= w);
+                const int next   = lo + (63 - __clzll(m)) * step;
+                n                = min(step, lo + n - next);
+                lo               = next;
+            }
+            const uint64_t m = __ballot(lane < n && pref[lo + lane] <= w);
+            return __builtin_amdgcn_readfirstlane(lo + (63 - __clzll(m)));
+        }
+
+        __global__ __launch_bounds__(256) void k_ghost_reset_batch(const FlowInstance* inst, const int64_t* pref, int n, int64_t nwaves, unsigned* ticket)
+        {
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+            {
+                *ticket = 0;
+            }
+            const int64_t w = int64_t(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+            if (w < nwaves)
+            {
+                const int k = instance_of(pref, n, w);
+                reset_wave(inst[k].f, int(w - pref[k]), inst[k].u);
+            }
+        }
+
+        template <int DIM, int S>
+        __global__ __launch_bounds__(BATCH_BLOCK) void k_ghost_flow_batch(const FlowInstance* inst, const int64_t* pref, int n, int64_t nwaves,
+                                                                          unsigned* ticket)
+        {
+            __shared__ unsigned t;
+            if (threadIdx.x == 0)
+            {
+                t = atomicAdd(ticket, 1u);
+            }
+            __syncthreads();
+            const int64_t w = int64_t(__builtin_amdgcn_readfirstlane(int(t))) * (BATCH_BLOCK / 64) + __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+            if (w < nwaves)
+            {
+                const int k = instance_of(pref, n, w);
+                flow_wave<DIM, S>(inst[k].f, int(w - pref[k]), inst[k].u, inst[k].bc);
             }
         }
     } // namespace
@@ -235,6 +302,33 @@ namespace smr::dev
         else
         {
             hipLaunchKernelGGL((k_ghost_flow<3, 1>), g, b, 0, s, f, u, nref, bc);
+        }
+    }
+
+    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, hipStream_t s)
+    {
+        if (nwaves <= 0)
+        {
+            return;
+        }
+        constexpr int W = BATCH_BLOCK / 64;
+        const dim3 g(unsigned((nwaves + W - 1) / W)), b(BATCH_BLOCK);
+        hipLaunchKernelGGL(k_ghost_reset_batch, dim3(unsigned((nwaves + 3) / 4)), dim3(256), 0, s, inst, wpref, n, nwaves, ticket);
+        if (dim == 2 && ps == 0)
+        {
+            hipLaunchKernelGGL((k_ghost_flow_batch<2, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+        }
+        else if (dim == 2)
+        {
+            hipLaunchKernelGGL((k_ghost_flow_batch<2, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+        }
+        else if (ps == 0)
+        {
+            hipLaunchKernelGGL((k_ghost_flow_batch<3, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+        }
+        else
+        {
+            hipLaunchKernelGGL((k_ghost_flow_batch<3, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
         }
     }
 } // namespace smr::dev

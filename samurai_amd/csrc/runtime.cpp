@@ -1343,86 +1343,6 @@ namespace smr
             return plan;
         }
 
-        // the dataflow launch of dm's update_ghost_mr for a field with a B.C.:
-        // the stages of ghost_plan in order, the recipes of a level as one
-        // item; null when the recipes have no such form, and where the staged
-        // launches cost at most 11 us by the count below (the reset and the flow
-        // take 9 to 17): a run of stages in one block 2 us and 0.9 us per 1024
-        // ghosts of each, a grid-wide stage 3.5 us.  Measured, the stages
-        // against the flow, with the operator that follows: WENO5 2D L7 13.4 /
-        // 17.3 us, L8 16.2 / 17.1, L9 22.0 / 19.2 (uniform meshes, 3 to 4 wide
-        // ghost stages); upwind, 348 ghosts in 9 stages 10.8 / 14.1, 570 in 10
-        // 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7.
-        const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
-        {
-            const RecipeFlow& rf = dm.recipe_flow;
-            if (!rf.ok)
-            {
-                return nullptr;
-            }
-            if (!dm.ghost_flow)
-            {
-                double staged_us = 0;
-                bool in_block    = false;
-                auto stage       = [&](int64_t n)
-                {
-                    if (n > kSeqSmall)
-                    {
-                        staged_us += 3.5;
-                        in_block = false;
-                    }
-                    else if (n > 0)
-                    {
-                        staged_us += (in_block ? 0.0 : 2.0) + 0.9 * double((n + 1023) / 1024);
-                        in_block = true;
-                    }
-                };
-                auto f = std::make_unique<dev::GhostFlow>();
-                f->proj = dm.projection.d;
-                f->pred = dm.prediction.d;
-                f->rec  = dm.flow_rec;
-                f->rsrc = dm.flow_src;
-                int64_t waves = 0;
-                auto add      = [&](int op, int64_t c0, int64_t c1)
-                {
-                    if (c1 > c0)
-                    {
-                        const int k = f->nitems++;
-                        f->op[k]    = op;
-                        f->c0[k]    = int32_t(c0);
-                        f->c1[k]    = int32_t(c1);
-                        f->wave0[k] = int32_t(waves);
-                        waves += (c1 - c0 + 63) / 64;
-                    }
-                };
-                int64_t c0, c1;
-                for (int level = cfg.max_level; level >= 0; --level)
-                {
-                    add(dev::SEQ_RECIPES, rf.level[size_t(level) + 1], rf.level[size_t(level)]);
-                    const Recipes& r = dm.outer[size_t(level)].host;
-                    for (size_t k = 0; k + 1 < r.stage_ptr.size(); ++k)
-                    {
-                        stage(r.stage_without_bc_only(k) ? 0 : r.stage_ptr[k + 1] - r.stage_ptr[k]);
-                    }
-                    if (level > 0)
-                    {
-                        dm.projection.cells_of_levels(level - 1, level, c0, c1);
-                        stage(c1 - c0);
-                        add(dev::SEQ_PROJECT, c0, c1);
-                    }
-                }
-                for (int level = 1; level <= cfg.max_level; ++level)
-                {
-                    dm.prediction.cells_of_levels(level, level + 1, c0, c1);
-                    stage(c1 - c0);
-                    add(dev::SEQ_PREDICT, c0, c1);
-                }
-                f->nwaves     = staged_us < 11.05 ? 0 : int(waves);
-                dm.ghost_flow = std::move(f);
-            }
-            return dm.ghost_flow->nwaves > 0 ? dm.ghost_flow.get() : nullptr;
-        }
-
         // maximum_op from the finest level down (mr/adapt.hpp:348-358)
         SeqPlan& max_plan(Ctx& ctx, DevMesh& dm, const MeshConfig& cfg)
         {
@@ -1444,6 +1364,87 @@ namespace smr
         }
     } // namespace
 
+    // The dataflow launch of dm's update_ghost_mr for a field with a B.C.: the
+    // stages of ghost_plan in order, the recipes of a level as one item; null
+    // when the recipes have no such form.  A single field takes it
+    // (dm.ghost_flow_pays) unless the staged launches cost at most 11 us by the
+    // count below (the reset and the flow take 9 to 17): a run of stages in one
+    // block 2 us and 0.9 us per 1024 ghosts of each, a grid-wide stage 3.5 us.
+    // Measured, the stages against the flow, with the operator that follows:
+    // WENO5 2D L7 13.4 / 17.3 us, L8 16.2 / 17.1, L9 22.0 / 19.2 (uniform meshes,
+    // 3 to 4 wide ghost stages); upwind, 348 ghosts in 9 stages 10.8 / 14.1, 570
+    // in 10 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7.
+    const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
+    {
+        const RecipeFlow& rf = dm.recipe_flow;
+        if (!rf.ok)
+        {
+            return nullptr;
+        }
+        if (!dm.ghost_flow)
+        {
+            double staged_us = 0;
+            bool in_block    = false;
+            auto stage       = [&](int64_t n)
+            {
+                if (n > kSeqSmall)
+                {
+                    staged_us += 3.5;
+                    in_block = false;
+                }
+                else if (n > 0)
+                {
+                    staged_us += (in_block ? 0.0 : 2.0) + 0.9 * double((n + 1023) / 1024);
+                    in_block = true;
+                }
+            };
+            auto f = std::make_unique<dev::GhostFlow>();
+            f->proj = dm.projection.d;
+            f->pred = dm.prediction.d;
+            f->rec  = dm.flow_rec;
+            f->rsrc = dm.flow_src;
+            int64_t waves = 0;
+            auto add      = [&](int op, int64_t c0, int64_t c1)
+            {
+                if (c1 > c0)
+                {
+                    const int k = f->nitems++;
+                    f->op[k]    = op;
+                    f->c0[k]    = int32_t(c0);
+                    f->c1[k]    = int32_t(c1);
+                    f->wave0[k] = int32_t(waves);
+                    waves += (c1 - c0 + 63) / 64;
+                }
+            };
+            int64_t c0, c1;
+            for (int level = cfg.max_level; level >= 0; --level)
+            {
+                add(dev::SEQ_RECIPES, rf.level[size_t(level) + 1], rf.level[size_t(level)]);
+                const Recipes& r = dm.outer[size_t(level)].host;
+                for (size_t k = 0; k + 1 < r.stage_ptr.size(); ++k)
+                {
+                    stage(r.stage_without_bc_only(k) ? 0 : r.stage_ptr[k + 1] - r.stage_ptr[k]);
+                }
+                if (level > 0)
+                {
+                    dm.projection.cells_of_levels(level - 1, level, c0, c1);
+                    stage(c1 - c0);
+                    add(dev::SEQ_PROJECT, c0, c1);
+                }
+            }
+            for (int level = 1; level <= cfg.max_level; ++level)
+            {
+                dm.prediction.cells_of_levels(level, level + 1, c0, c1);
+                stage(c1 - c0);
+                add(dev::SEQ_PREDICT, c0, c1);
+            }
+            f->nwaves          = int(waves);
+            dm.ghost_flow      = std::move(f);
+            dm.ghost_flow_pays = staged_us > 11.05;
+        }
+        return dm.ghost_flow.get();
+    }
+
     void update_ghost_mr(Field& f)
     {
         f.check_current();
@@ -1454,7 +1455,8 @@ namespace smr
         const int dim   = m.host.cfg.dim;
         const int ps    = m.host.cfg.pred_s;
         const double bc = f.bc_value;
-        if (const dev::GhostFlow* flow = f.has_bc ? ghost_flow(dm, m.host.cfg) : nullptr)
+        const dev::GhostFlow* flow = f.has_bc ? ghost_flow(dm, m.host.cfg) : nullptr;
+        if (flow && dm.ghost_flow_pays)
         {
             dev::ghost_flow(dim, ps, *flow, f.d, m.host.nref, bc, s);
             return;

@@ -232,6 +232,7 @@ namespace smr
         RecipeFlow recipe_flow;
         const int32_t *flow_rec = nullptr, *flow_src = nullptr;
         std::unique_ptr<dev::GhostFlow> ghost_flow;
+        bool ghost_flow_pays = false; // against the staged launches, for one field
         std::unique_ptr<Blob> flow_blob;
         // launch plans of update_ghost_mr and of the tag finalization
         SeqPlan ghost_plan, max_plan;
@@ -488,6 +489,9 @@ namespace smr
     dev::Thresholds make_thresholds(const MeshConfig& cfg, int ite, double eps, double regularity);
 
     void update_ghost_mr(Field& f);
+    // the dataflow form of dm's ghost update, put together on first use; null
+    // when there is none
+    const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg);
     void upwind(const double* a, double dt, Field& u, Field& unp1);
     // out = u - a * v on the cells (the field expression of the flux-based demos)
     void sub_scaled(Field& u, double a, Field& v, Field& out);
