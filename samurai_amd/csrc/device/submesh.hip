@@ -69,7 +69,8 @@ namespace smr::dev
         // union[l - 1] for l = l0 down to 1, by one block (small levels)
         __global__ __launch_bounds__(1024) void k_sm_union_cascade(PBits p, const uint64_t* C, uint64_t* U, int l0)
         {
-            union_chain(p, C, U, l0);
+            __shared__ uint64_t lds[kChainWords];
+            union_chain(p, C, U, l0, lds);
         }
 
         __global__ __launch_bounds__(SB) void k_sm_coarse(PBits p, const uint64_t* C, const uint64_t* G, uint64_t* K1, uint64_t* K2)
@@ -99,7 +100,8 @@ namespace smr::dev
         // projection steps t = 0 .. t1 - 1 by one block (small levels)
         __global__ __launch_bounds__(1024) void k_sm_project_cascade(PBits p, uint64_t* R, const uint64_t* U, uint64_t* J, int t1)
         {
-            project_chain(p, R, U, J, t1);
+            __shared__ uint64_t lds[kChainWords];
+            project_chain(p, R, U, J, t1, lds);
         }
 
         // the first word of the set that holds word i of consecutive sets (a few)
@@ -164,11 +166,12 @@ namespace smr::dev
         hipLaunchKernelGGL(k_sm_cells, dim3(sm_blocks(total)), dim3(SB), 0, st, b, leaves, p, C);
         hipLaunchKernelGGL(k_sm_dilate, dim3(sm_blocks(total)), dim3(SB), 0, st, p, C, G, r);
         // the union chain from the finest level down (union[hi] is empty): a
-        // launch per large level, then one block for the small ones
-        constexpr int64_t kSmall = 1024; // words of a level a single block takes
+        // launch per large level, then one block for the levels that fit in LDS
+        // (2D L4..12: from L9 on, 22.5 us; through global memory 25.5 from L8 on
+        // and 7.1 for the step from L9; 2D L2..8 16.1 instead of 25.4)
         hipLaunchKernelGGL(k_sm_zero, dim3(sm_blocks(total)), dim3(SB), 0, st, U, total);
         int l = p.hi;
-        for (; l >= 1 && p.off[l] - p.off[l - 1] > kSmall; --l)
+        for (; l >= 1 && p.off[l + 1] > kChainWords; --l)
         {
             const int64_t n = p.off[l] - p.off[l - 1];
             hipLaunchKernelGGL(k_sm_union_level, dim3(sm_blocks(n)), dim3(SB), 0, st, p, C, U, l);
@@ -188,19 +191,16 @@ namespace smr::dev
         if (mr)
         {
             // the projection chain from level 0 up: one block for the steps
-            // between small levels, then a launch per step
-            int t1 = 0;
-            while (t1 < p.hi && std::max(p.off[t1 + 1] - p.off[t1], p.off[t1 + 2] - p.off[t1 + 1]) <= kSmall)
-            {
-                ++t1;
-            }
+            // between the levels that fit in LDS, then a launch per step (2D
+            // L4..12: 15.8 us up to L8; before 12.5 up to L7 and 5.7 for the step)
+            const int t1 = chain_level(p, p.hi, kChainWords / 2);
             if (t1 > 0)
             {
                 hipLaunchKernelGGL(k_sm_project_cascade, dim3(1), dim3(1024), 0, st, p, R, U, J, t1);
             }
             for (int t = t1; t < p.hi; ++t)
             {
-                const int64_t n = std::max(p.off[t + 1] - p.off[t], p.off[t + 2] - p.off[t + 1]);
+                const int64_t n = step_words(p, t);
                 hipLaunchKernelGGL(k_sm_project_step, dim3(sm_blocks(n)), dim3(SB), 0, st, p, R, U, J, t);
             }
         }

@@ -44,6 +44,7 @@ namespace smr::dev
         __global__ __launch_bounds__(CB) void k_bs_union(const SubmeshItem* items, uint64_t* sets)
         {
             __shared__ uint64_t s_raw[kItemWords];
+            __shared__ uint64_t lds[kChainWords];
             const SubmeshItem& it = stage_item(s_raw, items[blockIdx.x]);
             __syncthreads();
             const PBits& p = it.p;
@@ -53,7 +54,7 @@ namespace smr::dev
                 U[i] = 0;
             }
             __syncthreads();
-            union_chain(p, item_set(it, sets, SM_CELLS), U, p.hi);
+            union_chain(p, item_set(it, sets, SM_CELLS), U, p.hi, lds);
         }
 
         __global__ __launch_bounds__(SB) void k_bs_coarse(const SubmeshItem* items, const int64_t* ppref, int n, uint64_t* sets, uint64_t* scratch)
@@ -85,6 +86,7 @@ namespace smr::dev
         __global__ __launch_bounds__(CB) void k_bs_project(const SubmeshItem* items, uint64_t* sets)
         {
             __shared__ uint64_t s_raw[kItemWords];
+            __shared__ uint64_t lds[kChainWords];
             const SubmeshItem& it = stage_item(s_raw, items[blockIdx.x]);
             __syncthreads();
             uint64_t* J = item_set(it, sets, SM_PROJ_CELLS);
@@ -95,7 +97,7 @@ namespace smr::dev
             __syncthreads();
             if (it.mr)
             {
-                project_chain(it.p, item_set(it, sets, SM_REFERENCE), item_set(it, sets, SM_UNION_CELLS), J, it.p.hi);
+                project_chain(it.p, item_set(it, sets, SM_REFERENCE), item_set(it, sets, SM_UNION_CELLS), J, it.p.hi, lds);
             }
         }
 

@@ -227,15 +227,52 @@ namespace smr::dev::smops
             U[p.off[t] + i]  = v & tail_mask(p, t, q.wx);
         }
 
-        // union[l - 1] for l = l0 down to 1 by the threads of one block
-        // (union[l0] must be clear)
-        __device__ __forceinline__ void union_chain(const PBits& p, const uint64_t* C, uint64_t* U, int l0)
+        // LDS words of the one-block chains, whose levels wait for each other:
+        // a level kept there costs its index arithmetic (1.6 us), one through
+        // global memory 2.8 us
+        constexpr int kChainWords = 7168;
+
+        // the finest level whose words and all coarser ones fit in n LDS words
+        __host__ __device__ __forceinline__ int chain_level(const PBits& p, int l, int64_t n)
         {
-            for (int l = l0; l >= 1; --l)
+            while (l > 0 && p.off[l + 1] > n)
+            {
+                --l;
+            }
+            return l;
+        }
+
+        // union[l - 1] for l = l0 down to 1 by the threads of one block
+        // (union[l0] must be clear or computed); lds: kChainWords words, which
+        // hold cells | union of the levels that fit
+        __device__ __forceinline__ void union_chain(const PBits& p, const uint64_t* C, uint64_t* U, int l0, uint64_t* lds)
+        {
+            int l = l0;
+            for (; l >= 1 && p.off[l + 1] > kChainWords; --l)
             {
                 for (int64_t i = threadIdx.x; i < p.off[l] - p.off[l - 1]; i += blockDim.x)
                 {
                     union_word(p, C, U, l - 1, i);
+                }
+                __syncthreads();
+            }
+            if (l < 1)
+            {
+                return;
+            }
+            for (int64_t i = threadIdx.x; i < p.off[l + 1]; i += blockDim.x)
+            {
+                lds[i] = C[i] | (i >= p.off[l] ? U[i] : 0ull);
+            }
+            __syncthreads();
+            for (; l >= 1; --l)
+            {
+                for (int64_t i = p.off[l - 1] + threadIdx.x; i < p.off[l]; i += blockDim.x)
+                {
+                    const PWord q    = pword(p, i);
+                    const uint64_t v = coarse_word(p, lds, l - 1, 1, q.Y, q.Z, 64 * q.wx) & tail_mask(p, l - 1, q.wx);
+                    U[i]             = v;
+                    lds[i] |= v;
                 }
                 __syncthreads();
             }
@@ -324,6 +361,13 @@ namespace smr::dev::smops
             }
         }
 
+        // words of projection step t: those of level t and of level t + 1
+        __host__ __device__ __forceinline__ int64_t step_words(const PBits& p, int t)
+        {
+            const int64_t a = p.off[t + 1] - p.off[t], b = p.off[t + 2] - p.off[t + 1];
+            return a > b ? a : b;
+        }
+
         // set[t - 1].on(t) for the 64 bits of word wx of padded row (Y, Z) at level t
         __device__ __forceinline__ uint64_t refine_word(const PBits& p, const uint64_t* set, int t, int64_t Y, int64_t Z, int64_t wx)
         {
@@ -337,13 +381,41 @@ namespace smr::dev::smops
             return spread_parents(load64(r, p.wpr[t - 1], (x0 >> 1) + pad), int(x0 & 1));
         }
 
-        // projection steps t = 0 .. t1 - 1 by the threads of one block
-        __device__ __forceinline__ void project_chain(const PBits& p, uint64_t* R, const uint64_t* U, uint64_t* J, int t1)
+        // projection steps t = 0 .. t1 - 1 by the threads of one block; lds:
+        // kChainWords words, which hold the reference and the union of the
+        // levels that fit
+        __device__ __forceinline__ void project_chain(const PBits& p, uint64_t* R, const uint64_t* U, uint64_t* J, int t1, uint64_t* lds)
         {
-            for (int t = 0; t < t1; ++t)
+            const int T      = chain_level(p, t1, kChainWords / 2);
+            const int64_t nT = p.off[T + 1];
+            int t            = 0;
+            if (nT <= kChainWords / 2)
             {
-                const int64_t n = p.off[t + 1] - p.off[t] > p.off[t + 2] - p.off[t + 1] ? p.off[t + 1] - p.off[t] : p.off[t + 2] - p.off[t + 1];
-                for (int64_t i = threadIdx.x; i < n; i += blockDim.x)
+                uint64_t* r = lds;
+                uint64_t* u = lds + kChainWords / 2;
+                for (int64_t i = threadIdx.x; i < nT; i += blockDim.x)
+                {
+                    r[i] = R[i];
+                    u[i] = U[i];
+                }
+                __syncthreads();
+                for (; t < T; ++t)
+                {
+                    for (int64_t i = threadIdx.x; i < step_words(p, t); i += blockDim.x)
+                    {
+                        project_word(p, r, u, J, t, i);
+                    }
+                    __syncthreads();
+                }
+                for (int64_t i = threadIdx.x; i < nT; i += blockDim.x)
+                {
+                    R[i] = r[i];
+                }
+                __syncthreads();
+            }
+            for (; t < t1; ++t)
+            {
+                for (int64_t i = threadIdx.x; i < step_words(p, t); i += blockDim.x)
                 {
                     project_word(p, R, U, J, t, i);
                 }
