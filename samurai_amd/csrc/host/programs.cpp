@@ -5,7 +5,6 @@
 #include <cstdlib>
 #include <numeric>
 #include <stdexcept>
-#include <unordered_map>
 
 namespace smr
 {
@@ -105,41 +104,84 @@ namespace smr
         return stage_ptr[k + 1] > stage_ptr[k];
     }
 
+    namespace
+    {
+        // the stages in which each slot was last written and read, by open
+        // addressing; kept per thread and cleared by counting `epoch` on
+        // (two unordered maps took most of the time of a 3D mesh's recipes)
+        class SlotStages
+        {
+          public:
+            struct Entry
+            {
+                int64_t slot;
+                uint32_t epoch;
+                int32_t write, read; // -1: not yet
+            };
+            // room for n slots
+            void begin(size_t n)
+            {
+                size_t cap = 64;
+                while (cap < 2 * n)
+                {
+                    cap *= 2;
+                }
+                if (cap > table_.size() || table_.size() > kKeep)
+                {
+                    table_.assign(cap, Entry{0, 0, -1, -1});
+                    table_.shrink_to_fit();
+                    epoch_ = 0;
+                }
+                if (++epoch_ == 0)
+                {
+                    table_.assign(table_.size(), Entry{0, 0, -1, -1});
+                    epoch_ = 1;
+                }
+            }
+            Entry& at(int64_t slot)
+            {
+                const size_t mask = table_.size() - 1;
+                size_t k          = size_t((uint64_t(slot) * 0x9E3779B97F4A7C15ull) >> 32) & mask;
+                while (table_[k].epoch == epoch_ && table_[k].slot != slot)
+                {
+                    k = (k + 1) & mask;
+                }
+                if (table_[k].epoch != epoch_)
+                {
+                    table_[k] = {slot, epoch_, -1, -1};
+                }
+                return table_[k];
+            }
+
+          private:
+            static constexpr size_t kKeep = size_t(1) << 18; // entries a thread keeps between calls
+            std::vector<Entry> table_;
+            uint32_t epoch_ = 0;
+        };
+    } // namespace
+
     void Recipes::stage()
     {
         const size_t n = dst.size();
         std::vector<int> st(n, 0);
-        std::unordered_map<int64_t, int> last_write, last_read;
-        last_write.reserve(n);
-        last_read.reserve(src.size());
+        thread_local SlotStages last;
+        last.begin(n + src.size());
         int nstages = 0;
         for (size_t r = 0; r < n; ++r)
         {
             int s = 0;
             for (int64_t k = src_ptr[r]; k < src_ptr[r + 1]; ++k)
             {
-                auto it = last_write.find(src[size_t(k)]);
-                if (it != last_write.end())
-                {
-                    s = std::max(s, it->second + 1);
-                }
+                s = std::max(s, last.at(src[size_t(k)]).write + 1);
             }
-            auto w = last_write.find(dst[r]);
-            if (w != last_write.end())
-            {
-                s = std::max(s, w->second + 1);
-            }
-            auto rd = last_read.find(dst[r]);
-            if (rd != last_read.end())
-            {
-                s = std::max(s, rd->second + 1);
-            }
-            st[r]               = s;
-            last_write[dst[r]]  = s;
+            SlotStages::Entry& d = last.at(dst[r]);
+            s                    = std::max({s, d.write + 1, d.read + 1});
+            st[r]                = s;
+            d.write              = s;
             for (int64_t k = src_ptr[r]; k < src_ptr[r + 1]; ++k)
             {
-                int& lr = last_read[src[size_t(k)]];
-                lr      = std::max(lr, s);
+                int32_t& lr = last.at(src[size_t(k)]).read;
+                lr          = std::max(lr, s);
             }
             nstages = std::max(nstages, s + 1);
         }
@@ -167,25 +209,38 @@ namespace smr
             }
             nstages = k;
         }
-        std::vector<size_t> order(n);
-        std::iota(order.begin(), order.end(), size_t(0));
-        std::stable_sort(order.begin(),
-                         order.end(),
-                         [&](size_t a, size_t b)
-                         {
-                             return st[a] < st[b];
-                         });
+        // the recipes by stage, in their order within each
         Recipes out;
         out.stage_ptr.assign(size_t(nstages) + 1, 0);
-        for (size_t r : order)
+        std::vector<int64_t> nsrc(size_t(nstages) + 1, 0);
+        for (size_t r = 0; r < n; ++r)
         {
-            out.push(dst[r], op[r], src.data() + src_ptr[r], int(src_ptr[r + 1] - src_ptr[r]));
-            out.stage_ptr[size_t(st[r]) + 1]++;
+            ++out.stage_ptr[size_t(st[r]) + 1];
+            nsrc[size_t(st[r]) + 1] += src_ptr[r + 1] - src_ptr[r];
         }
         for (size_t k = 1; k < out.stage_ptr.size(); ++k)
         {
             out.stage_ptr[k] += out.stage_ptr[k - 1];
+            nsrc[k] += nsrc[k - 1];
         }
+        out.dst.resize(n);
+        out.op.resize(n);
+        out.src_ptr.resize(n + 1);
+        out.src.resize(src.size());
+        std::vector<int64_t> at(out.stage_ptr.begin(), out.stage_ptr.end());
+        for (size_t r = 0; r < n; ++r)
+        {
+            const size_t q = size_t(at[size_t(st[r])]++);
+            int64_t& to    = nsrc[size_t(st[r])];
+            out.dst[q]     = dst[r];
+            out.op[q]      = op[r];
+            out.src_ptr[q] = to;
+            for (int64_t k = src_ptr[r]; k < src_ptr[r + 1]; ++k)
+            {
+                out.src[size_t(to++)] = src[size_t(k)];
+            }
+        }
+        out.src_ptr[n] = int64_t(src.size());
         *this = std::move(out);
     }
 
