@@ -509,6 +509,7 @@ namespace smr
             const int64_t W       = wpref[size_t(n)];
             constexpr int kPasses = 3;
             const int fs          = kPasses + 1;
+            const int64_t fw      = (int64_t(n) * fs + 1) / 2; // words of the flags
             // the item table and its prefixes, one upload
             const size_t ib = (size_t(n) * sizeof(dev::MeshItem) + 255) & ~size_t(255);
             const size_t pb = size_t(n + 1) * 8;
@@ -526,13 +527,14 @@ namespace smr
             const auto* d_wpref = reinterpret_cast<const int64_t*>(dt + ib);
             const auto* d_cpref = reinterpret_cast<const int64_t*>(dt + ib + pb);
             const auto* d_rpref = reinterpret_cast<const int64_t*>(dt + ib + 2 * pb);
-            // bitmaps: old, add, rem, two pass buffers, the projected marks; flags
+            // bitmaps: old, add, rem, each pass's projected marks and the flags (cleared
+            // together), then two pass buffers
             DevBuffer work;
-            uint64_t* w = static_cast<uint64_t*>(work.get(size_t(6 * std::max<int64_t>(W, 1)) * 8 + size_t(n) * fs * 4 + 256, s));
-            uint64_t* old = w, *add = w + W, *rem = w + 2 * W, *q = w + 5 * W;
-            uint64_t* buf[2] = {w + 3 * W, w + 4 * W};
-            int* flags       = reinterpret_cast<int*>(w + 6 * W);
-            dev::mesh_batch_zero(w, 3 * W, s);
+            uint64_t* w = static_cast<uint64_t*>(work.get(size_t((5 + kPasses) * std::max<int64_t>(W, 1) + fw) * 8 + 256, s));
+            uint64_t* old = w, *add = w + W, *rem = w + 2 * W, *q = w + 3 * W;
+            int* flags       = reinterpret_cast<int*>(q + kPasses * W);
+            uint64_t* buf[2] = {q + kPasses * W + fw, q + (kPasses + 1) * W + fw};
+            dev::mesh_batch_zero(w, (3 + kPasses) * W + fw, s);
             dev::mesh_batch_leaves(d_items, d_rpref, rpref[size_t(n)], n, old, s);
             dev::mesh_batch_tag_marks(d_items, d_cpref, cpref[size_t(n)], n, add, rem, s);
             dev::mesh_batch_combine(old, add, rem, buf[0], W, s);
@@ -544,13 +546,16 @@ namespace smr
                 {
                     throw std::logic_error("make_graduation: no fixed point");
                 }
-                hip_check(hipMemsetAsync(flags, 0, size_t(n) * fs * 4, s), "hipMemsetAsync(flags)");
+                if (batch > 0)
+                {
+                    dev::mesh_batch_zero(q, kPasses * W + fw, s);
+                }
                 for (int p = 0; p < kPasses; ++p)
                 {
-                    dev::mesh_batch_graduation_pass(d_items, d_wpref, W, n, buf[cur], q, buf[1 - cur], w2, flags, fs, p, s);
+                    dev::mesh_batch_graduation_pass(d_items, d_wpref, W, n, buf[cur], q + p * W, buf[1 - cur], w2, flags, fs, p,
+                                                    p + 1 == kPasses ? old : nullptr, s);
                     cur = 1 - cur;
                 }
-                dev::mesh_batch_differ(d_wpref, W, n, buf[cur], old, flags, fs, kPasses, s);
                 hip_check(hipMemcpyAsync(hf.data(), flags, hf.size() * 4, hipMemcpyDeviceToHost, s), "hipMemcpyAsync(flags)");
                 ctx.sync();
                 bool all = true;

@@ -99,28 +99,6 @@ namespace smr::dev::bitops
             return p;
         }
 
-        // .on(l) of level l + 1 for word wx of row (y, z) at level l: OR over
-        // the child rows and the child pairs of each bit
-        template <int DIM>
-        __device__ __forceinline__ uint64_t on_parent_word(const Bits& b, const uint64_t* src, int l, int32_t y, int32_t z, int64_t wx)
-        {
-            const int lc     = l + 1;
-            const int64_t cw = b.wpr[lc];
-            uint64_t acc     = 0;
-            const int nz     = DIM == 3 ? 2 : 1;
-            for (int dz = 0; dz < nz; ++dz)
-            {
-                for (int dy = 0; dy < 2; ++dy)
-                {
-                    const int64_t base = word_of(b, lc, 0, 2 * y + dy, DIM == 3 ? 2 * z + dz : 0);
-                    const uint64_t c0  = src[base + 2 * wx];
-                    const uint64_t c1  = (2 * wx + 1 < cw) ? src[base + 2 * wx + 1] : 0ull;
-                    acc |= pair_or_compress(c0) | (pair_or_compress(c1) << 32);
-                }
-            }
-            return acc;
-        }
-
         // one bit per run: does word w of row (y, z) at level l start a run
         // (a set bit whose left neighbour in the row is clear)
         __device__ __forceinline__ uint64_t run_starts(const uint64_t* bits, int64_t w, int64_t wx)
@@ -201,11 +179,41 @@ namespace smr::dev::bitops
             }
         }
 
-        // list_interval_to_refine_for_graduation (graduation.hpp:245-330),
-        // first half: every word of nestedExpand(ca[f], w2) (box dilation
-        // clipped to the domain) at a level f in [lo + 2, hi] is projected two
-        // levels down (.on(f - 2): OR over 4x4 blocks) and ORed into p[f - 2]
-        // (p zeroed beforehand; at most 16 fine words share a target word)
+        // ORs bits into the word of level c that holds (x, y, z), and their
+        // projections into every coarser level's: p[c] |= p[c + 1].on(c) down to
+        // lo.  Only the bits this call is the first to set go on to the next
+        // level (who set the others takes those), so a subtree is climbed about
+        // once; at most 8 (2D: 4) words share a parent.
+        __device__ __forceinline__ void mark_up(const Bits& b, uint64_t* p, int c, int32_t x, int32_t y, int32_t z, uint64_t bits)
+        {
+            for (;; --c)
+            {
+                uint64_t* target = p + word_of(b, c, x, y, z);
+                if ((__atomic_load_n(target, __ATOMIC_RELAXED) & bits) == bits)
+                {
+                    return;
+                }
+                bits &= ~atomicOr(reinterpret_cast<unsigned long long*>(target), bits);
+                if (bits == 0 || c == b.lo)
+                {
+                    return;
+                }
+                x    = (x & ~63) >> 1;
+                bits = pair_or_compress(bits) << (x & 63);
+                y >>= 1;
+                z >>= 1;
+            }
+        }
+
+        // list_interval_to_refine_for_graduation (graduation.hpp:245-330): every
+        // word of nestedExpand(ca[f], w2) (box dilation clipped to the domain) at
+        // a level f in [lo + 2, hi] is projected two levels down (.on(f - 2): OR
+        // over 4x4 blocks), ORed into p[f - 2] (p zeroed beforehand; at most 16
+        // fine words share a target word) and from there into the coarser levels,
+        // so that p[c] = union over f >= c + 2 of the dilated cells of level f
+        // projected on c.  2D L4..12: 12.0 us; without the coarser levels
+        // it took 9.1, and those, a launch per large level and one block for the
+        // rest, 8.9 and more.
         template <int DIM>
         __device__ __forceinline__ void dilate_project_word(const Bits& b, const uint64_t* ca, uint64_t* p, int w2, int64_t gw)
         {
@@ -241,52 +249,19 @@ namespace smr::dev::bitops
             {
                 return;
             }
-            const uint64_t m     = pair_or_compress(pair_or_compress(acc));
-            const int32_t cx     = int32_t(q.wx * 64) >> 2;
-            uint64_t* target     = p + word_of(b, q.l - 2, cx, q.y >> 2, q.z >> 2);
-            const uint64_t bits  = m << (cx & 63);
-            if ((__atomic_load_n(target, __ATOMIC_RELAXED) & bits) != bits)
-            {
-                atomicOr(reinterpret_cast<unsigned long long*>(target), bits);
-            }
-        }
-
-        // second half, by one block: p[c] |= p[c + 1].on(c) from c = hi - 3
-        // down to lo, a level at a time (these levels hold 1/64 of the words
-        // of the finest one and less), so that p[c] = union over f >= c + 2 of
-        // the dilated fine cells of level f projected on c
-        template <int DIM>
-        __device__ __forceinline__ void cascade_word(const Bits& b, uint64_t* p, int c, int64_t gw)
-        {
-            const WordPos q  = word_pos(b, DIM, gw);
-            const uint64_t v = on_parent_word<DIM>(b, p, c, q.y, q.z, q.wx);
-            if (v)
-            {
-                p[gw] |= v;
-            }
-        }
-
-        // levels c0 down to lo of the cascade, by the calling block
-        template <int DIM>
-        __device__ __forceinline__ void cascade_levels(const Bits& b, uint64_t* p, int c0)
-        {
-            for (int c = c0; c >= b.lo; --c)
-            {
-                const int64_t n0 = b.off[c], n1 = b.off[c + 1];
-                for (int64_t gw = n0 + threadIdx.x; gw < n1; gw += blockDim.x)
-                {
-                    cascade_word<DIM>(b, p, c, gw);
-                }
-                __syncthreads();
-            }
+            const uint64_t m = pair_or_compress(pair_or_compress(acc));
+            const int32_t cx = int32_t(q.wx * 64) >> 2;
+            mark_up(b, p, q.l - 2, cx, q.y >> 2, q.z >> 2, m << (cx & 63));
         }
 
         // one graduation pass (graduation.hpp:629-718): the cells of level c
         // under p[c] are replaced by their children:
         // out[l] = (ca[l] | children(rem[l-1])) & ~rem[l], rem[c] = p[c] & ca[c];
-        // *flag = 1 if any cell is refined
+        // *flag = 1 if any cell is refined; with old (the last pass before a
+        // readback), *differ = 1 if out differs from it
         template <int DIM>
-        __device__ __forceinline__ void grad_apply_word(const Bits& b, const uint64_t* ca, const uint64_t* p, uint64_t* out, int* flag, int64_t gw)
+        __device__ __forceinline__ void grad_apply_word(const Bits& b, const uint64_t* ca, const uint64_t* p, uint64_t* out, int* flag, int64_t gw,
+                                                        const uint64_t* old, int* differ)
         {
             const WordPos q    = word_pos(b, DIM, gw);
             const uint64_t c   = ca[gw];
@@ -300,10 +275,15 @@ namespace smr::dev::bitops
                 const uint64_t pr = p[pw] & ca[pw];
                 add               = spread(pr >> (32 * (q.wx & 1)));
             }
-            out[gw] = (c | add) & ~rem;
+            const uint64_t v = (c | add) & ~rem;
+            out[gw]          = v;
             if (rem != 0)
             {
                 flag[0] = 1;
+            }
+            if (old && v != old[gw])
+            {
+                differ[0] = 1;
             }
         }
 

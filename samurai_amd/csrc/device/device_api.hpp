@@ -89,12 +89,11 @@ namespace smr::dev
     // update_cell_array_from_tag's marks of every item (cpref: prefix of cells)
     void mesh_batch_tag_marks(const MeshItem* items, const int64_t* cpref, int64_t ncells, int n, uint64_t* add, uint64_t* rem, hipStream_t s);
     // one graduation pass of every item (wpref: prefix of bitmap words);
-    // flags[k * fstride + pass] = 1 when item k refines a cell
+    // flags[k * fstride + pass] = 1 when item k refines a cell and, with old,
+    // flags[k * fstride + fstride - 1] = 1 when its out differs from it (p, of
+    // zeros, and the flags not cleared)
     void mesh_batch_graduation_pass(const MeshItem* items, const int64_t* wpref, int64_t nwords, int n, const uint64_t* ca, uint64_t* p,
-                                    uint64_t* out, int w2, int* flags, int fstride, int pass, hipStream_t s);
-    // flags[k * fstride + slot] = 1 when item k's bitmaps a and c differ
-    void mesh_batch_differ(const int64_t* wpref, int64_t nwords, int n, const uint64_t* a, const uint64_t* c, int* flags, int fstride, int slot,
-                           hipStream_t s);
+                                    uint64_t* out, int w2, int* flags, int fstride, int pass, const uint64_t* old, hipStream_t s);
     size_t mesh_batch_scan_temp_bytes(int64_t nwords);
     // runs of the items whose flag `slot` is set: counts and their exclusive sum,
     // then (x0, x1, y, z, level, item) records, at most cap
@@ -606,19 +605,21 @@ namespace smr::dev
     // one dependency-free stage of outer-ghost recipes
     // (Dirichlet recipes are skipped when the field has no boundary condition)
     // mesh update of a harten call on bitmaps (rebuild.hip)
-    void bits_zero(const Bits& b, uint64_t* bits, hipStream_t s);
+    // p[0, n) = 0
+    void bits_zero(uint64_t* p, int64_t n, hipStream_t s);
     // bits = the leaves of a cells work list
     void bits_from_cells(const List& l, const Bits& b, uint64_t* bits, hipStream_t s);
     // update_cell_array_from_tag's additions and removals of the leaves of l
+    // (add and rem not cleared)
     void bits_tag_marks(int dim, const List& l, const Bits& b, const uint8_t* tag, int min_level, int max_level, uint64_t* add, uint64_t* rem,
                         hipStream_t s);
     // out = (old | add) & ~rem
     void bits_combine(const Bits& b, const uint64_t* old, const uint64_t* add, const uint64_t* rem, uint64_t* out, hipStream_t s);
     // one pass of make_graduation's fixed point from ca into out (p: scratch
-    // bitmap); *flag = 1 if a cell was refined (flag not cleared)
-    void bits_graduation_pass(int dim, const Bits& b, const uint64_t* ca, uint64_t* p, uint64_t* out, int w2, int* flag, hipStream_t s);
-    // *flag = 1 if a and c differ (flag not cleared)
-    void bits_differ(const Bits& b, const uint64_t* a, const uint64_t* c, int* flag, hipStream_t s);
+    // bitmap, zero); *flag = 1 if a cell was refined and, with old, *differ = 1
+    // if out differs from it (p and the flags not cleared)
+    void bits_graduation_pass(int dim, const Bits& b, const uint64_t* ca, uint64_t* p, uint64_t* out, int w2, int* flag, const uint64_t* old,
+                              int* differ, hipStream_t s);
     // run-length encoding: counts and exclusive offsets (one per word of
     // levels [lo, hi]) of the runs of bits, then the runs as (x0, x1, y, z,
     // level) in (level, z, y, x) order

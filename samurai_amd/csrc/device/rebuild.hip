@@ -76,41 +76,14 @@ namespace smr::dev
             }
         }
 
-        // one level c of the cascade, grid-wide (the large levels)
         template <int DIM>
-        __global__ __launch_bounds__(RB) void k_project_cascade_level(Bits b, uint64_t* p, int c)
-        {
-            const int64_t gw = b.off[c] + int64_t(blockIdx.x) * RB + threadIdx.x;
-            if (gw < b.off[c + 1])
-            {
-                cascade_word<DIM>(b, p, c, gw);
-            }
-        }
-
-        // levels c0 down to lo of the cascade by one block
-        template <int DIM>
-        __global__ __launch_bounds__(1024) void k_project_cascade(Bits b, uint64_t* p, int c0)
-        {
-            cascade_levels<DIM>(b, p, c0);
-        }
-
-        template <int DIM>
-        __global__ __launch_bounds__(RB) void k_grad_apply(Bits b, const uint64_t* ca, const uint64_t* p, uint64_t* out, int* flag)
+        __global__ __launch_bounds__(RB) void k_grad_apply(Bits b, const uint64_t* ca, const uint64_t* p, uint64_t* out, int* flag,
+                                                          const uint64_t* old, int* differ)
         {
             const int64_t w = int64_t(blockIdx.x) * RB + threadIdx.x;
             if (w < b.off[b.hi + 1] - b.off[b.lo])
             {
-                grad_apply_word<DIM>(b, ca, p, out, flag, b.off[b.lo] + w);
-            }
-        }
-
-        // *flag = 1 where a and b differ
-        __global__ __launch_bounds__(RB) void k_differ(const uint64_t* a, const uint64_t* c, int64_t n, int* flag)
-        {
-            const int64_t i = int64_t(blockIdx.x) * RB + threadIdx.x;
-            if (i < n && a[i] != c[i])
-            {
-                flag[0] = 1;
+                grad_apply_word<DIM>(b, ca, p, out, flag, b.off[b.lo] + w, old, differ);
             }
         }
 
@@ -140,18 +113,17 @@ namespace smr::dev
     // ------------------------------------------------------------------
     // launchers
     // ------------------------------------------------------------------
-    void bits_zero(const Bits& b, uint64_t* bits, hipStream_t s)
+    void bits_zero(uint64_t* p, int64_t n, hipStream_t s)
     {
-        const int64_t n = b.off[b.hi + 1];
         if (n > 0)
         {
-            hipLaunchKernelGGL(k_zero_words, dim3(blocks_for(n)), dim3(RB), 0, s, bits, n);
+            hipLaunchKernelGGL(k_zero_words, dim3(blocks_for(n)), dim3(RB), 0, s, p, n);
         }
     }
 
     void bits_from_cells(const List& l, const Bits& b, uint64_t* bits, hipStream_t s)
     {
-        bits_zero(b, bits, s);
+        bits_zero(bits, b.off[b.hi + 1], s);
         if (l.nruns > 0)
         {
             hipLaunchKernelGGL(k_bits_from_runs, dim3(blocks_for(l.nruns)), dim3(RB), 0, s, l, b, bits);
@@ -161,8 +133,6 @@ namespace smr::dev
     void bits_tag_marks(int dim, const List& l, const Bits& b, const uint8_t* tag, int min_level, int max_level, uint64_t* add, uint64_t* rem,
                         hipStream_t s)
     {
-        bits_zero(b, add, s);
-        bits_zero(b, rem, s);
         if (l.ncells > 0)
         {
             if (dim == 2)
@@ -185,52 +155,23 @@ namespace smr::dev
         }
     }
 
-    void bits_graduation_pass(int dim, const Bits& b, const uint64_t* ca, uint64_t* p, uint64_t* out, int w2, int* flag, hipStream_t s)
+    void bits_graduation_pass(int dim, const Bits& b, const uint64_t* ca, uint64_t* p, uint64_t* out, int w2, int* flag, const uint64_t* old,
+                              int* differ, hipStream_t s)
     {
         const int64_t n = b.off[b.hi + 1] - b.off[b.lo];
         if (n <= 0)
         {
             return;
         }
-        bits_zero(b, p, s);
-        // the cascade: a grid-wide launch per level of more than kSmall words,
-        // then one block for the rest
-        constexpr int64_t kSmall = 1024;
-        int c = b.hi - 3;
         if (dim == 2)
         {
             hipLaunchKernelGGL(k_dilate_project<2>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, w2);
-            for (; c >= b.lo && b.off[c + 1] - b.off[c] > kSmall; --c)
-            {
-                hipLaunchKernelGGL(k_project_cascade_level<2>, dim3(blocks_for(b.off[c + 1] - b.off[c])), dim3(RB), 0, s, b, p, c);
-            }
-            if (c >= b.lo)
-            {
-                hipLaunchKernelGGL(k_project_cascade<2>, dim3(1), dim3(1024), 0, s, b, p, c);
-            }
-            hipLaunchKernelGGL(k_grad_apply<2>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, out, flag);
+            hipLaunchKernelGGL(k_grad_apply<2>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, out, flag, old, differ);
         }
         else
         {
             hipLaunchKernelGGL(k_dilate_project<3>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, w2);
-            for (; c >= b.lo && b.off[c + 1] - b.off[c] > kSmall; --c)
-            {
-                hipLaunchKernelGGL(k_project_cascade_level<3>, dim3(blocks_for(b.off[c + 1] - b.off[c])), dim3(RB), 0, s, b, p, c);
-            }
-            if (c >= b.lo)
-            {
-                hipLaunchKernelGGL(k_project_cascade<3>, dim3(1), dim3(1024), 0, s, b, p, c);
-            }
-            hipLaunchKernelGGL(k_grad_apply<3>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, out, flag);
-        }
-    }
-
-    void bits_differ(const Bits& b, const uint64_t* a, const uint64_t* c, int* flag, hipStream_t s)
-    {
-        const int64_t n = b.off[b.hi + 1];
-        if (n > 0)
-        {
-            hipLaunchKernelGGL(k_differ, dim3(blocks_for(n)), dim3(RB), 0, s, a, c, n, flag);
+            hipLaunchKernelGGL(k_grad_apply<3>, dim3(blocks_for(n)), dim3(RB), 0, s, b, ca, p, out, flag, old, differ);
         }
     }
 

@@ -105,26 +105,8 @@ namespace smr::dev
             }
         }
 
-        // one block per instance: the coarse levels of the cascade
-        __global__ __launch_bounds__(1024) void k_b_cascade(const MeshItem* items, uint64_t* p)
-        {
-            const MeshItem& it = items[blockIdx.x];
-            if (it.b.hi - 3 < it.b.lo)
-            {
-                return;
-            }
-            if (it.dim == 2)
-            {
-                cascade_levels<2>(it.b, p + it.w0, it.b.hi - 3);
-            }
-            else
-            {
-                cascade_levels<3>(it.b, p + it.w0, it.b.hi - 3);
-            }
-        }
-
         __global__ __launch_bounds__(RB) void k_b_grad_apply(const MeshItem* items, const int64_t* wpref, int n, const uint64_t* ca,
-                                                             const uint64_t* p, uint64_t* out, int* flags, int fstride, int pass)
+                                                             const uint64_t* p, uint64_t* out, int* flags, int fstride, int pass, const uint64_t* old)
         {
             const int64_t i = int64_t(blockIdx.x) * RB + threadIdx.x;
             if (i >= wpref[n])
@@ -134,24 +116,15 @@ namespace smr::dev
             const int k        = find_instance(wpref, n, i);
             const MeshItem& it = items[k];
             int* flag          = flags + int64_t(k) * fstride + pass;
+            int* differ        = flags + int64_t(k) * fstride + fstride - 1;
+            const uint64_t* o  = old ? old + it.w0 : nullptr;
             if (it.dim == 2)
             {
-                grad_apply_word<2>(it.b, ca + it.w0, p + it.w0, out + it.w0, flag, i - wpref[k]);
+                grad_apply_word<2>(it.b, ca + it.w0, p + it.w0, out + it.w0, flag, i - wpref[k], o, differ);
             }
             else
             {
-                grad_apply_word<3>(it.b, ca + it.w0, p + it.w0, out + it.w0, flag, i - wpref[k]);
-            }
-        }
-
-        // flags[k * fstride + slot] = 1 where instance k's a and c differ
-        __global__ __launch_bounds__(RB) void k_b_differ(const int64_t* wpref, int n, const uint64_t* a, const uint64_t* c, int* flags,
-                                                         int fstride, int slot)
-        {
-            const int64_t i = int64_t(blockIdx.x) * RB + threadIdx.x;
-            if (i < wpref[n] && a[i] != c[i])
-            {
-                flags[int64_t(find_instance(wpref, n, i)) * fstride + slot] = 1;
+                grad_apply_word<3>(it.b, ca + it.w0, p + it.w0, out + it.w0, flag, i - wpref[k], o, differ);
             }
         }
 
@@ -234,25 +207,15 @@ namespace smr::dev
     }
 
     void mesh_batch_graduation_pass(const MeshItem* items, const int64_t* wpref, int64_t nwords, int n, const uint64_t* ca, uint64_t* p,
-                                    uint64_t* out, int w2, int* flags, int fstride, int pass, hipStream_t s)
+                                    uint64_t* out, int w2, int* flags, int fstride, int pass, const uint64_t* old, hipStream_t s)
     {
         if (nwords <= 0)
         {
             return;
         }
-        hipLaunchKernelGGL(k_zero_words_b, dim3(blocks_for(nwords)), dim3(RB), 0, s, p, nwords);
         hipLaunchKernelGGL(k_b_dilate_project, dim3(blocks_for(nwords)), dim3(RB), 0, s, items, wpref, n, ca, p, w2);
-        hipLaunchKernelGGL(k_b_cascade, dim3(unsigned(n)), dim3(1024), 0, s, items, p);
-        hipLaunchKernelGGL(k_b_grad_apply, dim3(blocks_for(nwords)), dim3(RB), 0, s, items, wpref, n, ca, p, out, flags, fstride, pass);
-    }
-
-    void mesh_batch_differ(const int64_t* wpref, int64_t nwords, int n, const uint64_t* a, const uint64_t* c, int* flags, int fstride, int slot,
-                           hipStream_t s)
-    {
-        if (nwords > 0)
-        {
-            hipLaunchKernelGGL(k_b_differ, dim3(blocks_for(nwords)), dim3(RB), 0, s, wpref, n, a, c, flags, fstride, slot);
-        }
+        hipLaunchKernelGGL(k_b_grad_apply, dim3(blocks_for(nwords)), dim3(RB), 0, s, items, wpref, n, ca, p, out, flags, fstride, pass,
+                           old);
     }
 
     void mesh_batch_run_offsets(const MeshItem* items, const int64_t* wpref, int64_t nwords, int n, const uint64_t* bits, const int* flags,

@@ -38,12 +38,17 @@ namespace smr::dev
             }
         }
 
-        __global__ __launch_bounds__(SB) void k_sm_cells(Bits b, const uint64_t* leaves, PBits p, uint64_t* C)
+        __global__ __launch_bounds__(SB) void k_sm_cells(Bits b, const uint64_t* leaves, PBits p, uint64_t* C, uint64_t* U)
         {
             const int64_t gw = int64_t(blockIdx.x) * SB + threadIdx.x;
             if (gw < p.off[p.hi + 1])
             {
-                C[gw] = cells_word(b, leaves, p, gw);
+                const uint64_t v = cells_word(b, leaves, p, gw);
+                C[gw]            = v;
+                if (v != 0)
+                {
+                    union_up(p, U, pword(p, gw), v);
+                }
             }
         }
 
@@ -54,23 +59,6 @@ namespace smr::dev
             {
                 G[gw] = dilate_word(p, C, r, gw);
             }
-        }
-
-        // union[l - 1] for one level l
-        __global__ __launch_bounds__(SB) void k_sm_union_level(PBits p, const uint64_t* C, uint64_t* U, int l)
-        {
-            const int64_t i = int64_t(blockIdx.x) * SB + threadIdx.x;
-            if (i < p.off[l] - p.off[l - 1])
-            {
-                union_word(p, C, U, l - 1, i);
-            }
-        }
-
-        // union[l - 1] for l = l0 down to 1, by one block (small levels)
-        __global__ __launch_bounds__(1024) void k_sm_union_cascade(PBits p, const uint64_t* C, uint64_t* U, int l0)
-        {
-            __shared__ uint64_t lds[kChainWords];
-            union_chain(p, C, U, l0, lds);
         }
 
         __global__ __launch_bounds__(SB) void k_sm_coarse(PBits p, const uint64_t* C, const uint64_t* G, uint64_t* K1, uint64_t* K2)
@@ -92,16 +80,13 @@ namespace smr::dev
             }
         }
 
-        __global__ __launch_bounds__(SB) void k_sm_project_step(PBits p, uint64_t* R, const uint64_t* U, uint64_t* J, int t)
+        __global__ __launch_bounds__(SB) void k_sm_project(PBits p, uint64_t* R, const uint64_t* U, uint64_t* J)
         {
-            project_word(p, R, U, J, t, int64_t(blockIdx.x) * SB + threadIdx.x);
-        }
-
-        // projection steps t = 0 .. t1 - 1 by one block (small levels)
-        __global__ __launch_bounds__(1024) void k_sm_project_cascade(PBits p, uint64_t* R, const uint64_t* U, uint64_t* J, int t1)
-        {
-            __shared__ uint64_t lds[kChainWords];
-            project_chain(p, R, U, J, t1, lds);
+            const int64_t gw = int64_t(blockIdx.x) * SB + threadIdx.x;
+            if (gw < p.off[p.hi + 1])
+            {
+                project_word(p, R, U, J, gw);
+            }
         }
 
         // the first word of the set that holds word i of consecutive sets (a few)
@@ -163,23 +148,9 @@ namespace smr::dev
         uint64_t* J = sets + SM_PROJ_CELLS * total;
         uint64_t* U = sets + SM_UNION_CELLS * total;
         uint64_t* R = sets + SM_REFERENCE * total;
-        hipLaunchKernelGGL(k_sm_cells, dim3(sm_blocks(total)), dim3(SB), 0, st, b, leaves, p, C);
-        hipLaunchKernelGGL(k_sm_dilate, dim3(sm_blocks(total)), dim3(SB), 0, st, p, C, G, r);
-        // the union chain from the finest level down (union[hi] is empty): a
-        // launch per large level, then one block for the levels that fit in LDS
-        // (2D L4..12: from L9 on, 22.5 us; through global memory 25.5 from L8 on
-        // and 7.1 for the step from L9; 2D L2..8 16.1 instead of 25.4)
         hipLaunchKernelGGL(k_sm_zero, dim3(sm_blocks(total)), dim3(SB), 0, st, U, total);
-        int l = p.hi;
-        for (; l >= 1 && p.off[l + 1] > kChainWords; --l)
-        {
-            const int64_t n = p.off[l] - p.off[l - 1];
-            hipLaunchKernelGGL(k_sm_union_level, dim3(sm_blocks(n)), dim3(SB), 0, st, p, C, U, l);
-        }
-        if (l >= 1)
-        {
-            hipLaunchKernelGGL(k_sm_union_cascade, dim3(1), dim3(1024), 0, st, p, C, U, l);
-        }
+        hipLaunchKernelGGL(k_sm_cells, dim3(sm_blocks(total)), dim3(SB), 0, st, b, leaves, p, C, U);
+        hipLaunchKernelGGL(k_sm_dilate, dim3(sm_blocks(total)), dim3(SB), 0, st, p, C, G, r);
         uint64_t* K1 = scratch;
         uint64_t* K2 = scratch + total;
         if (mr)
@@ -187,22 +158,13 @@ namespace smr::dev
             hipLaunchKernelGGL(k_sm_coarse, dim3(sm_blocks(total)), dim3(SB), 0, st, p, C, G, K1, K2);
         }
         hipLaunchKernelGGL(k_sm_reference, dim3(sm_blocks(total)), dim3(SB), 0, st, p, G, K1, K2, R, s, mr ? 1 : 0);
-        hipLaunchKernelGGL(k_sm_zero, dim3(sm_blocks(total)), dim3(SB), 0, st, J, total);
         if (mr)
         {
-            // the projection chain from level 0 up: one block for the steps
-            // between the levels that fit in LDS, then a launch per step (2D
-            // L4..12: 15.8 us up to L8; before 12.5 up to L7 and 5.7 for the step)
-            const int t1 = chain_level(p, p.hi, kChainWords / 2);
-            if (t1 > 0)
-            {
-                hipLaunchKernelGGL(k_sm_project_cascade, dim3(1), dim3(1024), 0, st, p, R, U, J, t1);
-            }
-            for (int t = t1; t < p.hi; ++t)
-            {
-                const int64_t n = step_words(p, t);
-                hipLaunchKernelGGL(k_sm_project_step, dim3(sm_blocks(n)), dim3(SB), 0, st, p, R, U, J, t);
-            }
+            hipLaunchKernelGGL(k_sm_project, dim3(sm_blocks(total)), dim3(SB), 0, st, p, R, U, J);
+        }
+        else
+        {
+            hipLaunchKernelGGL(k_sm_zero, dim3(sm_blocks(total)), dim3(SB), 0, st, J, total);
         }
     }
 

@@ -5,9 +5,7 @@
 // each mesh's slice.  A block whose words all belong to one mesh (nearly
 // every block: a mesh holds hundreds of words or more) stages that mesh's
 // layout in LDS; a block that straddles two meshes finds each thread's mesh
-// by bisection over the prefix of padded words.  The two level chains (union
-// from the finest level down, projection from level 0 up) run as one block
-// per mesh, with block barriers between the levels.
+// by bisection over the prefix of padded words.
 #include "submesh_ops.hpp"
 
 #include <hip/hip_runtime.h>
@@ -19,18 +17,29 @@ namespace smr::dev
 
     namespace
     {
-        constexpr int CB = 1024; // threads of a chain block
-
         __device__ __forceinline__ uint64_t* item_set(const SubmeshItem& it, uint64_t* sets, int id)
         {
             return sets + SM_NSETS * it.pw0 + int64_t(id) * item_words(it);
+        }
+
+        __global__ __launch_bounds__(SB) void k_bs_zero_union(const SubmeshItem* items, const int64_t* ppref, int n, uint64_t* sets)
+        {
+            for_word(items, ppref, n, 1, [&](const SubmeshItem& it, int, int64_t gw) { item_set(it, sets, SM_UNION_CELLS)[gw] = 0; });
         }
 
         __global__ __launch_bounds__(SB) void k_bs_cells(const SubmeshItem* items, const int64_t* ppref, int n, const uint64_t* leaves,
                                                          uint64_t* sets)
         {
             for_word(items, ppref, n, 1,
-                     [&](const SubmeshItem& it, int, int64_t gw) { item_set(it, sets, SM_CELLS)[gw] = cells_word(it.b, leaves + it.lw0, it.p, gw); });
+                     [&](const SubmeshItem& it, int, int64_t gw)
+                     {
+                         const uint64_t v                = cells_word(it.b, leaves + it.lw0, it.p, gw);
+                         item_set(it, sets, SM_CELLS)[gw] = v;
+                         if (v != 0)
+                         {
+                             union_up(it.p, item_set(it, sets, SM_UNION_CELLS), pword(it.p, gw), v);
+                         }
+                     });
         }
 
         __global__ __launch_bounds__(SB) void k_bs_dilate(const SubmeshItem* items, const int64_t* ppref, int n, uint64_t* sets)
@@ -38,23 +47,6 @@ namespace smr::dev
             for_word(items, ppref, n, 1,
                      [&](const SubmeshItem& it, int, int64_t gw)
                      { item_set(it, sets, SM_CELLS_AND_GHOSTS)[gw] = dilate_word(it.p, item_set(it, sets, SM_CELLS), it.r, gw); });
-        }
-
-        // one block per item: clear union[hi], then union[l - 1] for l = hi .. 1
-        __global__ __launch_bounds__(CB) void k_bs_union(const SubmeshItem* items, uint64_t* sets)
-        {
-            __shared__ uint64_t s_raw[kItemWords];
-            __shared__ uint64_t lds[kChainWords];
-            const SubmeshItem& it = stage_item(s_raw, items[blockIdx.x]);
-            __syncthreads();
-            const PBits& p = it.p;
-            uint64_t* U    = item_set(it, sets, SM_UNION_CELLS);
-            for (int64_t i = p.off[p.hi] + threadIdx.x; i < p.off[p.hi + 1]; i += blockDim.x)
-            {
-                U[i] = 0;
-            }
-            __syncthreads();
-            union_chain(p, item_set(it, sets, SM_CELLS), U, p.hi, lds);
         }
 
         __global__ __launch_bounds__(SB) void k_bs_coarse(const SubmeshItem* items, const int64_t* ppref, int n, uint64_t* sets, uint64_t* scratch)
@@ -82,23 +74,21 @@ namespace smr::dev
                      });
         }
 
-        // one block per item: clear proj, then the projection steps t = 0 .. hi - 1
-        __global__ __launch_bounds__(CB) void k_bs_project(const SubmeshItem* items, uint64_t* sets)
+        __global__ __launch_bounds__(SB) void k_bs_project(const SubmeshItem* items, const int64_t* ppref, int n, uint64_t* sets)
         {
-            __shared__ uint64_t s_raw[kItemWords];
-            __shared__ uint64_t lds[kChainWords];
-            const SubmeshItem& it = stage_item(s_raw, items[blockIdx.x]);
-            __syncthreads();
-            uint64_t* J = item_set(it, sets, SM_PROJ_CELLS);
-            for (int64_t i = threadIdx.x; i < item_words(it); i += blockDim.x)
-            {
-                J[i] = 0;
-            }
-            __syncthreads();
-            if (it.mr)
-            {
-                project_chain(it.p, item_set(it, sets, SM_REFERENCE), item_set(it, sets, SM_UNION_CELLS), J, it.p.hi, lds);
-            }
+            for_word(items, ppref, n, 1,
+                     [&](const SubmeshItem& it, int, int64_t gw)
+                     {
+                         uint64_t* J = item_set(it, sets, SM_PROJ_CELLS);
+                         if (it.mr)
+                         {
+                             project_word(it.p, item_set(it, sets, SM_REFERENCE), item_set(it, sets, SM_UNION_CELLS), J, gw);
+                         }
+                         else
+                         {
+                             J[gw] = 0;
+                         }
+                     });
         }
 
         // run counts of word gw of the item's SM_NSETS sets, at the word's
@@ -156,12 +146,12 @@ namespace smr::dev
             return;
         }
         const dim3 g(sm_blocks(pwords));
+        hipLaunchKernelGGL(k_bs_zero_union, g, dim3(SB), 0, st, items, ppref, n, sets);
         hipLaunchKernelGGL(k_bs_cells, g, dim3(SB), 0, st, items, ppref, n, leaves, sets);
         hipLaunchKernelGGL(k_bs_dilate, g, dim3(SB), 0, st, items, ppref, n, sets);
-        hipLaunchKernelGGL(k_bs_union, dim3(unsigned(n)), dim3(CB), 0, st, items, sets);
         hipLaunchKernelGGL(k_bs_coarse, g, dim3(SB), 0, st, items, ppref, n, sets, scratch);
         hipLaunchKernelGGL(k_bs_reference, g, dim3(SB), 0, st, items, ppref, n, sets, scratch);
-        hipLaunchKernelGGL(k_bs_project, dim3(unsigned(n)), dim3(CB), 0, st, items, sets);
+        hipLaunchKernelGGL(k_bs_project, g, dim3(SB), 0, st, items, ppref, n, sets);
     }
 
     void submesh_batch_run_offsets(const SubmeshItem* items, const int64_t* ppref, int64_t pwords, int n, const uint64_t* sets, int32_t* counts,

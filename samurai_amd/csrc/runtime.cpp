@@ -2199,15 +2199,19 @@ namespace smr
         // (a later one costs another readback)
         constexpr int kPasses = 2;
         DevBuffer work;
-        uint64_t* w   = static_cast<uint64_t*>(work.get(5 * wbytes + 256, s));
+        uint64_t* w   = static_cast<uint64_t*>(work.get((4 + kPasses) * wbytes + 256, s));
         uint64_t* add = w;
         uint64_t* rem = w + nw;
-        uint64_t* buf[2] = {w + 2 * nw, w + 3 * nw};
-        uint64_t* q   = w + 4 * nw;
-        int* flags    = reinterpret_cast<int*>(w + 5 * nw); // kPasses pass flags, then the differ flag
+        // each pass's projected marks, kPasses pass flags and the differ flag,
+        // cleared together with add and rem
+        uint64_t* q          = w + 2 * nw;
+        int* flags           = reinterpret_cast<int*>(q + kPasses * nw);
+        constexpr int64_t fw = (kPasses + 2) / 2;
+        uint64_t* buf[2]     = {q + kPasses * nw + fw, q + (kPasses + 1) * nw + fw};
         int h_flags[kPasses + 1];
         {
             ScopedTimer t(&ctx, "update_cell_array_from_tag");
+            dev::bits_zero(w, (2 + kPasses) * nw + fw, s);
             dev::bits_tag_marks(cfg.dim, dm.cells.d, b, tag, cfg.min_level, cfg.max_level, add, rem, s);
             dev::bits_combine(b, old, add, rem, buf[0], s);
         }
@@ -2225,13 +2229,16 @@ namespace smr
                 {
                     throw std::logic_error("make_graduation: no fixed point");
                 }
-                hip_check(hipMemsetAsync(flags, 0, sizeof(int) * (kPasses + 1), s), "hipMemsetAsync(flags)");
+                if (batch > 0)
+                {
+                    dev::bits_zero(q, kPasses * nw + fw, s);
+                }
                 for (int p = 0; p < kPasses; ++p)
                 {
-                    dev::bits_graduation_pass(cfg.dim, b, buf[cur], q, buf[1 - cur], 2 * cfg.grad_width, flags + p, s);
+                    dev::bits_graduation_pass(cfg.dim, b, buf[cur], q + p * nw, buf[1 - cur], 2 * cfg.grad_width, flags + p,
+                                              p + 1 == kPasses ? old : nullptr, flags + kPasses, s);
                     cur = 1 - cur;
                 }
-                dev::bits_differ(b, buf[cur], old, flags + kPasses, s);
                 hip_check(hipMemcpyAsync(h_flags, flags, sizeof(h_flags), hipMemcpyDeviceToHost, s), "hipMemcpyAsync(flags)");
                 ctx.sync();
                 bool fixed = false;

@@ -116,3 +116,26 @@ def test_device_built_work_lists_match_host(gpu_ctx, dim, lmin, lmax, seed):
         assert np.array_equal(o.cells(), mesh.cells()), step
         assert np.array_equal(o.values().view(np.uint64), u.cells().view(np.uint64)), step
     assert checked > 0
+
+
+@pytest.mark.parametrize("dim,lmin,lmax,s", [(2, 1, 4, 0), (2, 1, 6, 1), (2, 1, 9, 0), (3, 1, 3, 1), (3, 1, 4, 0), (3, 2, 6, 0)])
+def test_level_chains_match_host(gpu_ctx, dim, lmin, lmax, s):
+    """The sets whose levels depend on each other (graduation marks, union,
+    projection) for rows below, of and above one word, both prediction radii
+    and as many levels as the box allows: random flags that leave jumps of
+    several levels to the graduation, then whole families coarsened."""
+    import torch
+    print("level chains", dim, lmin, lmax, s, flush=True)
+    cells = adapted_cells(dim, lmin, lmax, 1)
+    cfg = sa.mesh_config(dim, lmin, lmax, s)
+    mh = sa.make_mesh_from_cells(gpu_ctx, cfg, cells)
+    md = sa.make_mesh_from_cells(gpu_ctx, cfg, cells)
+    rng = np.random.default_rng(7 * lmax + s)
+    for rnd, kind in enumerate(["bits", "families", "bits", "families", "families"]):
+        n = mh.nb_cells(sa.REFERENCE)
+        tags = synthetic_tags(mh.cells(), n, kind, rng, dim)
+        t = torch.tensor(tags, dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        assert mh.rebuild_from_tags(tags) == md.rebuild_from_device_tags(t.data_ptr(), n), rnd
+        for mid in (sa.CELLS, sa.CELLS_AND_GHOSTS, sa.PROJ_CELLS, sa.UNION_CELLS, sa.REFERENCE):
+            assert np.array_equal(mh.cells(mid), md.cells(mid)), (rnd, mid)
