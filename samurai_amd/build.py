@@ -16,7 +16,7 @@ LIB = os.path.join(HERE, "libsamurai_amd.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 HOST_SOURCES = ["host/interval_set.cpp", "host/mr_mesh.cpp", "host/programs.cpp", "host/convection.cpp", "runtime.cpp", "batch.cpp", "adjoint.cpp", "capi.cpp"]
-HIP_SOURCES = ["device/kernels.hip", "device/ghost_flow.hip", "device/adjoint_flow.hip", "device/convection.hip", "device/program.hip", "device/noalloc.hip", "device/rebuild.hip", "device/rebuild_batch.hip", "device/submesh.hip",
+HIP_SOURCES = ["device/kernels.hip", "device/ghost_flow.hip", "device/tag_flow.hip", "device/adjoint_flow.hip", "device/convection.hip", "device/program.hip", "device/noalloc.hip", "device/rebuild.hip", "device/rebuild_batch.hip", "device/submesh.hip",
                "device/submesh_batch.hip", "device/lists.hip"]
 
 CXXFLAGS = ["-O2", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math", "-Wall", "-Wextra",

@@ -594,6 +594,9 @@ namespace smr::dev
     void criteria(int dim, const List& l, int64_t c0, int64_t c1, const double* det, uint8_t* tag, const Thresholds& thr, int min_level,
                   int max_level, hipStream_t s, int ncomp = 1, int64_t cstride = 0);
     void maximum(int dim, const List& l, int64_t c0, int64_t c1, uint8_t* tag, hipStream_t s);
+    // maximum over the whole list, whose levels ascend, from the finest down
+    // (ticket: one scratch word)
+    void tag_flow(int dim, const List& l, uint8_t* tag, unsigned* ticket, hipStream_t s);
     void tag_init(const List& l, int64_t c0, int64_t c1, uint8_t* tag, hipStream_t s);
     // p[0, n) = 0 by a kernel (graph-capturable, unlike hipMemsetAsync)
     void zero_f64(double* p, int64_t n, hipStream_t s);

@@ -2412,6 +2412,13 @@ namespace smr
         {
             ScopedTimer timer(&ctx, "tag finalization");
             const SeqPlan& plan = max_plan(ctx, dm, cfg);
+            // two launches instead of three and more (tag_flow.hip); the word
+            // behind the first field's values is free after its ghost update
+            if (plan.steps.size() > 2)
+            {
+                dev::tag_flow(dim, dm.maximum.d, tag, reinterpret_cast<unsigned*>(fs[0]->d + n), s);
+                return;
+            }
             const auto* d_items = static_cast<const dev::SeqItem*>(plan.d_items.p);
             for (const SeqPlan::Step& st : plan.steps)
             {
