@@ -302,8 +302,8 @@ def bench_3d(sa, ctx, args):
 
 def bench_convection(sa, ctx, mesh, u, a, reps):
     """The flux-based convection operators on the final adapted mesh: time per
-    call (ghost update of the inputs + gather of the ordered contribution
-    lists), after one untimed call that builds and uploads the lists."""
+    call (ghost update of the inputs + the operator), after one untimed call
+    that builds the mesh's side kinds; terms counts the interface terms."""
     from initial_conditions import centers
     c = centers(mesh.cells())
     vel = []
@@ -452,7 +452,7 @@ def bench_adjoint(sa, ctx, args, eps, reg):
         "forward_cell_updates_per_s": ncells * steps / t_fwd,
         "backward_cell_updates_per_s": ncells * steps / t_bwd,
         "fd_u0_rel_err": abs(fd_u - ad_u) / abs(ad_u), "fd_a_rel_err": abs(fd_a - ga[0, 0]) / abs(ga[0, 0]),
-        "fd_h": h, "tuning": "library default (256, 0, 3): blocks of 256, precomputed 64-cell wave items, runs of small stages as one block per instance, each checkpoint segment replayed as a HIP graph",
+        "fd_h": h, "tuning": "library default: each checkpoint segment, and its adjoint, one dataflow launch over all instances",
         "setup_s": setup, "cpu_baseline_forward": cpu,
     }
 
