@@ -1369,11 +1369,14 @@ namespace smr
     // when the recipes have no such form.  A single field takes it
     // (dm.ghost_flow_pays) unless the staged launches cost at most 11 us by the
     // count below (the reset and the flow take 9 to 17): a run of stages in one
-    // block 2 us and 0.9 us per 1024 ghosts of each, a grid-wide stage 3.5 us.
+    // block 2 us and 0.9 us per 1024 ghosts of each (2D of prediction radius 0,
+    // one source per prediction: 0.45), a grid-wide stage 3.5 us.
     // Measured, the stages against the flow, with the operator that follows:
     // WENO5 2D L7 13.4 / 17.3 us, L8 16.2 / 17.1, L9 22.0 / 19.2 (uniform meshes,
     // 3 to 4 wide ghost stages); upwind, 348 ghosts in 9 stages 10.8 / 14.1, 570
-    // in 10 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7.
+    // in 10 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7; radius 0,
+    // three updates and a flux operator: 2D L2..7 38.4 / 44.0, 3D L2..4 (four)
+    // 67.6 / 63.0.
     const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
     {
         const RecipeFlow& rf = dm.recipe_flow;
@@ -1394,7 +1397,7 @@ namespace smr
                 }
                 else if (n > 0)
                 {
-                    staged_us += (in_block ? 0.0 : 2.0) + 0.9 * double((n + 1023) / 1024);
+                    staged_us += (in_block ? 0.0 : 2.0) + (cfg.dim == 2 && cfg.pred_s == 0 ? 0.45 : 0.9) * double((n + 1023) / 1024);
                     in_block = true;
                 }
             };
