@@ -250,6 +250,17 @@ int smr_mesh_validate(const smr_mesh* mesh);
  * mesh.  0 if identical, 1 if the image has no device-built lists,
  * SMR_ERR_RUNTIME if they differ. */
 int smr_mesh_check_device_lists(smr_mesh* mesh);
+/* Diagnostics (no counterpart in the reference): how update_ghost_mr of a field
+ * with a B.C. runs on the mesh.  0: a launch per stage (the mesh does not tile
+ * the box, or its outer ghosts need that order; also with
+ * smr_ctx_set_ghost_form 0), 1: the same, although a dataflow launch exists,
+ * because it is estimated to be cheaper, 2: the dataflow launch.  On a
+ * host-only context 0 or 1: whether the dataflow launch exists. */
+int smr_mesh_ghost_form(smr_mesh* mesh);
+/* Diagnostics: the form of update_ghost_mr on this context's meshes.  -1 (the
+ * default): the cheaper one; 0: the launches per stage; 1: the dataflow launch
+ * wherever it exists. */
+int smr_ctx_set_ghost_form(smr_ctx* ctx, int form);
 /* The HIP stream (hipStream_t) the context orders its work on, for timing
  * with HIP events; NULL for a host-only context. */
 void* smr_ctx_stream(smr_ctx* ctx);

@@ -80,6 +80,8 @@ def lib():
         _sig(L, "smr_mesh_check_device_lists", "argtypes", [vp])
         _sig(L, "smr_mesh_ghost_update_bytes", "restype", i64)
         _sig(L, "smr_mesh_ghost_update_bytes", "argtypes", [vp])
+        _sig(L, "smr_mesh_ghost_form", "argtypes", [vp])
+        _sig(L, "smr_ctx_set_ghost_form", "argtypes", [vp, i32])
         _sig(L, "smr_timers_enable", "argtypes", [i32])
         _sig(L, "smr_timers_report", "restype", i64)
         _sig(L, "smr_timers_report", "argtypes", [ctypes.c_char_p, i64])
@@ -200,6 +202,10 @@ class Context:
     def synchronize(self):
         _check(lib().smr_ctx_synchronize(self.h))
 
+    def set_ghost_form(self, form):
+        """-1: update_ghost_mr in its cheaper form (the default), 0: a launch per stage, 1: the dataflow launch wherever it exists."""
+        _check(lib().smr_ctx_set_ghost_form(self.h, int(form)))
+
     def stream(self):
         """The hipStream_t (as an integer) all work of this context runs on."""
         return lib().smr_ctx_stream(self.h)
@@ -275,6 +281,11 @@ class MRMesh(_Handle):
     def check_device_lists(self):
         """0 when the work lists the device built for this mesh equal the host's, 1 when it built none."""
         return _check(lib().smr_mesh_check_device_lists(self.h))
+
+    def ghost_form(self):
+        """How update_ghost_mr of a field with a B.C. runs here: 2 one dataflow launch, 1 a launch per stage (estimated cheaper), 0 a
+        launch per stage (there is no other form).  Host-only contexts: 1 if the dataflow launch exists, else 0."""
+        return _check(lib().smr_mesh_ghost_form(self.h))
 
     def refresh_config(self):
         """Re-read the configuration (the levels change when a restart file is loaded into the mesh)."""

@@ -1165,7 +1165,7 @@ namespace smr
         for (const Instance& in : inst_)
         {
             const MeshConfig& c = in.mesh->host.cfg;
-            if (!in.has_bc || c.dim != c0.dim || c.pred_s != c0.pred_s)
+            if (!in.has_bc || !in.mesh->host.tiles || c.dim != c0.dim || c.pred_s != c0.pred_s)
             {
                 return nullptr;
             }

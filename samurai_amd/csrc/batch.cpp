@@ -1478,8 +1478,8 @@ namespace smr
                                          r.converged = true;
                                          return;
                                      }
-                                     r.nm           = dev_ids ? std::move(nms[size_t(q)]) : build_mesh(c, std::move(cas[size_t(q)]));
-                                     r.nm.graduated = true;
+                                     r.nm = dev_ids ? std::move(nms[size_t(q)]) : build_mesh(c, std::move(cas[size_t(q)]));
+                                     adapted_from(r.nm, m.host);
                                      if (dev_lists)
                                      {
                                          r.device_lists = true;
@@ -1515,9 +1515,9 @@ namespace smr
                                          r.converged = true;
                                          return;
                                      }
-                                     r.nm           = build_mesh(c, std::move(ca));
-                                     r.nm.graduated = true;
-                                     r.img          = build_host_image(r.nm);
+                                     r.nm = build_mesh(c, std::move(ca));
+                                     adapted_from(r.nm, m.host);
+                                     r.img = build_host_image(r.nm);
                                      build_update_fields_lists(m.host, r.nm, r.copy, r.coarsen, r.refine);
                                  });
                 }
@@ -1788,7 +1788,7 @@ namespace smr
             const Field& u      = *inst_[size_t(ids[k])].u;
             const MeshConfig& c = u.mesh->host.cfg;
             const MeshConfig& d = inst_[size_t(ids[0])].u->mesh->host.cfg;
-            form[k]             = u.has_bc && c.dim == d.dim && c.pred_s == d.pred_s ? ghost_flow(*u.mesh->dev, c) : nullptr;
+            form[k]             = u.has_bc && c.dim == d.dim && c.pred_s == d.pred_s ? ghost_flow(*ctx_, *u.mesh->dev, c) : nullptr;
             if (!form[k])
             {
                 return;

@@ -103,7 +103,7 @@ namespace
     }
 
     // MRMesh(ca, cfg) (mr/mesh.hpp:386-396) from leaves given as rows
-    // (level, x, y, z); graduated is recorded, not enforced
+    // (level, x, y, z); graduated and tiles are recorded, not enforced
     smr::MRMeshData mesh_from_cells(const smr::MeshConfig& c, const int32_t* cells, int64_t n)
     {
         require(n >= 0, "negative cell count");
@@ -123,6 +123,7 @@ namespace
         smr::make_graduation(g, c.dim, c.grad_width);
         smr::MRMeshData m = smr::build_mesh(c, ca);
         m.graduated       = smr::ca_equal(g, ca);
+        m.tiles           = smr::tiles_box(m, false);
         return m;
     }
 
@@ -365,8 +366,8 @@ extern "C"
                 if (nm.nref < 0)
                 {
                     smr::ScopedTimer t3(nullptr, "mesh construction");
-                    nm           = smr::build_mesh(mm.host.cfg, ca);
-                    nm.graduated = true;
+                    nm = smr::build_mesh(mm.host.cfg, ca);
+                    smr::adapted_from(nm, mm.host);
                 }
                 mm.replace(std::move(nm), nullptr);
                 return 0;
@@ -397,8 +398,8 @@ extern "C"
                 smr::MRMeshData nm;
                 {
                     smr::ScopedTimer t3(nullptr, "mesh construction");
-                    nm           = smr::build_mesh(m.cfg, ca);
-                    nm.graduated = true;
+                    nm = smr::build_mesh(m.cfg, ca);
+                    smr::adapted_from(nm, m);
                 }
                 smr::WorkList copy, coarsen, refine;
                 smr::build_update_fields_lists(m, nm, copy, coarsen, refine);
@@ -583,6 +584,40 @@ extern "C"
                 {
                     throw std::out_of_range(why);
                 }
+                return 0;
+            });
+    }
+
+    int smr_mesh_ghost_form(smr_mesh* mesh)
+    {
+        return guarded(
+            [&]
+            {
+                require(mesh != nullptr, "null mesh");
+                smr::Mesh& m = mesh->m;
+                if (!m.ctx->has_device())
+                {
+                    const smr::GhostProgram g = smr::build_ghost_program(m.host);
+                    std::vector<const smr::Recipes*> levels;
+                    for (const smr::Recipes& r : g.outer)
+                    {
+                        levels.push_back(&r);
+                    }
+                    return m.host.tiles && smr::build_recipe_flow(levels, m.host.nref).ok ? 1 : 0;
+                }
+                smr::DevMesh& dm                = m.device_ghost();
+                const smr::dev::GhostFlow* flow = smr::ghost_flow(*m.ctx, dm, m.host.cfg);
+                return smr::takes_ghost_flow(*m.ctx, dm, flow) ? 2 : (flow ? 1 : 0);
+            });
+    }
+
+    int smr_ctx_set_ghost_form(smr_ctx* ctx, int form)
+    {
+        return guarded(
+            [&]
+            {
+                require(ctx && form >= -1 && form <= 1, "a ghost form of -1, 0 or 1 is expected");
+                ctx->c.ghost_form = form;
                 return 0;
             });
     }

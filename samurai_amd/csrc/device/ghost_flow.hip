@@ -21,7 +21,8 @@
 // (5.9 K cells) 19 against 26.
 //
 // Every wait ends.  Blocks take their place in the order of the ghosts from a
-// counter (the ticket), the order keeps every source before its readers, so
+// counter (the ticket), and the order keeps every source before its readers
+// where the cells tile the box (the other meshes keep the staged launches), so
 // the lowest unfinished wave waits for nothing that is not done; and a wave
 // gives up after kMaxSpins rounds and uses what it has read (which is the
 // right value when a cell itself holds the bits of the mark).

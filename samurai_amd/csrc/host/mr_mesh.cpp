@@ -374,7 +374,50 @@ namespace smr
         cells[size_t(cfg.max_level)]   = domain_at(cfg.dim, cfg.max_level);
         MRMeshData m                   = build_mesh(cfg, cells);
         m.graduated                    = true; // a single level
+        m.tiles                        = true;
         return m;
+    }
+
+    bool tiles_box(const MRMeshData& m, bool covered)
+    {
+        // in units of a cell of the finest level there can be: exact, the box
+        // being 2^60 of them in 3D
+        uint64_t volume = 0;
+        for (int l = 0; l < MAXL; ++l)
+        {
+            volume += uint64_t(m.ids[CELLS][size_t(l)].count()) << (m.cfg.dim * (MAXL - 1 - l));
+        }
+        if (volume != uint64_t(1) << (m.cfg.dim * (MAXL - 1)))
+        {
+            return false;
+        }
+        if (covered)
+        {
+            return true;
+        }
+        LevelSet above(m.cfg.dim, MAXL - 1); // the cells of this level with finer leaves in them
+        for (int l = MAXL - 1; l >= 0; --l)
+        {
+            const LevelSet& c = m.ids[CELLS][size_t(l)];
+            const int n       = 1 << l;
+            if ((l > m.cfg.max_level && !c.empty()) || !minus_box(c, {0, 0, 0}, {n, n, n}).empty() || !set_intersection(c, above).empty())
+            {
+                return false;
+            }
+            if (l > 0)
+            {
+                above = on(set_union(c, above), l - 1);
+            }
+        }
+        return true;
+    }
+
+    void adapted_from(MRMeshData& m, const MRMeshData& old)
+    {
+        m.graduated = true;
+        // a leaf is replaced by its children or its parent, never by less: the
+        // leaves still cover what they covered
+        m.tiles = tiles_box(m, old.tiles);
     }
 
     CellArray update_cell_array_from_tag(const MRMeshData& mesh, const uint8_t* tags)

@@ -63,6 +63,9 @@ namespace smr
         int64_t nref = 0;
         // the cells are known to satisfy the graduation (make_graduation leaves them unchanged)
         bool graduated = false;
+        // the cells tile the unit box (no hole, no overlap, none outside) on
+        // levels up to max_level
+        bool tiles = false;
 
         const LevelSet& get(int id, int level) const { return ids[id][size_t(level)]; }
         // storage index of a reference cell; throws std::out_of_range if absent
@@ -79,6 +82,11 @@ namespace smr
     // corners and renumbering of a mesh whose five ids are set (the ids built
     // elsewhere, e.g. on the device, as build_mesh would build them)
     void complete_mesh(MRMeshData& m);
+    // whether m's cells tile the unit box, from their volume alone when they are
+    // known to cover it
+    bool tiles_box(const MRMeshData& m, bool covered);
+    // sets the properties of m, the graduated mesh that tags made of `old`
+    void adapted_from(MRMeshData& m, const MRMeshData& old);
     // mra::make_mesh(unit box, cfg): all cells at max_level (mr/mesh.hpp:510-518)
     MRMeshData build_box_mesh(const MeshConfig& cfg);
 

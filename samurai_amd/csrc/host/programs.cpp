@@ -1222,6 +1222,98 @@ namespace smr
         return a == b ? "" : "values differ from the staged recipes";
     }
 
+    std::string validate_flow_order(const MRMeshData& m, const GhostProgram& g)
+    {
+        std::vector<const Recipes*> levels;
+        for (const Recipes& r : g.outer)
+        {
+            levels.push_back(&r);
+        }
+        const RecipeFlow f = build_recipe_flow(levels, m.nref);
+        if (!m.tiles || !f.ok)
+        {
+            return "";
+        }
+        // the turn in which a slot is written: 3 per level of the way down
+        // (recipes before the projection below), then the predictions
+        std::vector<int> turn(size_t(m.nref), -1);
+        std::string why;
+        // dst and reads(source) of the cells of a list's level
+        auto cells = [&](const WorkList& w, int level, bool fine, auto&& each)
+        {
+            int64_t r0       = 0;
+            const int64_t nr = w.runs_of_levels(level, level + 1, r0);
+            for (int64_t k = r0; k < r0 + nr; ++k)
+            {
+                const int32_t* iv = &w.iv[size_t(5 * k)];
+                for (int32_t x = iv[0]; x < iv[1]; ++x)
+                {
+                    std::vector<int64_t> src;
+                    const int s = m.cfg.pred_s, lo = fine ? 0 : -s, hi = fine ? 1 : s;
+                    for (int dz = m.cfg.dim == 3 ? lo : 0; dz <= (m.cfg.dim == 3 ? hi : 0); ++dz)
+                    {
+                        for (int dy = lo; dy <= hi; ++dy)
+                        {
+                            for (int dx = lo; dx <= hi; ++dx)
+                            {
+                                src.push_back(fine ? m.index(level + 1, 2 * x + dx, 2 * iv[2] + dy, 2 * iv[3] + dz)
+                                                   : m.index(level - 1, (x >> 1) + dx, (iv[2] >> 1) + dy, (iv[3] >> 1) + dz));
+                            }
+                        }
+                    }
+                    each(m.index(level, x, iv[2], iv[3]), src);
+                }
+            }
+        };
+        // what: 0 note who writes, 1 compare with who reads
+        for (int what = 0; what < 2; ++what)
+        {
+            auto op = [&](int t, int64_t dst, const std::vector<int64_t>& src, const char* name)
+            {
+                if (what == 0)
+                {
+                    if (turn[size_t(dst)] >= 0)
+                    {
+                        why = std::string(name) + " writes a slot again";
+                    }
+                    turn[size_t(dst)] = t;
+                    return;
+                }
+                for (int64_t s : src)
+                {
+                    // recipes of one level may read each other (validate_recipe_flow)
+                    if (turn[size_t(s)] > t || (turn[size_t(s)] == t && t % 3 != 0))
+                    {
+                        why = std::string(name) + " reads a slot written later";
+                    }
+                }
+            };
+            for (int level = MAXL - 1; level >= 0; --level)
+            {
+                const int t = 3 * (MAXL - level);
+                for (int32_t q = f.level[size_t(level) + 1]; q < f.level[size_t(level)]; ++q)
+                {
+                    const int32_t* r = &f.rec[size_t(4 * q)];
+                    std::vector<int64_t> src;
+                    for (int k = 0; k < (r[1] >> 8); ++k)
+                    {
+                        src.push_back(f.src[size_t(r[3] + k)]);
+                    }
+                    op(t, r[0], src, "a recipe");
+                }
+                if (level > 0)
+                {
+                    cells(g.projection, level - 1, true, [&](int64_t d, const std::vector<int64_t>& src) { op(t + 1, d, src, "a projection"); });
+                }
+            }
+            for (int level = 1; level < MAXL; ++level)
+            {
+                cells(g.prediction, level, false, [&](int64_t d, const std::vector<int64_t>& src) { op(3 * (MAXL + level) + 2, d, src, "a prediction"); });
+            }
+        }
+        return why;
+    }
+
     std::string validate_programs(const MRMeshData& m)
     {
         std::string why = validate_list(build_cells_list(m), m, m);
@@ -1241,6 +1333,10 @@ namespace smr
         if (!(why = validate_recipe_flow(g.outer, m.nref)).empty())
         {
             return "recipe flow: " + why;
+        }
+        if (!(why = validate_flow_order(m, g)).empty())
+        {
+            return "flow order: " + why;
         }
         AdaptProgram a = build_adapt_program(m);
         if (!(why = validate_list(a.detail, m, m)).empty())

@@ -86,7 +86,11 @@ namespace smr
     // anything reads it is left out.  ok is false when a recipe reads a slot
     // that a later recipe writes (then only the staged order gives its value).
     // Recipes read cells and slots outside the domain only, so projections
-    // and predictions (inside) are no part of this.
+    // and predictions (inside) are no part of this.  Among those every source
+    // precedes its readers on meshes whose cells tile the box, and on these the
+    // dataflow forms run: a child of a projected cell is then a cell or projected
+    // itself.  Where a leaf is missing it is predicted, from the very cell that
+    // reads it, and only the staged order has a value for either.
     struct RecipeFlow
     {
         bool ok = false;
@@ -150,6 +154,10 @@ namespace smr
     // the recipe flow writes each slot once, after its sources, and leaves the
     // values of the staged recipes
     std::string validate_recipe_flow(const std::vector<Recipes>& outer, int64_t nref);
-    // validate_list over every list of the mesh's programs, and the recipe flow
+    // on meshes that tile the box: the dataflow order (recipes and projection of
+    // each level, finest first, then the predictions) writes each slot once and
+    // after its sources
+    std::string validate_flow_order(const MRMeshData& m, const GhostProgram& g);
+    // validate_list over every list of the mesh's programs, the recipe flow and the flow order
     std::string validate_programs(const MRMeshData& m);
 } // namespace smr

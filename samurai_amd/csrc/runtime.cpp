@@ -468,14 +468,18 @@ namespace smr
             });
     }
 
-    void Packer::recipe_flow(DevMesh& dm, int64_t nref)
+    void Packer::recipe_flow(DevMesh& dm, const MRMeshData& m)
     {
+        if (!m.tiles)
+        {
+            return;
+        }
         std::vector<const Recipes*> outer;
         for (const DevRecipes& r : dm.outer)
         {
             outer.push_back(&r.host);
         }
-        dm.recipe_flow = build_recipe_flow(outer, nref);
+        dm.recipe_flow = build_recipe_flow(outer, m.nref);
         if (!dm.recipe_flow.ok)
         {
             return;
@@ -803,7 +807,7 @@ namespace smr
             dm.outer[l].host = std::move(h.ghost.outer[l]);
             p.recipes(dm.outer[l]);
         }
-        p.recipe_flow(dm, m.nref);
+        p.recipe_flow(dm, m);
         dm.cells.host      = std::move(h.cells);
         dm.projection.host = std::move(h.ghost.projection);
         dm.prediction.host = std::move(h.ghost.prediction);
@@ -941,7 +945,7 @@ namespace smr
             dm.outer[k].host = std::move(outer[k]);
             p.recipes(dm.outer[k]);
         }
-        p.recipe_flow(dm, m.nref);
+        p.recipe_flow(dm, m);
         dm.cells.host = std::move(cells);
         p.list(dm.cells);
         DevWorkList* dls[dev::DL_UF_COPY] = {&dm.projection, &dm.prediction, &dm.detail, &dm.criteria, &dm.maximum};
@@ -1133,7 +1137,7 @@ namespace smr
             }
             dm.flow_blob = std::make_unique<Blob>();
             Packer p(*dm.flow_blob);
-            p.recipe_flow(dm, host.nref);
+            p.recipe_flow(dm, host);
             p.finish(ctx->stream);
             dm.projection.host = std::move(gp.projection);
             dm.prediction.host = std::move(gp.prediction);
@@ -1366,7 +1370,7 @@ namespace smr
 
     // The dataflow launch of dm's update_ghost_mr for a field with a B.C.: the
     // stages of ghost_plan in order, the recipes of a level as one item; null
-    // when the recipes have no such form.  A single field takes it
+    // when the mesh does not tile the box or the recipes have no such form.  A single field takes it
     // (dm.ghost_flow_pays) unless the staged launches cost at most 11 us by the
     // count below (the reset and the flow take 9 to 17): a run of stages in one
     // block 2 us and 0.9 us per 1024 ghosts of each (2D of prediction radius 0,
@@ -1377,10 +1381,10 @@ namespace smr
     // in 10 13.8 / 14.6, 324 in 12 15.2 / 13.6, 579 in 14 18.3 / 14.7; radius 0,
     // three updates and a flux operator: 2D L2..7 38.4 / 44.0, 3D L2..4 (four)
     // 67.6 / 63.0.
-    const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg)
+    const dev::GhostFlow* ghost_flow(const Ctx& ctx, DevMesh& dm, const MeshConfig& cfg)
     {
         const RecipeFlow& rf = dm.recipe_flow;
-        if (!rf.ok)
+        if (!rf.ok || ctx.ghost_form == 0)
         {
             return nullptr;
         }
@@ -1448,6 +1452,11 @@ namespace smr
         return dm.ghost_flow.get();
     }
 
+    bool takes_ghost_flow(const Ctx& ctx, const DevMesh& dm, const dev::GhostFlow* flow)
+    {
+        return flow && (dm.ghost_flow_pays || ctx.ghost_form == 1);
+    }
+
     void update_ghost_mr(Field& f)
     {
         f.check_current();
@@ -1458,8 +1467,8 @@ namespace smr
         const int dim   = m.host.cfg.dim;
         const int ps    = m.host.cfg.pred_s;
         const double bc = f.bc_value;
-        const dev::GhostFlow* flow = f.has_bc ? ghost_flow(dm, m.host.cfg) : nullptr;
-        if (flow && dm.ghost_flow_pays)
+        const dev::GhostFlow* flow = f.has_bc ? ghost_flow(*m.ctx, dm, m.host.cfg) : nullptr;
+        if (takes_ghost_flow(*m.ctx, dm, flow))
         {
             dev::ghost_flow(dim, ps, *flow, f.d, m.host.nref, bc, s);
             return;
@@ -2277,8 +2286,8 @@ namespace smr
                 dev::submesh_build(b, old, p, cfg.radius, cfg.pred_s, cfg.max_level != cfg.min_level, o, o + dev::SM_NSETS * total, s);
                 old_sets = o;
             }
-            *mesh           = device_submesh(ctx, cfg, b, buf[cur], *current, old_sets, lists);
-            mesh->graduated = true;
+            *mesh = device_submesh(ctx, cfg, b, buf[cur], *current, old_sets, lists);
+            adapted_from(*mesh, *current);
             return true;
         }
         ScopedTimer t(&ctx, "leaves to host");
@@ -2483,8 +2492,8 @@ namespace smr
             if (nm.nref < 0)
             {
                 ScopedTimer t3(nullptr, "mesh construction");
-                nm           = build_mesh(cfg, std::move(new_ca));
-                nm.graduated = true;
+                nm = build_mesh(cfg, std::move(new_ca));
+                adapted_from(nm, m.host);
             }
         }
         if (dl.nlists == int(dev::DL_N))

@@ -265,8 +265,8 @@ namespace smr
         // several lists, their host arrays prepared in parallel
         void lists(const std::vector<DevWorkList*>& ls);
         void recipes(DevRecipes& r);
-        // the dataflow form of dm's recipes (dm.outer, whose host arrays are set)
-        void recipe_flow(DevMesh& dm, int64_t nref);
+        // the dataflow form of m's recipes (dm.outer, whose host arrays are set)
+        void recipe_flow(DevMesh& dm, const MRMeshData& m);
         // a list whose runs, prefixes and hints the device built (at iv,
         // pref, hint); its taps come from l.host
         void device_list(DevWorkList& l, const int32_t* iv, const int64_t* pref, const int32_t* hint, int64_t nruns, int64_t ncells);
@@ -360,6 +360,9 @@ namespace smr
         // recorded after a new mesh's runs are read back, so that the host can
         // complete the mesh while later kernels run
         hipEvent_t runs_back = nullptr;
+        // update_ghost_mr: -1 the cheaper form, 0 the staged launches, 1 the
+        // dataflow launch wherever there is one
+        int ghost_form = -1;
         void mark_runs_back();
         ~Ctx();
         int* d_flag() const { return d_err + 1; }
@@ -491,7 +494,9 @@ namespace smr
     void update_ghost_mr(Field& f);
     // the dataflow form of dm's ghost update, put together on first use; null
     // when there is none
-    const dev::GhostFlow* ghost_flow(DevMesh& dm, const MeshConfig& cfg);
+    const dev::GhostFlow* ghost_flow(const Ctx& ctx, DevMesh& dm, const MeshConfig& cfg);
+    // whether the update of one field takes it (flow: ghost_flow's)
+    bool takes_ghost_flow(const Ctx& ctx, const DevMesh& dm, const dev::GhostFlow* flow);
     void upwind(const double* a, double dt, Field& u, Field& unp1);
     // out = u - a * v on the cells (the field expression of the flux-based demos)
     void sub_scaled(Field& u, double a, Field& v, Field& out);
