@@ -261,6 +261,11 @@ int smr_mesh_ghost_form(smr_mesh* mesh);
  * default): the cheaper one; 0: the launches per stage; 1: the dataflow launch
  * wherever it exists. */
 int smr_ctx_set_ghost_form(smr_ctx* ctx, int form);
+/* Diagnostics: the rounds after which a wave of a dataflow launch gives up
+ * waiting for a value (default 2^17).  The next call that waits for the
+ * context's work then returns SMR_ERR_RUNTIME, unless the value is one the
+ * launch does not write. */
+int smr_ctx_set_wait_rounds(smr_ctx* ctx, int rounds);
 /* The HIP stream (hipStream_t) the context orders its work on, for timing
  * with HIP events; NULL for a host-only context. */
 void* smr_ctx_stream(smr_ctx* ctx);

@@ -82,6 +82,7 @@ def lib():
         _sig(L, "smr_mesh_ghost_update_bytes", "argtypes", [vp])
         _sig(L, "smr_mesh_ghost_form", "argtypes", [vp])
         _sig(L, "smr_ctx_set_ghost_form", "argtypes", [vp, i32])
+        _sig(L, "smr_ctx_set_wait_rounds", "argtypes", [vp, i32])
         _sig(L, "smr_timers_enable", "argtypes", [i32])
         _sig(L, "smr_timers_report", "restype", i64)
         _sig(L, "smr_timers_report", "argtypes", [ctypes.c_char_p, i64])
@@ -205,6 +206,10 @@ class Context:
     def set_ghost_form(self, form):
         """-1: update_ghost_mr in its cheaper form (the default), 0: a launch per stage, 1: the dataflow launch wherever it exists."""
         _check(lib().smr_ctx_set_ghost_form(self.h, int(form)))
+
+    def set_wait_rounds(self, rounds):
+        """After how many rounds a wave of a dataflow launch gives up waiting (diagnostics; the default is 2**17)."""
+        _check(lib().smr_ctx_set_wait_rounds(self.h, int(rounds)))
 
     def stream(self):
         """The hipStream_t (as an integer) all work of this context runs on."""

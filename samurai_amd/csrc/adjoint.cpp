@@ -1411,7 +1411,7 @@ namespace smr
         for (int sg = 0; sg < nseg_; ++sg)
         {
             double* at = w.ckpt + int64_t(sg) * w.f.n;
-            dev::adjoint_flow_forward(w.f, {at, w.states, at + w.f.n, every_}, true, ticket, s);
+            dev::adjoint_flow_forward(w.f, {at, w.states, at + w.f.n, every_}, true, ticket, ctx_->wait, s);
         }
         dev::adjoint_flow_cells(w.f, w.ckpt + int64_t(nseg_) * w.f.n, uT, true, s);
     }
@@ -1429,12 +1429,12 @@ namespace smr
         {
             double* at = w.ckpt + int64_t(sg) * w.f.n;
             const dev::FlowArrays states{at, w.states, at + w.f.n, every_};
-            dev::adjoint_flow_forward(w.f, states, false, ticket, s);
+            dev::adjoint_flow_forward(w.f, states, false, ticket, ctx_->wait, s);
             for (int done = 0; done < every_;)
             {
                 const int k = std::min(kFlowSteps, every_ - done);
                 const dev::FlowArrays lam{end[cur], w.between, end[1 - cur], k};
-                dev::adjoint_flow_backward(w.f, lam, ticket, s);
+                dev::adjoint_flow_backward(w.f, lam, ticket, ctx_->wait, s);
                 dev::adjoint_flow_velocity(w.f, lam, states, every_ - 1 - done, ga_arena_, s);
                 done += k;
                 cur = 1 - cur;

@@ -1825,7 +1825,7 @@ namespace smr
     {
         if (fs.ok)
         {
-            dev::ghost_flow_batch(fs.dim, fs.ps, fs.inst, fs.pref, fs.n, fs.nwaves, fs.ticket, ctx_->stream);
+            dev::ghost_flow_batch(fs.dim, fs.ps, fs.inst, fs.pref, fs.n, fs.nwaves, fs.ticket, ctx_->wait, ctx_->stream);
         }
     }
 

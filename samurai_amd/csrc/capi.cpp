@@ -177,6 +177,7 @@ extern "C"
                                        "hipMemPoolSetAttribute");
                         smr::hip_check(hipMalloc(reinterpret_cast<void**>(&c->c.d_err), 2 * sizeof(int)), "hipMalloc(err)");
                         smr::hip_check(hipMemsetAsync(c->c.d_err, 0, 2 * sizeof(int), c->c.stream), "hipMemsetAsync(err)");
+                        c->c.allocate_fault_words();
                         c->c.sync();
                         smr::noalloc_init(device);
                     }
@@ -618,6 +619,17 @@ extern "C"
             {
                 require(ctx && form >= -1 && form <= 1, "a ghost form of -1, 0 or 1 is expected");
                 ctx->c.ghost_form = form;
+                return 0;
+            });
+    }
+
+    int smr_ctx_set_wait_rounds(smr_ctx* ctx, int rounds)
+    {
+        return guarded(
+            [&]
+            {
+                require(ctx && rounds >= 0, "a number of rounds is expected");
+                ctx->c.wait.rounds = rounds;
                 return 0;
             });
     }

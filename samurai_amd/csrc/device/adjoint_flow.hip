@@ -58,7 +58,7 @@ namespace smr::dev
         }
 
         template <int DIM, int S>
-        __device__ __forceinline__ void ghost_project(const int32_t* __restrict__ tab, int64_t c, bool active, double* u)
+        __device__ __forceinline__ uint64_t ghost_project(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NR     = 1 << (DIM - 1);
             constexpr double inv = 1.0 / double(1 << DIM);
@@ -73,26 +73,27 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + r[1 + (k >> 1)] + (k & 1); };
             Sources<2 * NR, decltype(at)> s;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           if (!s.ready(at) && !last)
-                           {
-                               return false;
-                           }
-                           double sum = 0;
+            auto attempt = [&](bool last) -> int
+            {
+                const bool ok = s.ready(at);
+                if (!ok && !last)
+                {
+                    return WAITS;
+                }
+                double sum = 0;
 #pragma unroll
-                           for (int q = 0; q < NR; ++q)
-                           {
-                               sum += s.v[2 * q] + s.v[2 * q + 1];
-                           }
-                           publish(u + r[0], sum * inv);
-                           return true;
-                       });
+                for (int q = 0; q < NR; ++q)
+                {
+                    sum += s.v[2 * q] + s.v[2 * q + 1];
+                }
+                publish(u + r[0], sum * inv);
+                return ok ? DONE : MISSED;
+            };
+            return until_done(active, w, attempt);
         }
 
         template <int DIM, int S>
-        __device__ __forceinline__ void ghost_predict(const int32_t* __restrict__ tab, int64_t c, bool active, double* u)
+        __device__ __forceinline__ uint64_t ghost_predict(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NY = 2 * S + 1, NZ = DIM == 3 ? NY : 1;
             int32_t r[1 + NZ * NY] = {};
@@ -106,34 +107,35 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + r[1 + k / NY] + k % NY; };
             Sources<NZ * NY * NY, decltype(at)> s;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           if (!s.ready(at) && !last)
-                           {
-                               return false;
-                           }
-                           double v = s.v[0];
-                           if constexpr (S == 1)
-                           {
-                               const int px = (r[0] >> 28) & 1, py = (r[0] >> 29) & 1, pz = (r[0] >> 30) & 1;
-                               v            = 0;
+            auto attempt = [&](bool last) -> int
+            {
+                const bool ok = s.ready(at);
+                if (!ok && !last)
+                {
+                    return WAITS;
+                }
+                double v = s.v[0];
+                if constexpr (S == 1)
+                {
+                    const int px = (r[0] >> 28) & 1, py = (r[0] >> 29) & 1, pz = (r[0] >> 30) & 1;
+                    v            = 0;
 #pragma unroll
-                               for (int k = 0; k < NZ * 9; ++k)
-                               {
-                                   double coeff = 1.;
-                                   coeff *= pcoef(px, k % 3);
-                                   coeff *= pcoef(py, (k / 3) % 3);
-                                   if constexpr (DIM == 3)
-                                   {
-                                       coeff *= pcoef(pz, k / 9);
-                                   }
-                                   v += s.v[k] * coeff;
-                               }
-                           }
-                           publish(u + (r[0] & kFlowSlotMask), v);
-                           return true;
-                       });
+                    for (int k = 0; k < NZ * 9; ++k)
+                    {
+                        double coeff = 1.;
+                        coeff *= pcoef(px, k % 3);
+                        coeff *= pcoef(py, (k / 3) % 3);
+                        if constexpr (DIM == 3)
+                        {
+                            coeff *= pcoef(pz, k / 9);
+                        }
+                        v += s.v[k] * coeff;
+                    }
+                }
+                publish(u + (r[0] & kFlowSlotMask), v);
+                return ok ? DONE : MISSED;
+            };
+            return until_done(active, w, attempt);
         }
 
         // cell record: own slot, the rows below and above (2D) and in front
@@ -172,7 +174,7 @@ namespace smr::dev
         };
 
         template <int DIM>
-        __device__ __forceinline__ void cell_upwind(const AdjointFlow& f, int64_t c, bool active, const double* u, double* out)
+        __device__ __forceinline__ uint64_t cell_upwind(const AdjointFlow& f, int64_t c, bool active, const double* u, double* out, const FlowWait& w)
         {
             CellRec<DIM> r{};
             FlowParam p{};
@@ -183,38 +185,90 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + (k == 0 ? r.own : r.neighbour(k - 1)); };
             Sources<2 * DIM + 1, decltype(at)> s;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           if (!s.ready(at) && !last)
-                           {
-                               return false;
-                           }
-                           const double uc = s.v[0];
-                           const double FL = flux_h(.5 * p.a[0], .5 * fabs(p.a[0]), s.v[1], uc);
-                           const double FR = flux_h(.5 * p.a[0], .5 * fabs(p.a[0]), uc, s.v[2]);
-                           const double FD = flux_h(.5 * p.a[1], .5 * fabs(p.a[1]), s.v[3], uc);
-                           const double FU = flux_h(.5 * p.a[1], .5 * fabs(p.a[1]), uc, s.v[4]);
-                           double S;
-                           if constexpr (DIM == 2)
-                           {
-                               S = -FL + FR + -FD + FU;
-                           }
-                           else
-                           {
-                               const double FF = flux_h(.5 * p.a[2], .5 * fabs(p.a[2]), s.v[2 * DIM - 1], uc);
-                               const double FB = flux_h(.5 * p.a[2], .5 * fabs(p.a[2]), uc, s.v[2 * DIM]);
-                               S               = -FL + FR + -FD + FU + -FF + FB;
-                           }
-                           publish(out + r.own, uc - p.dt * (S * double(1 << r.level())));
-                           return true;
-                       });
+            auto attempt = [&](bool last) -> int
+            {
+                const bool ok = s.ready(at);
+                if (!ok && !last)
+                {
+                    return WAITS;
+                }
+                const double uc = s.v[0];
+                const double FL = flux_h(.5 * p.a[0], .5 * fabs(p.a[0]), s.v[1], uc);
+                const double FR = flux_h(.5 * p.a[0], .5 * fabs(p.a[0]), uc, s.v[2]);
+                const double FD = flux_h(.5 * p.a[1], .5 * fabs(p.a[1]), s.v[3], uc);
+                const double FU = flux_h(.5 * p.a[1], .5 * fabs(p.a[1]), uc, s.v[4]);
+                double S;
+                if constexpr (DIM == 2)
+                {
+                    S = -FL + FR + -FD + FU;
+                }
+                else
+                {
+                    const double FF = flux_h(.5 * p.a[2], .5 * fabs(p.a[2]), s.v[2 * DIM - 1], uc);
+                    const double FB = flux_h(.5 * p.a[2], .5 * fabs(p.a[2]), uc, s.v[2 * DIM]);
+                    S               = -FL + FR + -FD + FU + -FF + FB;
+                }
+                publish(out + r.own, uc - p.dt * (S * double(1 << r.level())));
+                return ok ? DONE : MISSED;
+            };
+            return until_done(active, w, attempt);
+        }
+
+        // a lane that missed a source of operation c of item k (a step's, on the
+        // array u, whose cells are the launch's input when input): a fault unless
+        // the launch only reads what it waited for
+        __device__ __forceinline__ void report_missed(const AdjointFlow& f, const LookBack& b, bool input, const FlowWait& w)
+        {
+            if (b.slot < 0 || f.kind[b.slot] == 2 || (f.kind[b.slot] == 1 && !input))
+            {
+                report_fault(w, FAULT_ADJOINT);
+            }
+            else
+            {
+                excuse_faults(w);
+            }
+        }
+
+        template <int DIM, int S>
+        __device__ __forceinline__ void step_missed(const AdjointFlow& f, int k, int64_t c, const double* u, bool input, const FlowWait& w)
+        {
+            LookBack b;
+            keep_apart(c);
+            if (f.op[k] == FLOW_RECIPES)
+            {
+                recipe_sources(f.rec, f.rsrc, c, u, b);
+            }
+            else if (f.op[k] == FLOW_UPWIND)
+            {
+                CellRec<DIM> r;
+                r.load(f.cell, c);
+                b.source(u, r.own);
+#pragma unroll
+                for (int d = 0; d < 2 * DIM; ++d)
+                {
+                    b.source(u, r.neighbour(d));
+                }
+            }
+            else
+            {
+                const bool fine  = f.op[k] == FLOW_PROJECT;
+                const int32_t* t = fine ? f.proj + proj_words(DIM) * c : f.pred + pred_words(DIM, S) * c;
+                const int rows   = fine ? 1 << (DIM - 1) : (DIM == 3 ? (2 * S + 1) * (2 * S + 1) : 2 * S + 1);
+                for (int q = 1; q <= rows; ++q)
+                {
+                    for (int x = 0; x < (fine ? 2 : 2 * S + 1); ++x)
+                    {
+                        b.source(u, t[q] + x);
+                    }
+                }
+            }
+            report_missed(f, b, input, w);
         }
 
         // a.steps time steps: the ghosts of each state, then the next state's
         // cells (not the last one's without `last`)
         template <int DIM, int S>
-        __global__ __launch_bounds__(FB) void k_adj_forward(AdjointFlow f, FlowArrays a, int last, unsigned* ticket)
+        __global__ __launch_bounds__(FB) void k_adj_forward(AdjointFlow f, FlowArrays a, int last, unsigned* ticket, FlowWait fw)
         {
             const int64_t g = take_wave(ticket);
             const int j     = int(g / f.nwaves);
@@ -230,6 +284,7 @@ namespace smr::dev
             const int64_t c  = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + lane;
             const bool act   = c < f.c1[k];
             double* u        = segment_array(a, j, f.n);
+            uint64_t missed  = 0;
             switch (f.op[k])
             {
                 case FLOW_RECIPES:
@@ -240,17 +295,21 @@ namespace smr::dev
                         const int4 r = reinterpret_cast<const int4*>(f.rec)[c];
                         bc           = (r.y & 255) == 1 ? f.par[r.w].bc : 0.0;
                     }
-                    flow_recipe(f.rec, f.rsrc, c, act, u, bc);
+                    missed = flow_recipe(f.rec, f.rsrc, c, act, u, bc, fw);
                     break;
                 }
-                case FLOW_PROJECT: ghost_project<DIM, S>(f.proj, c, act, u); break;
-                case FLOW_PREDICT: ghost_predict<DIM, S>(f.pred, c, act, u); break;
+                case FLOW_PROJECT: missed = ghost_project<DIM, S>(f.proj, c, act, u, fw); break;
+                case FLOW_PREDICT: missed = ghost_predict<DIM, S>(f.pred, c, act, u, fw); break;
                 default:
                     if (j + 1 < a.steps || last)
                     {
-                        cell_upwind<DIM>(f, c, act, u, segment_array(a, j + 1, f.n));
+                        missed = cell_upwind<DIM>(f, c, act, u, segment_array(a, j + 1, f.n), fw);
                     }
                     break;
+            }
+            if ((missed >> lane) & 1)
+            {
+                step_missed<DIM, S>(f, k, c, u, j == 0, fw);
             }
         }
 
@@ -260,6 +319,7 @@ namespace smr::dev
         {
             int32_t k, end;
             double group = 0;
+            bool missed  = false;
             __device__ __forceinline__ bool run(const AdjointFlow& f, const double* mu, double& m, bool last)
             {
                 for (; k < end; ++k)
@@ -270,9 +330,13 @@ namespace smr::dev
                     if (marked(x))
                     {
                         x = look_again(p);
-                        if (marked(x) && !last)
+                        if (marked(x))
                         {
-                            return false;
+                            if (!last)
+                            {
+                                return false;
+                            }
+                            missed = true;
                         }
                     }
                     group += f.ew[k] * x;
@@ -286,10 +350,19 @@ namespace smr::dev
             }
         };
 
+        // the sources of operation q of an adjoint step
+        __device__ __forceinline__ void gathered_sources(const AdjointFlow& f, int64_t q, const double* lam, LookBack& b)
+        {
+            for (int32_t e = f.rowptr[q]; e < f.rowptr[q + 1]; ++e)
+            {
+                b.source(lam, f.esrc[e] & kFlowSlotMask);
+            }
+        }
+
         // a.steps adjoint steps: per step the ghosts' adjoint values, then the
         // cells' of the step before
         template <int DIM>
-        __global__ __launch_bounds__(FB) void k_adj_backward(AdjointFlow f, FlowArrays a, unsigned* ticket)
+        __global__ __launch_bounds__(FB) void k_adj_backward(AdjointFlow f, FlowArrays a, unsigned* ticket, FlowWait fw)
         {
             const int64_t g   = take_wave(ticket);
             const int64_t nwg = (f.naghost + 63) / 64, nw = nwg + (f.ncells + 63) / 64;
@@ -326,38 +399,58 @@ namespace smr::dev
                     in.end   = f.rowptr[q + 1];
                 }
                 int d = 0;
-                until_done(act,
-                           [&](bool last)
-                           {
+                auto attempt = [&](bool last) -> int
+                {
 #pragma unroll
-                               for (int e = 0; e < 2 * DIM; ++e)
-                               {
-                                   if (e == d)
-                                   {
-                                       if (cells[e] >= 0)
-                                       {
-                                           double x = look(lam + cells[e]);
-                                           if (marked(x))
-                                           {
-                                               x = look_again(lam + cells[e]);
-                                               if (marked(x) && !last)
-                                               {
-                                                   return false;
-                                               }
-                                           }
-                                           const double aa = p.a[e >> 1];
-                                           m += (e & 1) ? -kk * fmin(aa, 0.0) * x : kk * fmax(aa, 0.0) * x;
-                                       }
-                                       ++d;
-                                   }
-                               }
-                               if (!in.run(f, lam, m, last))
-                               {
-                                   return false;
-                               }
-                               publish(lam + dst, m);
-                               return true;
-                           });
+                    for (int e = 0; e < 2 * DIM; ++e)
+                    {
+                        if (e == d)
+                        {
+                            if (cells[e] >= 0)
+                            {
+                                double x = look(lam + cells[e]);
+                                if (marked(x))
+                                {
+                                    x = look_again(lam + cells[e]);
+                                    if (marked(x))
+                                    {
+                                        if (!last)
+                                        {
+                                            return WAITS;
+                                        }
+                                        in.missed = true;
+                                    }
+                                }
+                                const double aa = p.a[e >> 1];
+                                m += (e & 1) ? -kk * fmin(aa, 0.0) * x : kk * fmax(aa, 0.0) * x;
+                            }
+                            ++d;
+                        }
+                    }
+                    if (!in.run(f, lam, m, last))
+                    {
+                        return WAITS;
+                    }
+                    publish(lam + dst, m);
+                    return in.missed ? MISSED : DONE;
+                };
+                const uint64_t missed = until_done(act, fw, attempt);
+                if ((missed >> lane) & 1)
+                {
+                    LookBack b;
+                    int64_t g2 = q;
+                    keep_apart(g2);
+                    for (int e = 0; e < 2 * DIM; ++e)
+                    {
+                        const int32_t beside = f.aghost[8 * g2 + 2 + e];
+                        if (beside >= 0)
+                        {
+                            b.source(lam, beside);
+                        }
+                    }
+                    gathered_sources(f, g2, lam, b);
+                    report_missed(f, b, j == 0, fw);
+                }
                 return;
             }
             const int64_t c = (w - nwg) * 64 + lane;
@@ -379,42 +472,61 @@ namespace smr::dev
             Sources<2 * DIM + 1, decltype(at)> s;
             bool begun = false;
             double m   = 0;
-            until_done(act,
-                       [&](bool last)
-                       {
-                           if (!begun)
-                           {
-                               if (!s.ready(at) && !last)
-                               {
-                                   return false;
-                               }
-                               const double k = p.dt * ldexp(1.0, r.level());
-                               double v[2 * DIM];
+            auto attempt = [&](bool last) -> int
+            {
+                if (!begun)
+                {
+                    if (!s.ready(at))
+                    {
+                        if (!last)
+                        {
+                            return WAITS;
+                        }
+                        in.missed = true;
+                    }
+                    const double k = p.dt * ldexp(1.0, r.level());
+                    double v[2 * DIM];
 #pragma unroll
-                               for (int d = 0; d < 2 * DIM; ++d)
-                               {
-                                   v[d] = r.ghost(d) ? 0.0 : s.v[1 + d];
-                               }
-                               double self = fabs(p.a[0]) + fabs(p.a[1]);
-                               if constexpr (DIM == 3)
-                               {
-                                   self += fabs(p.a[2]);
-                               }
-                               m = (1.0 - k * self) * s.v[0];
+                    for (int d = 0; d < 2 * DIM; ++d)
+                    {
+                        v[d] = r.ghost(d) ? 0.0 : s.v[1 + d];
+                    }
+                    double self = fabs(p.a[0]) + fabs(p.a[1]);
+                    if constexpr (DIM == 3)
+                    {
+                        self += fabs(p.a[2]);
+                    }
+                    m = (1.0 - k * self) * s.v[0];
 #pragma unroll
-                               for (int d = 0; d < DIM; ++d)
-                               {
-                                   m += k * fmax(p.a[d], 0.0) * v[2 * d + 1] - k * fmin(p.a[d], 0.0) * v[2 * d];
-                               }
-                               begun = true;
-                           }
-                           if (!in.run(f, lam, m, last))
-                           {
-                               return false;
-                           }
-                           publish(out + r.own, m);
-                           return true;
-                       });
+                    for (int d = 0; d < DIM; ++d)
+                    {
+                        m += k * fmax(p.a[d], 0.0) * v[2 * d + 1] - k * fmin(p.a[d], 0.0) * v[2 * d];
+                    }
+                    begun = true;
+                }
+                if (!in.run(f, lam, m, last))
+                {
+                    return WAITS;
+                }
+                publish(out + r.own, m);
+                return in.missed ? MISSED : DONE;
+            };
+            const uint64_t missed = until_done(act, fw, attempt);
+            if ((missed >> lane) & 1)
+            {
+                LookBack b;
+                int64_t c2 = c;
+                keep_apart(c2);
+                CellRec<DIM> r2;
+                r2.load(f.cell, c2);
+                b.source(lam, r2.own);
+                for (int d = 0; d < 2 * DIM; ++d)
+                {
+                    b.source(lam, r2.ghost(d) ? r2.own : r2.neighbour(d));
+                }
+                gathered_sources(f, f.naghost + c2, lam, b);
+                report_missed(f, b, j == 0, fw);
+            }
         }
 
         // the velocity-gradient terms of a.steps adjoint steps (all values in
@@ -516,7 +628,7 @@ namespace smr::dev
         }
     }
 
-    void adjoint_flow_forward(const AdjointFlow& f, const FlowArrays& a, bool last, unsigned* ticket, hipStream_t s)
+    void adjoint_flow_forward(const AdjointFlow& f, const FlowArrays& a, bool last, unsigned* ticket, const FlowWait& w, hipStream_t s)
     {
         if (f.ncells <= 0)
         {
@@ -526,23 +638,23 @@ namespace smr::dev
         const dim3 g(blocks_of(int64_t(f.nwaves) * a.steps, FB / 64)), b(FB);
         if (f.dim == 2 && f.ps == 0)
         {
-            hipLaunchKernelGGL((k_adj_forward<2, 0>), g, b, 0, s, f, a, int(last), ticket);
+            hipLaunchKernelGGL((k_adj_forward<2, 0>), g, b, 0, s, f, a, int(last), ticket, w);
         }
         else if (f.dim == 2)
         {
-            hipLaunchKernelGGL((k_adj_forward<2, 1>), g, b, 0, s, f, a, int(last), ticket);
+            hipLaunchKernelGGL((k_adj_forward<2, 1>), g, b, 0, s, f, a, int(last), ticket, w);
         }
         else if (f.ps == 0)
         {
-            hipLaunchKernelGGL((k_adj_forward<3, 0>), g, b, 0, s, f, a, int(last), ticket);
+            hipLaunchKernelGGL((k_adj_forward<3, 0>), g, b, 0, s, f, a, int(last), ticket, w);
         }
         else
         {
-            hipLaunchKernelGGL((k_adj_forward<3, 1>), g, b, 0, s, f, a, int(last), ticket);
+            hipLaunchKernelGGL((k_adj_forward<3, 1>), g, b, 0, s, f, a, int(last), ticket, w);
         }
     }
 
-    void adjoint_flow_backward(const AdjointFlow& f, const FlowArrays& a, unsigned* ticket, hipStream_t s)
+    void adjoint_flow_backward(const AdjointFlow& f, const FlowArrays& a, unsigned* ticket, const FlowWait& w, hipStream_t s)
     {
         if (f.ncells <= 0)
         {
@@ -553,11 +665,11 @@ namespace smr::dev
         const dim3 g(blocks_of(nw * a.steps, FB / 64)), b(FB);
         if (f.dim == 2)
         {
-            hipLaunchKernelGGL(k_adj_backward<2>, g, b, 0, s, f, a, ticket);
+            hipLaunchKernelGGL(k_adj_backward<2>, g, b, 0, s, f, a, ticket, w);
         }
         else
         {
-            hipLaunchKernelGGL(k_adj_backward<3>, g, b, 0, s, f, a, ticket);
+            hipLaunchKernelGGL(k_adj_backward<3>, g, b, 0, s, f, a, ticket, w);
         }
     }
 

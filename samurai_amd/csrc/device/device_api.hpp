@@ -344,6 +344,23 @@ namespace smr::dev
     void sequence(int dim, int ps, const SeqItem* items, int i0, int i1, const List& l_proj, const List& l_pred, const List& l_max, double* u,
                   uint8_t* tag, bool has_bc, double bc_value, hipStream_t s);
 
+    // The waits of a dataflow launch (flow_ops.hpp): the rounds after which a
+    // wave gives up, and the context's fault words (pinned host memory).  A wave
+    // that gave up on a value of the launch itself sets the first to one of
+    // Fault, one that gave up on a value it only reads sets the second.
+    // Ctx::sync reads and clears them, and throws for the first without the second.
+    struct FlowWait
+    {
+        int rounds;
+        int* fault;
+    };
+    enum Fault : int
+    {
+        FAULT_GHOSTS  = 1, // update_ghost_mr
+        FAULT_ADJOINT = 2, // frozen steps or their adjoint
+        FAULT_TAGS    = 3  // the maximum pass of the tags
+    };
+
     // update_ghost_mr as one dataflow launch (ghost_flow.hip): the ghosts in an
     // order that keeps every source before its readers, cut into items of one
     // kind and level.  Item k is the indices [c0[k], c1[k]) of the projection
@@ -361,7 +378,7 @@ namespace smr::dev
         int32_t wave0[kFlowItems], c0[kFlowItems], c1[kFlowItems];
         int32_t op[kFlowItems]; // SeqOp
     };
-    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s);
+    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, const FlowWait& w, hipStream_t s);
     // the same of many fields in one launch: instance k takes the waves
     // [wpref[k], wpref[k + 1]) of wpref[n] = nwaves (device arrays; ticket: one
     // scratch word)
@@ -371,7 +388,8 @@ namespace smr::dev
         double* u;
         double bc;
     };
-    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, hipStream_t s);
+    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, const FlowWait& w,
+                          hipStream_t s);
 
     // Frozen-mesh steps of many instances and their adjoint as dataflow
     // launches (adjoint_flow.hip).  Slots number the storages of all instances
@@ -424,9 +442,9 @@ namespace smr::dev
     void adjoint_flow_cells(const AdjointFlow& f, double* array, double* compact, bool to_compact, hipStream_t s);
     // a.steps time steps from the cells of the first array; with `last` the
     // cells of the last array are computed too
-    void adjoint_flow_forward(const AdjointFlow& f, const FlowArrays& a, bool last, unsigned* ticket, hipStream_t s);
+    void adjoint_flow_forward(const AdjointFlow& f, const FlowArrays& a, bool last, unsigned* ticket, const FlowWait& w, hipStream_t s);
     // a.steps adjoint steps from the cells of the first array to the last's
-    void adjoint_flow_backward(const AdjointFlow& f, const FlowArrays& a, unsigned* ticket, hipStream_t s);
+    void adjoint_flow_backward(const AdjointFlow& f, const FlowArrays& a, unsigned* ticket, const FlowWait& w, hipStream_t s);
     // adds the velocity-gradient terms of the adjoint steps of lam to ga (dim
     // per cell): step j with state st0 - j of st
     void adjoint_flow_velocity(const AdjointFlow& f, const FlowArrays& lam, const FlowArrays& st, int st0, double* ga, hipStream_t s);
@@ -596,7 +614,7 @@ namespace smr::dev
     void maximum(int dim, const List& l, int64_t c0, int64_t c1, uint8_t* tag, hipStream_t s);
     // maximum over the whole list, whose levels ascend, from the finest down
     // (ticket: one scratch word)
-    void tag_flow(int dim, const List& l, uint8_t* tag, unsigned* ticket, hipStream_t s);
+    void tag_flow(int dim, const List& l, uint8_t* tag, unsigned* ticket, const FlowWait& w, hipStream_t s);
     void tag_init(const List& l, int64_t c0, int64_t c1, uint8_t* tag, hipStream_t s);
     // p[0, n) = 0 by a kernel (graph-capturable, unlike hipMemsetAsync)
     void zero_f64(double* p, int64_t n, hipStream_t s);

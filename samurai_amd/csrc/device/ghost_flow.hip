@@ -24,8 +24,9 @@
 // counter (the ticket), and the order keeps every source before its readers
 // where the cells tile the box (the other meshes keep the staged launches), so
 // the lowest unfinished wave waits for nothing that is not done; and a wave
-// gives up after kMaxSpins rounds and uses what it has read (which is the
-// right value when a cell itself holds the bits of the mark).
+// gives up after FlowWait::rounds looks and uses what it has read (the right
+// value when a cell itself holds the bits of the mark; when the source is a
+// ghost of the update, the fault word says so).
 #include "flow_ops.hpp"
 
 namespace smr::dev
@@ -34,7 +35,7 @@ namespace smr::dev
     {
         // projection_op_ (op_project_at) on waited-for sources
         template <int DIM>
-        __device__ __forceinline__ void flow_project(const List& l, int64_t c, bool active, double* u)
+        __device__ __forceinline__ uint64_t flow_project(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NR     = 1 << (DIM - 1);
             constexpr double inv = 1.0 / double(1 << DIM);
@@ -53,27 +54,28 @@ namespace smr::dev
             }
             auto at = [&](int k) { return row[k >> 1] + (k & 1); };
             Sources<2 * NR, decltype(at)> s;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           if (!s.ready(at) && !last)
-                           {
-                               return false;
-                           }
-                           double sum = 0;
+            auto attempt = [&](bool last) -> int
+            {
+                const bool ok = s.ready(at);
+                if (!ok && !last)
+                {
+                    return WAITS;
+                }
+                double sum = 0;
 #pragma unroll
-                           for (int r = 0; r < NR; ++r)
-                           {
-                               sum += s.v[2 * r] + s.v[2 * r + 1];
-                           }
-                           publish(dst, sum * inv);
-                           return true;
-                       });
+                for (int r = 0; r < NR; ++r)
+                {
+                    sum += s.v[2 * r] + s.v[2 * r + 1];
+                }
+                publish(dst, sum * inv);
+                return ok ? DONE : MISSED;
+            };
+            return until_done(active, w, attempt);
         }
 
         // prediction_op <s,false> (op_predict_fine_at) on waited-for sources
         template <int DIM, int S>
-        __device__ __forceinline__ void flow_predict(const List& l, int64_t c, bool active, double* u)
+        __device__ __forceinline__ uint64_t flow_predict(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NY = 2 * S + 1, NZ = DIM == 3 ? NY : 1, N = NZ * NY * NY;
             double* dst = nullptr;
@@ -95,46 +97,47 @@ namespace smr::dev
             }
             auto at = [&](int k) { return row[k / NY] + k % NY; };
             Sources<N, decltype(at)> s;
-            until_done(active,
-                       [&](bool last)
-                       {
-                           if (!s.ready(at) && !last)
-                           {
-                               return false;
-                           }
-                           double v;
-                           if constexpr (S == 0)
-                           {
-                               v = s.v[0];
-                           }
-                           else
-                           {
-                               v = 0;
+            auto attempt = [&](bool last) -> int
+            {
+                const bool ok = s.ready(at);
+                if (!ok && !last)
+                {
+                    return WAITS;
+                }
+                double v;
+                if constexpr (S == 0)
+                {
+                    v = s.v[0];
+                }
+                else
+                {
+                    v = 0;
 #pragma unroll
-                               for (int rz = 0; rz < NZ; ++rz)
-                               {
+                    for (int rz = 0; rz < NZ; ++rz)
+                    {
 #pragma unroll
-                                   for (int ry = 0; ry < 3; ++ry)
-                                   {
+                        for (int ry = 0; ry < 3; ++ry)
+                        {
 #pragma unroll
-                                       for (int sx = 0; sx < 3; ++sx)
-                                       {
-                                           const double f = s.v[(rz * 3 + ry) * 3 + sx];
-                                           double coeff   = 1.;
-                                           coeff *= pcoef(px, sx);
-                                           coeff *= pcoef(py, ry);
-                                           if constexpr (DIM == 3)
-                                           {
-                                               coeff *= pcoef(pz, rz);
-                                           }
-                                           v += f * coeff;
-                                       }
-                                   }
-                               }
-                           }
-                           publish(dst, v);
-                           return true;
-                       });
+                            for (int sx = 0; sx < 3; ++sx)
+                            {
+                                const double f = s.v[(rz * 3 + ry) * 3 + sx];
+                                double coeff   = 1.;
+                                coeff *= pcoef(px, sx);
+                                coeff *= pcoef(py, ry);
+                                if constexpr (DIM == 3)
+                                {
+                                    coeff *= pcoef(pz, rz);
+                                }
+                                v += f * coeff;
+                            }
+                        }
+                    }
+                }
+                publish(dst, v);
+                return ok ? DONE : MISSED;
+            };
+            return until_done(active, w, attempt);
         }
 
         // the item of wave w: the last one whose first wave is at most w
@@ -170,18 +173,81 @@ namespace smr::dev
             u[dst] = __longlong_as_double((long long)kMark);
         }
 
+        __device__ __forceinline__ bool in_list(const List& l, int64_t slot)
+        {
+            for (int64_t r = 0; r < l.nruns; ++r)
+            {
+                const int64_t x = slot - l.base[r * l.ntaps];
+                if (x >= l.iv[5 * r] && x < l.iv[5 * r + 1])
+                {
+                    return true;
+                }
+            }
+            return false;
+        }
+
+        // a lane that missed a source of ghost c of item k: a fault unless the
+        // update does not write what it waited for
+        template <int DIM, int S>
+        __device__ __forceinline__ void flow_missed(const GhostFlow& f, int k, int64_t c, const double* u, const FlowWait& w)
+        {
+            LookBack b;
+            keep_apart(c);
+            if (f.op[k] == SEQ_RECIPES)
+            {
+                recipe_sources(f.rec, f.rsrc, c, u, b);
+            }
+            else
+            {
+                const bool fine    = f.op[k] == SEQ_PROJECT;
+                const List& l      = fine ? f.proj : f.pred;
+                const Cell cell    = locate(l, c);
+                const int64_t* row = bases(l, cell.run);
+                const int n        = fine ? 2 : 2 * S + 1;
+                const int32_t x0   = fine ? 2 * cell.x : (cell.x >> 1) - S;
+                for (int r = 1; r < l.ntaps; ++r)
+                {
+                    for (int x = 0; x < n; ++x)
+                    {
+                        b.source(u, row[r] + x0 + x);
+                    }
+                }
+            }
+            bool own = b.slot < 0 || in_list(f.proj, b.slot) || in_list(f.pred, b.slot);
+            for (int q = 0; q < f.nitems; ++q)
+            {
+                for (int32_t e = f.op[q] == SEQ_RECIPES ? f.c0[q] : f.c1[q]; e < f.c1[q]; ++e)
+                {
+                    own = own || f.rec[4 * int64_t(e)] == b.slot;
+                }
+            }
+            if (own)
+            {
+                report_fault(w, FAULT_GHOSTS);
+            }
+            else
+            {
+                excuse_faults(w);
+            }
+        }
+
         // computes the ghosts of wave w
         template <int DIM, int S>
-        __device__ __forceinline__ void flow_wave(const GhostFlow& f, int w, double* u, double bc)
+        __device__ __forceinline__ void flow_wave(const GhostFlow& f, int w, double* u, double bc, const FlowWait& fw)
         {
             const int k       = item_of(f, w);
             const int64_t c   = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
             const bool active = c < f.c1[k];
+            uint64_t missed;
             switch (f.op[k])
             {
-                case SEQ_RECIPES: flow_recipe(f.rec, f.rsrc, c, active, u, bc); break;
-                case SEQ_PROJECT: flow_project<DIM>(f.proj, c, active, u); break;
-                default: flow_predict<DIM, S>(f.pred, c, active, u); break;
+                case SEQ_RECIPES: missed = flow_recipe(f.rec, f.rsrc, c, active, u, bc, fw); break;
+                case SEQ_PROJECT: missed = flow_project<DIM>(f.proj, c, active, u, fw); break;
+                default: missed = flow_predict<DIM, S>(f.pred, c, active, u, fw); break;
+            }
+            if ((missed >> (threadIdx.x & 63)) & 1)
+            {
+                flow_missed<DIM, S>(f, k, c, u, fw);
             }
         }
 
@@ -203,7 +269,7 @@ namespace smr::dev
         constexpr int FLOW_BLOCK = 512;
 
         template <int DIM, int S>
-        __global__ __launch_bounds__(FLOW_BLOCK) void k_ghost_flow(GhostFlow f, double* u, int64_t nref, double bc)
+        __global__ __launch_bounds__(FLOW_BLOCK) void k_ghost_flow(GhostFlow f, double* u, int64_t nref, double bc, FlowWait fw)
         {
             __shared__ unsigned ticket;
             if (threadIdx.x == 0)
@@ -214,7 +280,7 @@ namespace smr::dev
             const int w = __builtin_amdgcn_readfirstlane(int(ticket * (blockDim.x >> 6) + (threadIdx.x >> 6)));
             if (w < f.nwaves)
             {
-                flow_wave<DIM, S>(f, w, u, bc);
+                flow_wave<DIM, S>(f, w, u, bc, fw);
             }
         }
 
@@ -258,7 +324,7 @@ namespace smr::dev
 
         template <int DIM, int S>
         __global__ __launch_bounds__(BATCH_BLOCK) void k_ghost_flow_batch(const FlowInstance* inst, const int64_t* pref, int n, int64_t nwaves,
-                                                                          unsigned* ticket)
+                                                                          unsigned* ticket, FlowWait fw)
         {
             __shared__ unsigned t;
             if (threadIdx.x == 0)
@@ -270,12 +336,12 @@ namespace smr::dev
             if (w < nwaves)
             {
                 const int k = instance_of(pref, n, w);
-                flow_wave<DIM, S>(inst[k].f, int(w - pref[k]), inst[k].u, inst[k].bc);
+                flow_wave<DIM, S>(inst[k].f, int(w - pref[k]), inst[k].u, inst[k].bc, fw);
             }
         }
     } // namespace
 
-    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, hipStream_t s)
+    void ghost_flow(int dim, int ps, const GhostFlow& f, double* u, int64_t nref, double bc, const FlowWait& w, hipStream_t s)
     {
         if (f.nwaves <= 0)
         {
@@ -290,23 +356,24 @@ namespace smr::dev
         hipLaunchKernelGGL(k_ghost_reset, dim3(unsigned((f.nwaves + 3) / 4)), dim3(256), 0, s, f, u, nref);
         if (dim == 2 && ps == 0)
         {
-            hipLaunchKernelGGL((k_ghost_flow<2, 0>), g, b, 0, s, f, u, nref, bc);
+            hipLaunchKernelGGL((k_ghost_flow<2, 0>), g, b, 0, s, f, u, nref, bc, w);
         }
         else if (dim == 2)
         {
-            hipLaunchKernelGGL((k_ghost_flow<2, 1>), g, b, 0, s, f, u, nref, bc);
+            hipLaunchKernelGGL((k_ghost_flow<2, 1>), g, b, 0, s, f, u, nref, bc, w);
         }
         else if (ps == 0)
         {
-            hipLaunchKernelGGL((k_ghost_flow<3, 0>), g, b, 0, s, f, u, nref, bc);
+            hipLaunchKernelGGL((k_ghost_flow<3, 0>), g, b, 0, s, f, u, nref, bc, w);
         }
         else
         {
-            hipLaunchKernelGGL((k_ghost_flow<3, 1>), g, b, 0, s, f, u, nref, bc);
+            hipLaunchKernelGGL((k_ghost_flow<3, 1>), g, b, 0, s, f, u, nref, bc, w);
         }
     }
 
-    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, hipStream_t s)
+    void ghost_flow_batch(int dim, int ps, const FlowInstance* inst, const int64_t* wpref, int n, int64_t nwaves, unsigned* ticket, const FlowWait& w,
+                          hipStream_t s)
     {
         if (nwaves <= 0)
         {
@@ -317,19 +384,19 @@ namespace smr::dev
         hipLaunchKernelGGL(k_ghost_reset_batch, dim3(unsigned((nwaves + 3) / 4)), dim3(256), 0, s, inst, wpref, n, nwaves, ticket);
         if (dim == 2 && ps == 0)
         {
-            hipLaunchKernelGGL((k_ghost_flow_batch<2, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+            hipLaunchKernelGGL((k_ghost_flow_batch<2, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket, w);
         }
         else if (dim == 2)
         {
-            hipLaunchKernelGGL((k_ghost_flow_batch<2, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+            hipLaunchKernelGGL((k_ghost_flow_batch<2, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket, w);
         }
         else if (ps == 0)
         {
-            hipLaunchKernelGGL((k_ghost_flow_batch<3, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+            hipLaunchKernelGGL((k_ghost_flow_batch<3, 0>), g, b, 0, s, inst, wpref, n, nwaves, ticket, w);
         }
         else
         {
-            hipLaunchKernelGGL((k_ghost_flow_batch<3, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket);
+            hipLaunchKernelGGL((k_ghost_flow_batch<3, 1>), g, b, 0, s, inst, wpref, n, nwaves, ticket, w);
         }
     }
 } // namespace smr::dev

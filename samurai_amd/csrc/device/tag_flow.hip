@@ -5,7 +5,8 @@
 // k_tag_open opens every coarse cell of the list (a bit of its tag byte that
 // no rule uses), k_tag_flow closes them, finest level first: blocks take their
 // place from a counter, so the lowest unfinished wave waits for nothing that is
-// not done, and a wave gives up waiting after kMaxSpins rounds.  The tags
+// not done, and a wave gives up waiting after FlowWait::rounds looks (which
+// only a broken order would make it do: the fault word says so).  The tags
 // travel through agent-scope byte loads and stores.
 //
 // Bound: latency, a store-to-load trip per level.  The staged form is a launch
@@ -38,7 +39,7 @@ namespace smr::dev
         }
 
         template <int DIM>
-        __global__ __launch_bounds__(TB) void k_tag_flow(List l, uint8_t* tag, unsigned* ticket)
+        __global__ __launch_bounds__(TB) void k_tag_flow(List l, uint8_t* tag, unsigned* ticket, FlowWait fw)
         {
             __shared__ unsigned place;
             if (threadIdx.x == 0)
@@ -65,40 +66,44 @@ namespace smr::dev
                     row[r] = tag + b[1 + r] + 2 * cell.x;
                 }
             }
-            until_done(active,
-                       [&](bool last)
-                       {
-                           unsigned t[2 * NR], any = 0, all = 2;
+            auto attempt = [&](bool last) -> int
+            {
+                unsigned t[2 * NR], any = 0, all = 2;
 #pragma unroll
-                           for (int k = 0; k < 2 * NR; ++k)
-                           {
-                               t[k] = __hip_atomic_load(row[k >> 1] + (k & 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                               any |= t[k];
-                               all &= t[k];
-                           }
-                           if ((any & kOpen) && !last)
-                           {
-                               return false;
-                           }
-                           // a child that is kept keeps the others, and the
-                           // cell; the children go together or not at all
-                           const bool keep = any & 1;
+                for (int k = 0; k < 2 * NR; ++k)
+                {
+                    t[k] = __hip_atomic_load(row[k >> 1] + (k & 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    any |= t[k];
+                    all &= t[k];
+                }
+                if ((any & kOpen) && !last)
+                {
+                    return WAITS;
+                }
+                // a child that is kept keeps the others, and the
+                // cell; the children go together or not at all
+                const bool keep = any & 1;
 #pragma unroll
-                           for (int k = 0; k < 2 * NR; ++k)
-                           {
-                               const unsigned w = keep ? t[k] | 1u : (all ? t[k] : t[k] & ~2u);
-                               if (w != t[k])
-                               {
-                                   __hip_atomic_store(row[k >> 1] + (k & 1), uint8_t(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                               }
-                           }
-                           __hip_atomic_store(own, uint8_t(keep || all ? v | 1u : v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                           return true;
-                       });
+                for (int k = 0; k < 2 * NR; ++k)
+                {
+                    const unsigned w = keep ? t[k] | 1u : (all ? t[k] : t[k] & ~2u);
+                    if (w != t[k])
+                    {
+                        __hip_atomic_store(row[k >> 1] + (k & 1), uint8_t(w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+                __hip_atomic_store(own, uint8_t(keep || all ? v | 1u : v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                return any & kOpen ? MISSED : DONE;
+            };
+            const uint64_t missed = until_done(active, fw, attempt);
+            if (missed != 0)
+            {
+                report_fault(fw, FAULT_TAGS);
+            }
         }
     } // namespace
 
-    void tag_flow(int dim, const List& l, uint8_t* tag, unsigned* ticket, hipStream_t s)
+    void tag_flow(int dim, const List& l, uint8_t* tag, unsigned* ticket, const FlowWait& w, hipStream_t s)
     {
         if (l.ncells <= 0)
         {
@@ -108,11 +113,11 @@ namespace smr::dev
         hipLaunchKernelGGL(k_tag_open, g, b, 0, s, l, tag, ticket);
         if (dim == 2)
         {
-            hipLaunchKernelGGL(k_tag_flow<2>, g, b, 0, s, l, tag, ticket);
+            hipLaunchKernelGGL(k_tag_flow<2>, g, b, 0, s, l, tag, ticket, w);
         }
         else
         {
-            hipLaunchKernelGGL(k_tag_flow<3>, g, b, 0, s, l, tag, ticket);
+            hipLaunchKernelGGL(k_tag_flow<3>, g, b, 0, s, l, tag, ticket, w);
         }
     }
 } // namespace smr::dev

@@ -364,6 +364,10 @@ namespace smr
         {
             (void)hipFree(d_err);
         }
+        if (fault)
+        {
+            (void)hipHostFree(fault);
+        }
         if (stream)
         {
             dev_cache_release(stream);
@@ -389,9 +393,32 @@ namespace smr
         }
     }
 
+    void Ctx::allocate_fault_words()
+    {
+        hip_check(hipHostMalloc(reinterpret_cast<void**>(&fault), 2 * sizeof(int), hipHostMallocMapped), "hipHostMalloc(fault words)");
+        fault[0] = fault[1] = 0;
+        void* p             = nullptr;
+        hip_check(hipHostGetDevicePointer(&p, fault, 0), "hipHostGetDevicePointer(fault words)");
+        wait.fault = static_cast<int*>(p);
+    }
+
     void Ctx::sync()
     {
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+        volatile int* f = fault;
+        if (!f || (f[0] == 0 && f[1] == 0))
+        {
+            return;
+        }
+        const int code = f[1] ? 0 : f[0];
+        f[0] = f[1] = 0;
+        switch (code)
+        {
+            case 0: return;
+            case dev::FAULT_GHOSTS: throw std::runtime_error("update_ghost_mr: a ghost went on without one of its sources");
+            case dev::FAULT_ADJOINT: throw std::runtime_error("adjoint: a value of a frozen step went on without one of its sources");
+            default: throw std::runtime_error("tag finalization: a cell went on without the tags of its children");
+        }
     }
 
     void Ctx::check_resolve()
@@ -1470,7 +1497,7 @@ namespace smr
         const dev::GhostFlow* flow = f.has_bc ? ghost_flow(*m.ctx, dm, m.host.cfg) : nullptr;
         if (takes_ghost_flow(*m.ctx, dm, flow))
         {
-            dev::ghost_flow(dim, ps, *flow, f.d, m.host.nref, bc, s);
+            dev::ghost_flow(dim, ps, *flow, f.d, m.host.nref, bc, m.ctx->wait, s);
             return;
         }
         const SeqPlan& plan = ghost_plan(*m.ctx, dm, m.host.cfg, f.has_bc);
@@ -2428,7 +2455,7 @@ namespace smr
             // behind the first field's values is free after its ghost update
             if (plan.steps.size() > 2)
             {
-                dev::tag_flow(dim, dm.maximum.d, tag, reinterpret_cast<unsigned*>(fs[0]->d + n), s);
+                dev::tag_flow(dim, dm.maximum.d, tag, reinterpret_cast<unsigned*>(fs[0]->d + n), ctx.wait, s);
                 return;
             }
             const auto* d_items = static_cast<const dev::SeqItem*>(plan.d_items.p);

@@ -363,6 +363,12 @@ namespace smr
         // update_ghost_mr: -1 the cheaper form, 0 the staged launches, 1 the
         // dataflow launch wherever there is one
         int ghost_form = -1;
+        // what a kernel reports that went on without a value it needed
+        // (dev::FlowWait): two words of pinned host memory, and the waits of the
+        // dataflow launches, which write them
+        int* fault = nullptr;
+        dev::FlowWait wait{1 << 17, nullptr};
+        void allocate_fault_words();
         void mark_runs_back();
         ~Ctx();
         int* d_flag() const { return d_err + 1; }
