@@ -15,9 +15,14 @@
 //   3. right, then left face to finer cells,
 //   4. right, then left boundary face.
 //
-// Bound: latency of about four dependent loads, as the upwind step.  The
+// Bound: latency of about four dependent loads, as the upwind step: the words of
+// the fine sides are loaded together, then the values of a direction.  The
 // ordered per-cell term lists this replaces cost 24 B per term to read and
-// were built on the host (14.5 ms for 141 K cells of a 2D L4..12 mesh).
+// were built on the host (14.5 ms for 141 K cells of a 2D L4..12 mesh).  Whole
+// calls on small meshes of prediction radius 0 (term lists / one fine face after
+// the other and the output cleared by a launch of its own / as below): 2D L2..6
+// 17.4 / 18.5 / 16.0 us, 3D L2..4 19.2 / 22.5 / 17.9 (Burgers) and 53.1 / 61.9 /
+// 51.2 (velocity field, four ghost updates).
 #include "cell_ops.hpp"
 
 namespace smr::dev
@@ -88,9 +93,14 @@ namespace smr::dev
             return k >= k0 && x + span <= t.run_e[k] ? t.run_idx[k] + x : -1;
         }
 
-        __global__ __launch_bounds__(CB) void k_leaf_flags(List l, uint8_t* leaf)
+        // leaf[slot] = 1 for the cells and past the nref slots (0 beforehand)
+        __global__ __launch_bounds__(CB) void k_leaf_flags(List l, uint8_t* leaf, int64_t nref)
         {
             const int64_t c = int64_t(blockIdx.x) * CB + threadIdx.x;
+            if (c < conv_leaf_bytes(nref) - nref)
+            {
+                leaf[nref + c] = 1;
+            }
             if (c < l.ncells)
             {
                 const Cell cell = locate(l, c);
@@ -240,11 +250,15 @@ namespace smr::dev
         }
 
         // the term of an interface between slots sl and sr along d with the
-        // signed factor f
+        // signed factor f (linear: the velocity in it)
         template <int OP>
-        __device__ __forceinline__ double interface_term(const ConvFields& a, int d, int64_t sl, int64_t sr, double f)
+        __device__ __forceinline__ double interface_term(const ConvFields& a, int d, int64_t sl, int64_t sr, double f, bool from_left)
         {
-            if constexpr (OP == CONV_BURGERS)
+            if constexpr (OP == CONV_LINEAR)
+            {
+                return f * a.u[from_left ? sl : sr];
+            }
+            else if constexpr (OP == CONV_BURGERS)
             {
                 return burgers_flux(a.u[sl], a.u[sr]) * f;
             }
@@ -253,55 +267,106 @@ namespace smr::dev
                 // w = 0.5 * (v_d[left] + v_d[right]) (convection_lin.hpp:210-226)
                 const double* v    = d == 0 ? a.v[0] : (d == 1 ? a.v[1] : a.v[2]);
                 const double w     = 0.5 * (v[sl] + v[sr]);
-                const double value = w >= 0 ? a.u[sl] : a.u[sr];
-                return (f * w) * value;
+                // both loaded, so that neither waits for w
+                const double ul = a.u[sl], ur = a.u[sr];
+                return (f * w) * (w >= 0 ? ul : ur);
             }
         }
 
+        // the terms of a side to finer cells (up: the right one), loaded at once:
+        // one per entry, in the order in which they are added
         template <int DIM, int OP>
-        __global__ __launch_bounds__(CB) void k_convection(List l, ConvSides sd, ConvFields a, double* __restrict__ out)
+        struct FineTerms
         {
-            constexpr int NF = 1 << (DIM - 1);
-            const int64_t c  = int64_t(blockIdx.x) * CB + threadIdx.x;
-            if (c >= l.ncells)
+            static constexpr int NF = 1 << (DIM - 1);
+            double t[NF];
+            bool ok[NF];
+            __device__ __forceinline__ void load(const ConvFields& a, int d, const int32_t (&e)[NF], bool up, double f, bool from_left)
             {
-                return;
+#pragma unroll
+                for (int k = 0; k < NF; ++k)
+                {
+                    // along x an entry is a face, else two are a pair of faces
+                    const int32_t first = d == 0 ? e[k] : e[k & ~1];
+                    ok[k]               = first >= 0;
+                    const int64_t in    = ok[k] ? (d == 0 ? first : first + (k & 1)) : 0;
+                    const int64_t o     = ok[k] ? (d == 0 ? first + (up ? 1 : -1) : e[k | 1] + (k & 1)) : 0;
+                    t[k]                = interface_term<OP>(a, d, up ? in : o, up ? o : in, f, from_left);
+                }
             }
+            __device__ __forceinline__ void add(double& acc, int d) const
+            {
+                if (OP == CONV_LINEAR && d != 0)
+                {
+#pragma unroll
+                    for (int k = 0; k < NF; k += 2)
+                    {
+                        acc = ok[k] ? acc + (t[k] + t[k + 1]) : acc;
+                    }
+                    return;
+                }
+#pragma unroll
+                for (int k = 0; k < NF; ++k)
+                {
+                    acc = ok[k] ? acc + t[k] : acc;
+                }
+            }
+        };
+
+        template <int DIM, int OP>
+        __device__ __forceinline__ void convect_cell(const List& l, const ConvSides& sd, const ConvFields& a, int64_t c, double* __restrict__ out)
+        {
+            constexpr int NF   = 1 << (DIM - 1);
             const int32_t word = sd.word[c];
+            const int32_t* fe  = sd.fine + sd.fine_at[c];
             const Cell cell    = locate(l, c);
             const int64_t* b   = bases(l, cell.run);
             const int64_t own  = b[0] + cell.x;
             const double fa    = double(int64_t(1) << cell.level);   // h^(dim-1) / h^dim
             const double ff    = fa / double(NF);                    // (h/2)^(dim-1) / h^dim: a face to a finer cell
-            const int32_t* fe  = nullptr;
-            double acc         = 0;
+            // the entries of all sides to finer cells, NF words each
+            int32_t entry[2 * DIM][NF];
+#pragma unroll
+            for (int s = 0; s < 2 * DIM; ++s)
+            {
+                if (side_of(word, s) == SIDE_FINE)
+                {
+                    __builtin_memcpy(entry[s], __builtin_assume_aligned(fe, 4 * NF), 4 * NF);
+                    fe += NF;
+                }
+            }
+            double acc = 0;
 #pragma unroll
             for (int d = 0; d < DIM; ++d)
             {
                 const int64_t left = d == 0 ? own - 1 : b[2 * d - 1] + cell.x, right = d == 0 ? own + 1 : b[2 * d] + cell.x;
                 const int kl = side_of(word, 2 * d), kr = side_of(word, 2 * d + 1);
-                const double v = OP == CONV_LINEAR ? a.vel[d] : 0.0;
+                const double v = OP == CONV_LINEAR ? a.vel[d] : 1.0;
                 if (OP == CONV_LINEAR && v == 0.0)
                 {
-                    // no terms; its entries are passed over
-                    if (kl == SIDE_FINE || kr == SIDE_FINE)
-                    {
-                        fe = fe ? fe : sd.fine + sd.fine_at[c];
-                        fe += NF * ((kl == SIDE_FINE) + (kr == SIDE_FINE));
-                    }
-                    continue;
+                    continue; // no terms
                 }
                 // linear: the upwind side carries the velocity; the left
                 // cell of an interface adds, the right one subtracts
                 const bool from_left = v >= 0;
+                const double fc = OP == CONV_LINEAR ? fa * v : fa;
                 double tl = 0, tr = 0; // the terms of the left and right face
                 if (kl != SIDE_FINE && kl != SIDE_NONE)
                 {
-                    tl = OP == CONV_LINEAR ? -(fa * v) * a.u[from_left ? left : own] : interface_term<OP>(a, d, left, own, -fa);
+                    tl = interface_term<OP>(a, d, left, own, -fc, from_left);
                 }
                 if (kr != SIDE_FINE && kr != SIDE_NONE)
                 {
-                    tr = OP == CONV_LINEAR ? (fa * v) * a.u[from_left ? own : right] : interface_term<OP>(a, d, own, right, fa);
+                    tr = interface_term<OP>(a, d, own, right, fc, from_left);
+                }
+                FineTerms<DIM, OP> fl, fr;
+                if (kr == SIDE_FINE)
+                {
+                    fr.load(a, d, entry[2 * d + 1], true, OP == CONV_LINEAR ? ff * v : ff, from_left);
+                }
+                if (kl == SIDE_FINE)
+                {
+                    fl.load(a, d, entry[2 * d], false, OP == CONV_LINEAR ? -ff * v : -ff, from_left);
                 }
                 if (OP == CONV_LINEAR && d == 0)
                 {
@@ -333,43 +398,13 @@ namespace smr::dev
                 {
                     acc += tr;
                 }
-                if (kl == SIDE_FINE || kr == SIDE_FINE)
+                if (kr == SIDE_FINE)
                 {
-                    fe = fe ? fe : sd.fine + sd.fine_at[c];
-                    const int32_t* of[2] = {fe, fe + (kl == SIDE_FINE ? NF : 0)};
-                    for (int up = 1; up >= 0; --up)
-                    {
-                        if ((up ? kr : kl) != SIDE_FINE)
-                        {
-                            continue;
-                        }
-                        const double f = up ? ff : -ff;
-                        for (int k = 0; k < NF; k += (d == 0 ? 1 : 2))
-                        {
-                            const int64_t in = of[up][k];
-                            if (in < 0)
-                            {
-                                continue;
-                            }
-                            const int64_t o = d == 0 ? in + (up ? 1 : -1) : of[up][k + 1];
-                            const int64_t sl = up ? in : o, sr = up ? o : in;
-                            if constexpr (OP == CONV_LINEAR)
-                            {
-                                const int64_t s = from_left ? sl : sr;
-                                const double g  = f * v;
-                                acc += d == 0 ? g * a.u[s] : g * a.u[s] + g * a.u[s + 1];
-                            }
-                            else
-                            {
-                                acc += interface_term<OP>(a, d, sl, sr, f);
-                                if (d != 0)
-                                {
-                                    acc += interface_term<OP>(a, d, sl + 1, sr + 1, f);
-                                }
-                            }
-                        }
-                    }
-                    fe += NF * ((kl == SIDE_FINE) + (kr == SIDE_FINE));
+                    fr.add(acc, d);
+                }
+                if (kl == SIDE_FINE)
+                {
+                    fl.add(acc, d);
                 }
                 if (kr == SIDE_BOUNDARY)
                 {
@@ -383,6 +418,37 @@ namespace smr::dev
             out[own] = acc;
         }
 
+        // the first blocks take the cells; the others, 8 slots a thread, zero the
+        // slots that are no cells (a clearing of the whole output ahead of the
+        // launch was another 2 us of a small mesh's 18)
+        template <int DIM, int OP>
+        __global__ __launch_bounds__(CB) void k_convection(List l, ConvSides sd, ConvFields a, double* __restrict__ out, unsigned cell_blocks)
+        {
+            if (blockIdx.x < cell_blocks)
+            {
+                const int64_t c = int64_t(blockIdx.x) * CB + threadIdx.x;
+                if (c < l.ncells)
+                {
+                    convect_cell<DIM, OP>(l, sd, a, c, out);
+                }
+                return;
+            }
+            const int64_t s0 = 8 * (int64_t(blockIdx.x - cell_blocks) * CB + threadIdx.x);
+            if (s0 >= sd.nref)
+            {
+                return;
+            }
+            const uint64_t cells = *reinterpret_cast<const uint64_t*>(sd.leaf + s0);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+            {
+                if (!((cells >> (8 * k)) & 1))
+                {
+                    out[s0 + k] = 0.0;
+                }
+            }
+        }
+
         unsigned blocks(int64_t n)
         {
             return unsigned((n + CB - 1) / CB);
@@ -391,12 +457,13 @@ namespace smr::dev
         template <int DIM>
         void launch(int op, const List& l, const ConvSides& sd, const ConvFields& a, double* out, hipStream_t s)
         {
-            const dim3 g(blocks(l.ncells)), b(CB);
+            const unsigned nc = blocks(l.ncells);
+            const dim3 g(nc + blocks((sd.nref + 7) / 8)), b(CB);
             switch (op)
             {
-                case CONV_LINEAR: hipLaunchKernelGGL((k_convection<DIM, CONV_LINEAR>), g, b, 0, s, l, sd, a, out); break;
-                case CONV_BURGERS: hipLaunchKernelGGL((k_convection<DIM, CONV_BURGERS>), g, b, 0, s, l, sd, a, out); break;
-                default: hipLaunchKernelGGL((k_convection<DIM, CONV_FIELD>), g, b, 0, s, l, sd, a, out); break;
+                case CONV_LINEAR: hipLaunchKernelGGL((k_convection<DIM, CONV_LINEAR>), g, b, 0, s, l, sd, a, out, nc); break;
+                case CONV_BURGERS: hipLaunchKernelGGL((k_convection<DIM, CONV_BURGERS>), g, b, 0, s, l, sd, a, out, nc); break;
+                default: hipLaunchKernelGGL((k_convection<DIM, CONV_FIELD>), g, b, 0, s, l, sd, a, out, nc); break;
             }
         }
     } // namespace
@@ -408,9 +475,9 @@ namespace smr::dev
         {
             return;
         }
-        zero_u8(leaf, nref, s);
+        zero_u8(leaf, conv_leaf_bytes(nref), s);
         zero_f64(used, 1, s);
-        hipLaunchKernelGGL(k_leaf_flags, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, leaf);
+        hipLaunchKernelGGL(k_leaf_flags, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, leaf, nref);
         auto* count = reinterpret_cast<unsigned long long*>(used);
         if (dim == 2)
         {

@@ -542,7 +542,7 @@ namespace smr::dev
     // The flux-based convection operators without term lists (convection.hip),
     // on graduated meshes: per cell the kinds of its sides (3 bits each, x-1,
     // x+1, y-1, ...) and where its entries of fine (slots across its faces to
-    // finer cells) begin.
+    // finer cells) begin; per slot whether it is a cell (1 past the slots).
     enum ConvOp : int
     {
         CONV_LINEAR  = 0,
@@ -552,7 +552,10 @@ namespace smr::dev
     struct ConvSides
     {
         const int32_t *word, *fine_at, *fine;
+        const uint8_t* leaf;
+        int64_t nref;
     };
+    constexpr int64_t conv_leaf_bytes(int64_t nref) { return (nref + 7) & ~int64_t(7); }
     struct ConvFields
     {
         const double* u;
@@ -560,11 +563,11 @@ namespace smr::dev
         double vel[3];      // CONV_LINEAR
     };
     // word, fine_at (one per cell) and fine (at most room entries) of the
-    // cells list l; leaf: nref scratch bytes, used: one scratch word; *err = 1
-    // when a stencil slot is missing
+    // cells list l, and leaf (conv_leaf_bytes(nref)); used: one scratch word; *err =
+    // 1 when a stencil slot is missing
     void conv_sides(int dim, const List& l, const Table& t, uint8_t* leaf, int64_t nref, int32_t* word, int32_t* fine_at, int32_t* fine, double* used,
                     int64_t room, int* err, hipStream_t s);
-    // out[cell] = the operator on the cells of l
+    // out[cell] = the operator on the cells of l, 0 in the other slots
     void convection(int dim, int op, const List& l, const ConvSides& sd, const ConvFields& a, double* out, hipStream_t s);
     // out[row[r]] = ordered sum of the terms of row r (flux-based convection)
     void conv_gather(const int64_t* row, const int64_t* ptr, const int64_t* src, const double* coef, int64_t nrows, const double* u,

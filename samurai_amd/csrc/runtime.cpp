@@ -1649,7 +1649,6 @@ namespace smr
         ScopedTimer timer(m.ctx, "convection operator");
         if (const dev::ConvSides* sides = conv_sides(m, dm))
         {
-            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, m.ctx->stream), "hipMemsetAsync(convection)");
             dev::convection(dim, dev::CONV_LINEAR, dm.cells.d, *sides, {u.d, {}, {v[0], v[1], dim == 3 ? v[2] : 0.0}}, out.d, m.ctx->stream);
             return;
         }
@@ -1721,7 +1720,6 @@ namespace smr
         hipStream_t s = m.ctx->stream;
         if (const dev::ConvSides* sides = conv_sides(m, dm))
         {
-            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, s), "hipMemsetAsync(convection)");
             dev::convection(m.host.cfg.dim, dev::CONV_BURGERS, dm.cells.d, *sides, {u.d, {}, {}}, out.d, s);
             return;
         }
@@ -1805,7 +1803,6 @@ namespace smr
         hipStream_t s = m.ctx->stream;
         if (const dev::ConvSides* sides = conv_sides(m, dm))
         {
-            hip_check(hipMemsetAsync(out.d, 0, size_t(out.size) * 8, s), "hipMemsetAsync(convection)");
             dev::convection(dim, dev::CONV_FIELD, dm.cells.d, *sides, {u.d, {vel[0], vel[1], vel[2]}, {}}, out.d, s);
             return;
         }
