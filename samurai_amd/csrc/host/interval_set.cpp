@@ -7,12 +7,22 @@ namespace smr
 {
     int64_t LevelSet::count() const
     {
-        int64_t n = 0;
-        for (const auto& r : runs)
+        // several sums side by side: one waits for its own last addition
+        int64_t n[4]   = {0, 0, 0, 0};
+        size_t k       = 0;
+        const size_t m = runs.size() & ~size_t(3);
+        for (; k < m; k += 4)
         {
-            n += r.e - r.s;
+            n[0] += runs[k].e - runs[k].s;
+            n[1] += runs[k + 1].e - runs[k + 1].s;
+            n[2] += runs[k + 2].e - runs[k + 2].s;
+            n[3] += runs[k + 3].e - runs[k + 3].s;
         }
-        return n;
+        for (; k < runs.size(); ++k)
+        {
+            n[0] += runs[k].e - runs[k].s;
+        }
+        return n[0] + n[1] + n[2] + n[3];
     }
 
     bool LevelSet::operator==(const LevelSet& o) const

@@ -395,18 +395,21 @@ namespace smr
         {
             return true;
         }
-        LevelSet above(m.cfg.dim, MAXL - 1); // the cells of this level with finer leaves in them
-        for (int l = MAXL - 1; l >= 0; --l)
+        // each level within the box, and no cell that holds finer ones (the union
+        // reaches up from max_level)
+        for (int l = 0; l < MAXL; ++l)
         {
             const LevelSet& c = m.ids[CELLS][size_t(l)];
-            const int n       = 1 << l;
-            if ((l > m.cfg.max_level && !c.empty()) || !minus_box(c, {0, 0, 0}, {n, n, n}).empty() || !set_intersection(c, above).empty())
+            const int32_t n   = int32_t(1) << l;
+            bool inside       = l <= m.cfg.max_level || c.empty();
+            for (size_t r = 0; r < c.nrows() && inside; ++r)
+            {
+                inside = c.ry[r] >= 0 && c.ry[r] < n && (m.cfg.dim == 2 || (c.rz[r] >= 0 && c.rz[r] < n))
+                      && c.runs[size_t(c.rp[r])].s >= 0 && c.runs[size_t(c.rp[r + 1]) - 1].e <= n;
+            }
+            if (!inside || !set_intersection(c, m.ids[UNION_CELLS][size_t(l)]).empty())
             {
                 return false;
-            }
-            if (l > 0)
-            {
-                above = on(set_union(c, above), l - 1);
             }
         }
         return true;
