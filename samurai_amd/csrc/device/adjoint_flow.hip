@@ -58,7 +58,7 @@ namespace smr::dev
         }
 
         template <int DIM, int S>
-        __device__ __forceinline__ uint64_t ghost_project(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
+        __device__ __forceinline__ bool ghost_project(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NR     = 1 << (DIM - 1);
             constexpr double inv = 1.0 / double(1 << DIM);
@@ -73,12 +73,11 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + r[1 + (k >> 1)] + (k & 1); };
             Sources<2 * NR, decltype(at)> s;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
-                const bool ok = s.ready(at);
-                if (!ok && !last)
+                if (!s.ready(at) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 double sum = 0;
 #pragma unroll
@@ -87,13 +86,13 @@ namespace smr::dev
                     sum += s.v[2 * q] + s.v[2 * q + 1];
                 }
                 publish(u + r[0], sum * inv);
-                return ok ? DONE : MISSED;
+                return true;
             };
             return until_done(active, w, attempt);
         }
 
         template <int DIM, int S>
-        __device__ __forceinline__ uint64_t ghost_predict(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
+        __device__ __forceinline__ bool ghost_predict(const int32_t* __restrict__ tab, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NY = 2 * S + 1, NZ = DIM == 3 ? NY : 1;
             int32_t r[1 + NZ * NY] = {};
@@ -107,12 +106,11 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + r[1 + k / NY] + k % NY; };
             Sources<NZ * NY * NY, decltype(at)> s;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
-                const bool ok = s.ready(at);
-                if (!ok && !last)
+                if (!s.ready(at) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 double v = s.v[0];
                 if constexpr (S == 1)
@@ -133,7 +131,7 @@ namespace smr::dev
                     }
                 }
                 publish(u + (r[0] & kFlowSlotMask), v);
-                return ok ? DONE : MISSED;
+                return true;
             };
             return until_done(active, w, attempt);
         }
@@ -174,7 +172,7 @@ namespace smr::dev
         };
 
         template <int DIM>
-        __device__ __forceinline__ uint64_t cell_upwind(const AdjointFlow& f, int64_t c, bool active, const double* u, double* out, const FlowWait& w)
+        __device__ __forceinline__ bool cell_upwind(const AdjointFlow& f, int64_t c, bool active, const double* u, double* out, const FlowWait& w)
         {
             CellRec<DIM> r{};
             FlowParam p{};
@@ -185,12 +183,11 @@ namespace smr::dev
             }
             auto at = [&](int k) { return u + (k == 0 ? r.own : r.neighbour(k - 1)); };
             Sources<2 * DIM + 1, decltype(at)> s;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
-                const bool ok = s.ready(at);
-                if (!ok && !last)
+                if (!s.ready(at) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 const double uc = s.v[0];
                 const double FL = flux_h(.5 * p.a[0], .5 * fabs(p.a[0]), s.v[1], uc);
@@ -209,60 +206,9 @@ namespace smr::dev
                     S               = -FL + FR + -FD + FU + -FF + FB;
                 }
                 publish(out + r.own, uc - p.dt * (S * double(1 << r.level())));
-                return ok ? DONE : MISSED;
+                return true;
             };
             return until_done(active, w, attempt);
-        }
-
-        // a lane that missed a source of operation c of item k (a step's, on the
-        // array u, whose cells are the launch's input when input): a fault unless
-        // the launch only reads what it waited for
-        __device__ __forceinline__ void report_missed(const AdjointFlow& f, const LookBack& b, bool input, const FlowWait& w)
-        {
-            if (b.slot < 0 || f.kind[b.slot] == 2 || (f.kind[b.slot] == 1 && !input))
-            {
-                report_fault(w, FAULT_ADJOINT);
-            }
-            else
-            {
-                excuse_faults(w);
-            }
-        }
-
-        template <int DIM, int S>
-        __device__ __forceinline__ void step_missed(const AdjointFlow& f, int k, int64_t c, const double* u, bool input, const FlowWait& w)
-        {
-            LookBack b;
-            keep_apart(c);
-            if (f.op[k] == FLOW_RECIPES)
-            {
-                recipe_sources(f.rec, f.rsrc, c, u, b);
-            }
-            else if (f.op[k] == FLOW_UPWIND)
-            {
-                CellRec<DIM> r;
-                r.load(f.cell, c);
-                b.source(u, r.own);
-#pragma unroll
-                for (int d = 0; d < 2 * DIM; ++d)
-                {
-                    b.source(u, r.neighbour(d));
-                }
-            }
-            else
-            {
-                const bool fine  = f.op[k] == FLOW_PROJECT;
-                const int32_t* t = fine ? f.proj + proj_words(DIM) * c : f.pred + pred_words(DIM, S) * c;
-                const int rows   = fine ? 1 << (DIM - 1) : (DIM == 3 ? (2 * S + 1) * (2 * S + 1) : 2 * S + 1);
-                for (int q = 1; q <= rows; ++q)
-                {
-                    for (int x = 0; x < (fine ? 2 : 2 * S + 1); ++x)
-                    {
-                        b.source(u, t[q] + x);
-                    }
-                }
-            }
-            report_missed(f, b, input, w);
         }
 
         // a.steps time steps: the ghosts of each state, then the next state's
@@ -284,7 +230,7 @@ namespace smr::dev
             const int64_t c  = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + lane;
             const bool act   = c < f.c1[k];
             double* u        = segment_array(a, j, f.n);
-            uint64_t missed  = 0;
+            bool late        = false;
             switch (f.op[k])
             {
                 case FLOW_RECIPES:
@@ -295,21 +241,21 @@ namespace smr::dev
                         const int4 r = reinterpret_cast<const int4*>(f.rec)[c];
                         bc           = (r.y & 255) == 1 ? f.par[r.w].bc : 0.0;
                     }
-                    missed = flow_recipe(f.rec, f.rsrc, c, act, u, bc, fw);
+                    late = flow_recipe(f.rec, f.rsrc, c, act, u, bc, fw);
                     break;
                 }
-                case FLOW_PROJECT: missed = ghost_project<DIM, S>(f.proj, c, act, u, fw); break;
-                case FLOW_PREDICT: missed = ghost_predict<DIM, S>(f.pred, c, act, u, fw); break;
+                case FLOW_PROJECT: late = ghost_project<DIM, S>(f.proj, c, act, u, fw); break;
+                case FLOW_PREDICT: late = ghost_predict<DIM, S>(f.pred, c, act, u, fw); break;
                 default:
                     if (j + 1 < a.steps || last)
                     {
-                        missed = cell_upwind<DIM>(f, c, act, u, segment_array(a, j + 1, f.n), fw);
+                        late = cell_upwind<DIM>(f, c, act, u, segment_array(a, j + 1, f.n), fw);
                     }
                     break;
             }
-            if ((missed >> lane) & 1)
+            if (late)
             {
-                step_missed<DIM, S>(f, k, c, u, j == 0, fw);
+                report_fault(fw, FAULT_ADJOINT);
             }
         }
 
@@ -319,7 +265,6 @@ namespace smr::dev
         {
             int32_t k, end;
             double group = 0;
-            bool missed  = false;
             __device__ __forceinline__ bool run(const AdjointFlow& f, const double* mu, double& m, bool last)
             {
                 for (; k < end; ++k)
@@ -330,13 +275,9 @@ namespace smr::dev
                     if (marked(x))
                     {
                         x = look_again(p);
-                        if (marked(x))
+                        if (marked(x) && !last)
                         {
-                            if (!last)
-                            {
-                                return false;
-                            }
-                            missed = true;
+                            return false;
                         }
                     }
                     group += f.ew[k] * x;
@@ -349,15 +290,6 @@ namespace smr::dev
                 return true;
             }
         };
-
-        // the sources of operation q of an adjoint step
-        __device__ __forceinline__ void gathered_sources(const AdjointFlow& f, int64_t q, const double* lam, LookBack& b)
-        {
-            for (int32_t e = f.rowptr[q]; e < f.rowptr[q + 1]; ++e)
-            {
-                b.source(lam, f.esrc[e] & kFlowSlotMask);
-            }
-        }
 
         // a.steps adjoint steps: per step the ghosts' adjoint values, then the
         // cells' of the step before
@@ -399,7 +331,7 @@ namespace smr::dev
                     in.end   = f.rowptr[q + 1];
                 }
                 int d = 0;
-                auto attempt = [&](bool last) -> int
+                auto attempt = [&](bool last)
                 {
 #pragma unroll
                     for (int e = 0; e < 2 * DIM; ++e)
@@ -412,13 +344,9 @@ namespace smr::dev
                                 if (marked(x))
                                 {
                                     x = look_again(lam + cells[e]);
-                                    if (marked(x))
+                                    if (marked(x) && !last)
                                     {
-                                        if (!last)
-                                        {
-                                            return WAITS;
-                                        }
-                                        in.missed = true;
+                                        return false;
                                     }
                                 }
                                 const double aa = p.a[e >> 1];
@@ -429,27 +357,15 @@ namespace smr::dev
                     }
                     if (!in.run(f, lam, m, last))
                     {
-                        return WAITS;
+                        return false;
                     }
                     publish(lam + dst, m);
-                    return in.missed ? MISSED : DONE;
+                    return true;
                 };
-                const uint64_t missed = until_done(act, fw, attempt);
-                if ((missed >> lane) & 1)
+                const bool late = until_done(act, fw, attempt);
+                if (late)
                 {
-                    LookBack b;
-                    int64_t g2 = q;
-                    keep_apart(g2);
-                    for (int e = 0; e < 2 * DIM; ++e)
-                    {
-                        const int32_t beside = f.aghost[8 * g2 + 2 + e];
-                        if (beside >= 0)
-                        {
-                            b.source(lam, beside);
-                        }
-                    }
-                    gathered_sources(f, g2, lam, b);
-                    report_missed(f, b, j == 0, fw);
+                    report_fault(fw, FAULT_ADJOINT);
                 }
                 return;
             }
@@ -472,17 +388,13 @@ namespace smr::dev
             Sources<2 * DIM + 1, decltype(at)> s;
             bool begun = false;
             double m   = 0;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
                 if (!begun)
                 {
-                    if (!s.ready(at))
+                    if (!s.ready(at) && !last)
                     {
-                        if (!last)
-                        {
-                            return WAITS;
-                        }
-                        in.missed = true;
+                        return false;
                     }
                     const double k = p.dt * ldexp(1.0, r.level());
                     double v[2 * DIM];
@@ -506,26 +418,15 @@ namespace smr::dev
                 }
                 if (!in.run(f, lam, m, last))
                 {
-                    return WAITS;
+                    return false;
                 }
                 publish(out + r.own, m);
-                return in.missed ? MISSED : DONE;
+                return true;
             };
-            const uint64_t missed = until_done(act, fw, attempt);
-            if ((missed >> lane) & 1)
+            const bool late = until_done(act, fw, attempt);
+            if (late)
             {
-                LookBack b;
-                int64_t c2 = c;
-                keep_apart(c2);
-                CellRec<DIM> r2;
-                r2.load(f.cell, c2);
-                b.source(lam, r2.own);
-                for (int d = 0; d < 2 * DIM; ++d)
-                {
-                    b.source(lam, r2.ghost(d) ? r2.own : r2.neighbour(d));
-                }
-                gathered_sources(f, f.naghost + c2, lam, b);
-                report_missed(f, b, j == 0, fw);
+                report_fault(fw, FAULT_ADJOINT);
             }
         }
 
@@ -593,7 +494,8 @@ namespace smr::dev
             }
         }
 
-        // compact cell vectors: to = 1 from the array, 0 into it
+        // compact cell vectors: to = 1 from the array, 0 into it (stored quiet, so
+        // that no cell of an array holds the bits of the mark)
         __global__ __launch_bounds__(256) void k_adj_cells(const int32_t* __restrict__ cell, int words, int64_t ncells, double* array, double* compact,
                                                            int to)
         {
@@ -609,7 +511,7 @@ namespace smr::dev
             }
             else
             {
-                *p = compact[c];
+                publish(p, compact[c]);
             }
         }
 

@@ -346,9 +346,9 @@ namespace smr::dev
 
     // The waits of a dataflow launch (flow_ops.hpp): the rounds after which a
     // wave gives up, and the context's fault words (pinned host memory).  A wave
-    // that gave up on a value of the launch itself sets the first to one of
-    // Fault, one that gave up on a value it only reads sets the second.
-    // Ctx::sync reads and clears them, and throws for the first without the second.
+    // that gave up sets the first to one of Fault, and the second when what it
+    // waited for is an input that holds the bits of the mark.  Ctx::sync reads and
+    // clears them, and throws for the first without the second.
     struct FlowWait
     {
         int rounds;

@@ -25,8 +25,8 @@
 // where the cells tile the box (the other meshes keep the staged launches), so
 // the lowest unfinished wave waits for nothing that is not done; and a wave
 // gives up after FlowWait::rounds looks and uses what it has read (the right
-// value when a cell itself holds the bits of the mark; when the source is a
-// ghost of the update, the fault word says so).
+// value when a cell itself holds the bits of the mark; otherwise the fault words
+// say so).
 #include "flow_ops.hpp"
 
 namespace smr::dev
@@ -35,7 +35,7 @@ namespace smr::dev
     {
         // projection_op_ (op_project_at) on waited-for sources
         template <int DIM>
-        __device__ __forceinline__ uint64_t flow_project(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
+        __device__ __forceinline__ bool flow_project(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NR     = 1 << (DIM - 1);
             constexpr double inv = 1.0 / double(1 << DIM);
@@ -54,12 +54,11 @@ namespace smr::dev
             }
             auto at = [&](int k) { return row[k >> 1] + (k & 1); };
             Sources<2 * NR, decltype(at)> s;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
-                const bool ok = s.ready(at);
-                if (!ok && !last)
+                if (!s.ready(at) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 double sum = 0;
 #pragma unroll
@@ -68,14 +67,14 @@ namespace smr::dev
                     sum += s.v[2 * r] + s.v[2 * r + 1];
                 }
                 publish(dst, sum * inv);
-                return ok ? DONE : MISSED;
+                return true;
             };
             return until_done(active, w, attempt);
         }
 
         // prediction_op <s,false> (op_predict_fine_at) on waited-for sources
         template <int DIM, int S>
-        __device__ __forceinline__ uint64_t flow_predict(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
+        __device__ __forceinline__ bool flow_predict(const List& l, int64_t c, bool active, double* u, const FlowWait& w)
         {
             constexpr int NY = 2 * S + 1, NZ = DIM == 3 ? NY : 1, N = NZ * NY * NY;
             double* dst = nullptr;
@@ -97,12 +96,11 @@ namespace smr::dev
             }
             auto at = [&](int k) { return row[k / NY] + k % NY; };
             Sources<N, decltype(at)> s;
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
-                const bool ok = s.ready(at);
-                if (!ok && !last)
+                if (!s.ready(at) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 double v;
                 if constexpr (S == 0)
@@ -135,7 +133,7 @@ namespace smr::dev
                     }
                 }
                 publish(dst, v);
-                return ok ? DONE : MISSED;
+                return true;
             };
             return until_done(active, w, attempt);
         }
@@ -186,16 +184,47 @@ namespace smr::dev
             return false;
         }
 
-        // a lane that missed a source of ghost c of item k: a fault unless the
-        // update does not write what it waited for
-        template <int DIM, int S>
-        __device__ __forceinline__ void flow_missed(const GhostFlow& f, int k, int64_t c, const double* u, const FlowWait& w)
+        // whether slot holds the mark and the update does not write it
+        __device__ __forceinline__ bool marked_input(const GhostFlow& f, const double* u, int64_t slot)
         {
-            LookBack b;
-            keep_apart(c);
+            if (!marked(look_again(u + slot)) || in_list(f.proj, slot) || in_list(f.pred, slot))
+            {
+                return false;
+            }
+            for (int k = 0; k < f.nitems; ++k)
+            {
+                for (int32_t c = f.op[k] == SEQ_RECIPES ? f.c0[k] : f.c1[k]; c < f.c1[k]; ++c)
+                {
+                    if (f.rec[4 * int64_t(c)] == slot)
+                    {
+                        return false;
+                    }
+                }
+            }
+            return true;
+        }
+
+        // a wave that gave up, on ghost c of item k: a fault, unless some wave
+        // waited for an input that holds the mark
+        template <int DIM, int S>
+        __device__ __forceinline__ void gave_up(const GhostFlow& f, int k, int64_t c, bool active, const double* u, const FlowWait& w)
+        {
+            report_fault(w, FAULT_GHOSTS);
+            if (!active)
+            {
+                return;
+            }
+            // the sources are located anew, so that the wait holds no registers
+            // for this (kept from before it: 126 -> 166 in 3D)
+            asm volatile("" : "+v"(c));
+            bool input = false;
             if (f.op[k] == SEQ_RECIPES)
             {
-                recipe_sources(f.rec, f.rsrc, c, u, b);
+                const int4 r = reinterpret_cast<const int4*>(f.rec)[c];
+                for (int q = 0; q < r.y >> 8; ++q)
+                {
+                    input = input || marked_input(f, u, q == 0 ? r.z : f.rsrc[r.w + q]);
+                }
             }
             else
             {
@@ -205,27 +234,12 @@ namespace smr::dev
                 const int64_t* row = bases(l, cell.run);
                 const int n        = fine ? 2 : 2 * S + 1;
                 const int32_t x0   = fine ? 2 * cell.x : (cell.x >> 1) - S;
-                for (int r = 1; r < l.ntaps; ++r)
+                for (int q = 0; q < n * (l.ntaps - 1); ++q)
                 {
-                    for (int x = 0; x < n; ++x)
-                    {
-                        b.source(u, row[r] + x0 + x);
-                    }
+                    input = input || marked_input(f, u, row[1 + q / n] + x0 + q % n);
                 }
             }
-            bool own = b.slot < 0 || in_list(f.proj, b.slot) || in_list(f.pred, b.slot);
-            for (int q = 0; q < f.nitems; ++q)
-            {
-                for (int32_t e = f.op[q] == SEQ_RECIPES ? f.c0[q] : f.c1[q]; e < f.c1[q]; ++e)
-                {
-                    own = own || f.rec[4 * int64_t(e)] == b.slot;
-                }
-            }
-            if (own)
-            {
-                report_fault(w, FAULT_GHOSTS);
-            }
-            else
+            if (input)
             {
                 excuse_faults(w);
             }
@@ -238,16 +252,16 @@ namespace smr::dev
             const int k       = item_of(f, w);
             const int64_t c   = int64_t(f.c0[k]) + int64_t(w - f.wave0[k]) * 64 + int(threadIdx.x & 63);
             const bool active = c < f.c1[k];
-            uint64_t missed;
+            bool late;
             switch (f.op[k])
             {
-                case SEQ_RECIPES: missed = flow_recipe(f.rec, f.rsrc, c, active, u, bc, fw); break;
-                case SEQ_PROJECT: missed = flow_project<DIM>(f.proj, c, active, u, fw); break;
-                default: missed = flow_predict<DIM, S>(f.pred, c, active, u, fw); break;
+                case SEQ_RECIPES: late = flow_recipe(f.rec, f.rsrc, c, active, u, bc, fw); break;
+                case SEQ_PROJECT: late = flow_project<DIM>(f.proj, c, active, u, fw); break;
+                default: late = flow_predict<DIM, S>(f.pred, c, active, u, fw); break;
             }
-            if ((missed >> (threadIdx.x & 63)) & 1)
+            if (late)
             {
-                flow_missed<DIM, S>(f, k, c, u, fw);
+                gave_up<DIM, S>(f, k, c, active, u, fw);
             }
         }
 

@@ -6,7 +6,7 @@
 // no rule uses), k_tag_flow closes them, finest level first: blocks take their
 // place from a counter, so the lowest unfinished wave waits for nothing that is
 // not done, and a wave gives up waiting after FlowWait::rounds looks (which
-// only a broken order would make it do: the fault word says so).  The tags
+// only a broken order would make it do: the fault words say so).  The tags
 // travel through agent-scope byte loads and stores.
 //
 // Bound: latency, a store-to-load trip per level.  The staged form is a launch
@@ -66,7 +66,7 @@ namespace smr::dev
                     row[r] = tag + b[1 + r] + 2 * cell.x;
                 }
             }
-            auto attempt = [&](bool last) -> int
+            auto attempt = [&](bool last)
             {
                 unsigned t[2 * NR], any = 0, all = 2;
 #pragma unroll
@@ -78,7 +78,7 @@ namespace smr::dev
                 }
                 if ((any & kOpen) && !last)
                 {
-                    return WAITS;
+                    return false;
                 }
                 // a child that is kept keeps the others, and the
                 // cell; the children go together or not at all
@@ -93,10 +93,10 @@ namespace smr::dev
                     }
                 }
                 __hip_atomic_store(own, uint8_t(keep || all ? v | 1u : v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                return any & kOpen ? MISSED : DONE;
+                return true;
             };
-            const uint64_t missed = until_done(active, fw, attempt);
-            if (missed != 0)
+            const bool late = until_done(active, fw, attempt);
+            if (late)
             {
                 report_fault(fw, FAULT_TAGS);
             }

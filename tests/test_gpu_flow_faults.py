@@ -76,6 +76,13 @@ def test_gradient(ctx, host_ctx, dim, lmin, lmax, s):
     ctx.set_wait_rounds(1 << 17)
     for a, b in zip(want, both()):
         assert np.array_equal(a, b)
+    # values with the bits the launches mark their slots with are only NaN
+    u0[0] = gT[1] = torch.tensor([0x7FF05A3C96E1D2B4]).view(torch.float64)[0]
+    torch.cuda.synchronize()
+    got = both()
+    p.set_tuning(256, 0, 1)
+    for a, b in zip(got, both()):
+        assert np.isnan(a).any() and np.array_equal(a, b, equal_nan=True)
 
 
 def large_coarse_levels(mesh):
