@@ -853,6 +853,10 @@ namespace smr
     void Adjoint::forward(const double* u0, double* uT)
     {
         check_meshes();
+        if (staged_)
+        {
+            flow_ = nullptr;
+        }
         if (flow_)
         {
             ScopedTimer t(ctx_, "adjoint forward");

@@ -66,11 +66,12 @@ namespace smr
         void forward(const double* u0, double* uT);
         // gT = dL/duT -> g0 = dL/du0 (device), ga = dL/da (host, n*3)
         void backward(const double* gT, double* g0, double* ga);
-        // selects the stage programs, in that launch shape
+        // selects the stage programs, in that launch shape, from the next forward
+        // on (a backward before it belongs to the last forward)
         void set_tuning(const Tuning& t)
         {
             tuning_ = t;
-            flow_   = nullptr;
+            staged_ = true;
         }
         const Tuning& tuning() const { return tuning_; }
         int steps() const { return steps_; }
@@ -145,6 +146,7 @@ namespace smr
         // adjoint steps per launch (their arrays are all in memory)
         static constexpr int kFlowSteps = 16;
         std::unique_ptr<Flow> flow_;
+        bool staged_         = false; // the next forward gives flow_ up
         bool forward_done_   = false; // with the velocity set last
         bool programs_built_ = false; // the lists and arrays of the stage programs
         std::unique_ptr<Flow> make_flow();

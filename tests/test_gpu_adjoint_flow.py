@@ -54,3 +54,31 @@ def test_flow_matches_stage_programs(gpu_ctx, dim, lmax, s, n, steps, every):
     for got, want in zip(flow, staged):
         for g, w in zip(got, want):
             assert np.array_equal(g, w)
+
+
+def test_tuning_between_forward_and_backward(gpu_ctx):
+    """A launch shape set after a forward is used from the next one on: the
+    backward of the one before still has its states."""
+    import samurai_amd as sa
+    import torch
+    print("tuning in between", flush=True)
+    mesh, u = frozen(sa, gpu_ctx, 2, 6, 1, 7)
+    p = sa.AdjointProblem(gpu_ctx, [mesh], [0.2 / 64], bc=[0.5], steps=6, checkpoint_every=3)
+    u0 = torch.tensor(u, device="cuda")
+    gT = torch.tensor(np.random.default_rng(3).standard_normal(u0.numel()), device="cuda")
+    uT, g0 = torch.empty_like(u0), torch.empty_like(u0)
+    torch.cuda.synchronize()
+    p.set_velocity([[0.7, -0.3]])
+    got = []
+    for shape in ((256, 0, 1), (512, 2, 0), None):
+        p.forward_ptr(u0.data_ptr(), uT.data_ptr())
+        if shape:
+            p.set_tuning(*shape)
+        ga = p.backward_ptr(gT.data_ptr(), g0.data_ptr())
+        got.append((uT.cpu().numpy(), g0.cpu().numpy(), ga))
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a, b)
+    p.set_velocity([[0.1, -0.3]])
+    with pytest.raises(sa.SamuraiError):
+        p.backward_ptr(gT.data_ptr(), g0.data_ptr())
