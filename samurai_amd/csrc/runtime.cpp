@@ -1588,21 +1588,10 @@ namespace smr
 
     namespace
     {
-        // the cells fill the unit box
-        bool fills_box(const MRMeshData& m)
-        {
-            const CellArray& cells = m.ids[CELLS];
-            double volume          = 0; // sums of powers of two, exact
-            for (int l = 0; l < MAXL; ++l)
-            {
-                volume += std::ldexp(double(cells[size_t(l)].count()), -m.cfg.dim * l);
-            }
-            return volume == 1.0;
-        }
-
         // the side table of m's cells, or null where the operators run on term
-        // lists: a mesh that is not graduated or has holes (jumps of several
-        // levels, part-refined faces), or more table entries than an int32 counts
+        // lists: a mesh that is not graduated (jumps of several levels) or does not
+        // tile the box (part-refined faces, cells over cells), or more table
+        // entries than an int32 counts
         const dev::ConvSides* conv_sides(Mesh& m, DevMesh& dm)
         {
             const int dim     = m.host.cfg.dim;
@@ -1611,7 +1600,7 @@ namespace smr
             const int64_t room = ca_min_level(cells) == ca_max_level(cells) ? 0 : 2 * dim * n;
             if (!dm.sides)
             {
-                if (!m.host.graduated || room > INT32_MAX || m.host.nref > INT32_MAX || !fills_box(m.host))
+                if (!m.host.graduated || !m.host.tiles || room > INT32_MAX || m.host.nref > INT32_MAX)
                 {
                     return nullptr;
                 }
