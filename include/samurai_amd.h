@@ -266,6 +266,11 @@ int smr_ctx_set_ghost_form(smr_ctx* ctx, int form);
  * context's work then returns SMR_ERR_RUNTIME, unless the value is one the
  * launch does not write. */
 int smr_ctx_set_wait_rounds(smr_ctx* ctx, int rounds);
+/* Diagnostics: at most n entries for the tables the flux operators build of the
+ * faces to finer cells (by default as many as there can be).  When a table is
+ * incomplete, the next call that waits for the context's work returns
+ * SMR_ERR_RUNTIME, and from then on the operators run on term lists. */
+int smr_ctx_set_side_entries(smr_ctx* ctx, int64_t n);
 /* The HIP stream (hipStream_t) the context orders its work on, for timing
  * with HIP events; NULL for a host-only context. */
 void* smr_ctx_stream(smr_ctx* ctx);

@@ -83,6 +83,7 @@ def lib():
         _sig(L, "smr_mesh_ghost_form", "argtypes", [vp])
         _sig(L, "smr_ctx_set_ghost_form", "argtypes", [vp, i32])
         _sig(L, "smr_ctx_set_wait_rounds", "argtypes", [vp, i32])
+        _sig(L, "smr_ctx_set_side_entries", "argtypes", [vp, i64])
         _sig(L, "smr_timers_enable", "argtypes", [i32])
         _sig(L, "smr_timers_report", "restype", i64)
         _sig(L, "smr_timers_report", "argtypes", [ctypes.c_char_p, i64])
@@ -210,6 +211,10 @@ class Context:
     def set_wait_rounds(self, rounds):
         """After how many rounds a wave of a dataflow launch gives up waiting (diagnostics; the default is 2**17)."""
         _check(lib().smr_ctx_set_wait_rounds(self.h, int(rounds)))
+
+    def set_side_entries(self, n):
+        """Room for the flux operators' tables of the faces to finer cells (diagnostics)."""
+        _check(lib().smr_ctx_set_side_entries(self.h, int(n)))
 
     def stream(self):
         """The hipStream_t (as an integer) all work of this context runs on."""

@@ -634,6 +634,17 @@ extern "C"
             });
     }
 
+    int smr_ctx_set_side_entries(smr_ctx* ctx, int64_t n)
+    {
+        return guarded(
+            [&]
+            {
+                require(ctx && n >= 0, "a number of entries is expected");
+                ctx->c.side_entries = n;
+                return 0;
+            });
+    }
+
     int smr_mesh_check_device_lists(smr_mesh* mesh)
     {
         return guarded(

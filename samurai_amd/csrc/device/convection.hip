@@ -116,12 +116,13 @@ namespace smr::dev
         // -1 where no interface is
         template <int DIM>
         __global__ __launch_bounds__(CB) void k_side_kinds(List l, Table t, const uint8_t* __restrict__ leaf, int32_t* word, int32_t* fine_at,
-                                                           int32_t* fine, unsigned long long* used, int64_t room, int* err)
+                                                           int32_t* fine, unsigned long long* used, int64_t room, int* fault)
         {
             constexpr int NF = 1 << (DIM - 1); // entries of a side
             const int64_t c   = int64_t(blockIdx.x) * CB + threadIdx.x;
             const bool active = c < l.ncells;
             int32_t w = 0, n = 0;
+            bool fail = false;
             int32_t slots[2 * DIM * NF];
             if (active)
             {
@@ -184,7 +185,7 @@ namespace smr::dev
                                     const bool ok = in >= 0 && out >= 0 && leaf[out] && leaf[out + 1];
                                     if (out >= 0 && (leaf[out] || leaf[out + 1]) && !ok)
                                     {
-                                        err[0] = 1;
+                                        fail = true;
                                     }
                                     e[2 * f]     = ok ? int32_t(in) : -1;
                                     e[2 * f + 1] = ok ? int32_t(out) : -1;
@@ -229,9 +230,13 @@ namespace smr::dev
             }
             if (at + n > room)
             {
-                err[0]  = 1;
+                fail    = true;
                 w       = 0;
                 n       = 0;
+            }
+            if (fail)
+            {
+                __hip_atomic_store(fault, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             }
             word[c]    = w;
             fine_at[c] = int32_t(at);
@@ -469,7 +474,7 @@ namespace smr::dev
     } // namespace
 
     void conv_sides(int dim, const List& l, const Table& t, uint8_t* leaf, int64_t nref, int32_t* word, int32_t* fine_at, int32_t* fine, double* used,
-                    int64_t room, int* err, hipStream_t s)
+                    int64_t room, int* fault, hipStream_t s)
     {
         if (l.ncells <= 0)
         {
@@ -481,11 +486,11 @@ namespace smr::dev
         auto* count = reinterpret_cast<unsigned long long*>(used);
         if (dim == 2)
         {
-            hipLaunchKernelGGL(k_side_kinds<2>, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, t, leaf, word, fine_at, fine, count, room, err);
+            hipLaunchKernelGGL(k_side_kinds<2>, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, t, leaf, word, fine_at, fine, count, room, fault);
         }
         else
         {
-            hipLaunchKernelGGL(k_side_kinds<3>, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, t, leaf, word, fine_at, fine, count, room, err);
+            hipLaunchKernelGGL(k_side_kinds<3>, dim3(blocks(l.ncells)), dim3(CB), 0, s, l, t, leaf, word, fine_at, fine, count, room, fault);
         }
     }
 

@@ -563,10 +563,10 @@ namespace smr::dev
         double vel[3];      // CONV_LINEAR
     };
     // word, fine_at (one per cell) and fine (at most room entries) of the
-    // cells list l, and leaf (conv_leaf_bytes(nref)); used: one scratch word; *err =
-    // 1 when a stencil slot is missing
+    // cells list l, and leaf (conv_leaf_bytes(nref)); used: one scratch word; *fault
+    // = 1 when a face lacks its pair or there is no room
     void conv_sides(int dim, const List& l, const Table& t, uint8_t* leaf, int64_t nref, int32_t* word, int32_t* fine_at, int32_t* fine, double* used,
-                    int64_t room, int* err, hipStream_t s);
+                    int64_t room, int* fault, hipStream_t s);
     // out[cell] = the operator on the cells of l, 0 in the other slots
     void convection(int dim, int op, const List& l, const ConvSides& sd, const ConvFields& a, double* out, hipStream_t s);
     // out[row[r]] = ordered sum of the terms of row r (flux-based convection)

@@ -395,9 +395,9 @@ namespace smr
 
     void Ctx::allocate_fault_words()
     {
-        hip_check(hipHostMalloc(reinterpret_cast<void**>(&fault), 2 * sizeof(int), hipHostMallocMapped), "hipHostMalloc(fault words)");
-        fault[0] = fault[1] = 0;
-        void* p             = nullptr;
+        hip_check(hipHostMalloc(reinterpret_cast<void**>(&fault), 3 * sizeof(int), hipHostMallocMapped), "hipHostMalloc(fault words)");
+        fault[0] = fault[1] = fault[2] = 0;
+        void* p                        = nullptr;
         hip_check(hipHostGetDevicePointer(&p, fault, 0), "hipHostGetDevicePointer(fault words)");
         wait.fault = static_cast<int*>(p);
     }
@@ -406,12 +406,18 @@ namespace smr
     {
         hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
         volatile int* f = fault;
-        if (!f || (f[0] == 0 && f[1] == 0))
+        if (!f || (f[0] == 0 && f[1] == 0 && f[2] == 0))
         {
             return;
         }
         const int code = f[1] ? 0 : f[0];
-        f[0] = f[1] = 0;
+        const bool sides = f[2] != 0;
+        f[0] = f[1] = f[2] = 0;
+        if (sides)
+        {
+            no_sides = true;
+            throw std::runtime_error("flux operator: the side table of a mesh is incomplete (the next calls use term lists)");
+        }
         switch (code)
         {
             case 0: return;
@@ -1597,10 +1603,15 @@ namespace smr
             const int dim     = m.host.cfg.dim;
             const int64_t n   = dm.cells.d.ncells;
             const auto& cells = m.host.ids[CELLS];
-            const int64_t room = ca_min_level(cells) == ca_max_level(cells) ? 0 : 2 * dim * n;
+            const int64_t full = ca_min_level(cells) == ca_max_level(cells) ? 0 : 2 * dim * n;
+            const int64_t room = std::min(full, m.ctx->side_entries);
+            if (m.ctx->no_sides)
+            {
+                return nullptr; // a table was incomplete, perhaps this one
+            }
             if (!dm.sides)
             {
-                if (!m.host.graduated || !m.host.tiles || room > INT32_MAX || m.host.nref > INT32_MAX)
+                if (!m.host.graduated || !m.host.tiles || full > INT32_MAX || m.host.nref > INT32_MAX)
                 {
                     return nullptr;
                 }
@@ -1615,7 +1626,7 @@ namespace smr
                 auto* used    = reinterpret_cast<double*>(p + 2 * wb + fb);
                 DevBuffer leaf;
                 dev::conv_sides(dim, dm.cells.d, dm.table, static_cast<uint8_t*>(leaf.get(size_t(m.host.nref), s)), m.host.nref, word, fine_at, fine,
-                                used, room, m.ctx->d_err, s);
+                                used, room, m.ctx->wait.fault + 2, s);
                 sides->d = {word, fine_at, fine};
                 dm.sides = std::move(sides);
             }

@@ -364,11 +364,13 @@ namespace smr
         // dataflow launch wherever there is one
         int ghost_form = -1;
         // what a kernel reports that went on without a value it needed
-        // (dev::FlowWait): two words of pinned host memory, and the waits of the
-        // dataflow launches, which write them
+        // (dev::FlowWait; the third word: a side table was incomplete): words of
+        // pinned host memory, and the waits of the dataflow launches
         int* fault = nullptr;
         dev::FlowWait wait{1 << 17, nullptr};
         void allocate_fault_words();
+        int64_t side_entries = INT64_MAX; // room for a side table's entries
+        bool no_sides        = false;     // set when one was incomplete
         void mark_runs_back();
         ~Ctx();
         int* d_flag() const { return d_err + 1; }

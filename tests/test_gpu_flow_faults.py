@@ -1,6 +1,7 @@
 """A wave of a dataflow launch that goes on without a value of the launch says
 so: with no rounds to wait (the kernels end as ever, at once) the next call that
-waits for the context's work fails, and the context works on afterwards."""
+waits for the context's work fails, and the context works on afterwards.  So
+does a side table without room."""
 import numpy as np
 import pytest
 
@@ -112,3 +113,20 @@ def test_tags(ctx, host_ctx, dim, lmin, lmax):
             with pytest.raises(sa.SamuraiError, match="tag finalization"):
                 ctx.synchronize()
     assert torch.equal(tags[0], tags[2])
+
+
+@pytest.mark.parametrize("dim,lmin,lmax,s", [(2, 2, 6, 1), (3, 2, 4, 0)])
+def test_side_table(ctx, host_ctx, dim, lmin, lmax, s):
+    print("side table fault", dim, lmin, lmax, s, flush=True)
+    ops = (sa.make_convection_upwind([0.6, -0.8, 0.3][:dim]), sa.make_convection_upwind())
+    mesh, u = field(ctx, host_ctx, dim, lmin, lmax, s)
+    out = sa.make_scalar_field("f", mesh)
+    want = [op(u, out=out).storage() for op in ops]
+    ctx.set_side_entries(8)
+    mesh, u = field(ctx, host_ctx, dim, lmin, lmax, s)  # its table is built anew
+    out = sa.make_scalar_field("f", mesh)
+    with pytest.raises(sa.SamuraiError, match="side table"):
+        ops[0](u, out=out).storage()
+    for _ in range(2):
+        for op, w in zip(ops, want):
+            assert np.array_equal(op(u, out=out).storage(), w)
