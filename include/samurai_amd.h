@@ -261,6 +261,8 @@ int smr_mesh_ghost_form(smr_mesh* mesh);
  * default): the cheaper one; 0: the launches per stage; 1: the dataflow launch
  * wherever it exists. */
 int smr_ctx_set_ghost_form(smr_ctx* ctx, int form);
+/* The same for the maximum pass of the tags. */
+int smr_ctx_set_tag_form(smr_ctx* ctx, int form);
 /* Diagnostics: the rounds after which a wave of a dataflow launch gives up
  * waiting for a value (default 2^17).  The next call that waits for the
  * context's work then returns SMR_ERR_RUNTIME, unless the value is one the

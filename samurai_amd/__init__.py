@@ -82,6 +82,7 @@ def lib():
         _sig(L, "smr_mesh_ghost_update_bytes", "argtypes", [vp])
         _sig(L, "smr_mesh_ghost_form", "argtypes", [vp])
         _sig(L, "smr_ctx_set_ghost_form", "argtypes", [vp, i32])
+        _sig(L, "smr_ctx_set_tag_form", "argtypes", [vp, i32])
         _sig(L, "smr_ctx_set_wait_rounds", "argtypes", [vp, i32])
         _sig(L, "smr_ctx_set_side_entries", "argtypes", [vp, i64])
         _sig(L, "smr_timers_enable", "argtypes", [i32])
@@ -207,6 +208,10 @@ class Context:
     def set_ghost_form(self, form):
         """-1: update_ghost_mr in its cheaper form (the default), 0: a launch per stage, 1: the dataflow launch wherever it exists."""
         _check(lib().smr_ctx_set_ghost_form(self.h, int(form)))
+
+    def set_tag_form(self, form):
+        """-1: the maximum pass of the tags in its cheaper form (the default), 0: a launch per level, 1: the dataflow launch."""
+        _check(lib().smr_ctx_set_tag_form(self.h, int(form)))
 
     def set_wait_rounds(self, rounds):
         """After how many rounds a wave of a dataflow launch gives up waiting (diagnostics; the default is 2**17)."""

@@ -623,6 +623,17 @@ extern "C"
             });
     }
 
+    int smr_ctx_set_tag_form(smr_ctx* ctx, int form)
+    {
+        return guarded(
+            [&]
+            {
+                require(ctx && form >= -1 && form <= 1, "a tag form of -1, 0 or 1 is expected");
+                ctx->c.tag_form = form;
+                return 0;
+            });
+    }
+
     int smr_ctx_set_wait_rounds(smr_ctx* ctx, int rounds)
     {
         return guarded(

@@ -2448,9 +2448,15 @@ namespace smr
         {
             ScopedTimer timer(&ctx, "tag finalization");
             const SeqPlan& plan = max_plan(ctx, dm, cfg);
-            // two launches instead of three and more (tag_flow.hip); the word
-            // behind the first field's values is free after its ghost update
-            if (plan.steps.size() > 2)
+            // two launches instead of three and more (tag_flow.hip), unless the
+            // tickets of their blocks cost more: 10 ns per 256 cells against
+            // 3.7 us per launch.  Whole calls, two launches against three: 88 K
+            // coarse cells 61.3 / 63.0 us, 246 K 98.0 / 89.4, 750 K 166 / 138,
+            // 2.7 M 570 / 457 (a larger block trades few cells' time for many:
+            // with 1024 threads 246 K 89.1, 2.7 M 480).  The word behind the first
+            // field's values is free after its ghost update.
+            const auto steps = int64_t(plan.steps.size());
+            if (ctx.tag_form >= 0 ? ctx.tag_form == 1 : steps > 2 && dm.maximum.d.ncells <= 110000 + 90000 * (steps - 3))
             {
                 dev::tag_flow(dim, dm.maximum.d, tag, reinterpret_cast<unsigned*>(fs[0]->d + n), ctx.wait, s);
                 return;

@@ -363,6 +363,7 @@ namespace smr
         // update_ghost_mr: -1 the cheaper form, 0 the staged launches, 1 the
         // dataflow launch wherever there is one
         int ghost_form = -1;
+        int tag_form   = -1; // the same for the maximum pass of the tags
         // what a kernel reports that went on without a value it needed
         // (dev::FlowWait; the third word: a side table was incomplete): words of
         // pinned host memory, and the waits of the dataflow launches
