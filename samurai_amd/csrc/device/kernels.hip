@@ -243,6 +243,12 @@ namespace smr::dev
         // weights from 0.1, 0.6, 0.3 with eps = 1e-6 (2.15-2.16), weighted sum
         // (2.10), in the reference's operation order; its pow(x, 2) is the
         // correctly rounded square x * x.
+        // NEWTON: the divisions by newton_rcp, for meshes of 2^17 cells and more (on
+        // smaller ones, where a launch is short, the second copy of the arithmetic
+        // costs more than it gives; whole calls without / with it: 2D L5 13.6 /
+        // 13.9 us, L8 16.3 / 16.5, L9 20.2 / 19.9; 3D L3 15.8 / 16.4, L5 18.7 / 19.1,
+        // L6 26.7 / 26.2).
+        template <bool NEWTON>
         __device__ __forceinline__ double weno5_flux(double f0, double f1, double f2, double f3, double f4)
         {
             const double eps = 1e-6;
@@ -264,7 +270,7 @@ namespace smr::dev
             // range, and the three divisions by the sum share one reciprocal
             // (larger values, infinities and NaN take the plain divisions).
             const double limit = 0x1p300;
-            if (g0 < limit && g1 < limit && g2 < limit)
+            if (NEWTON && g0 < limit && g1 < limit && g2 < limit)
             {
                 const double a0  = markstein_div(0.1, g0, newton_rcp(g0));
                 const double a1  = markstein_div(0.6, g1, newton_rcp(g1));
@@ -307,11 +313,11 @@ namespace smr::dev
                 double F;
                 if (vd >= 0)
                 {
-                    F = weno5_flux(w[0] * vd, w[1] * vd, w[2] * vd, w[3] * vd, w[4] * vd);
+                    F = weno5_flux<false>(w[0] * vd, w[1] * vd, w[2] * vd, w[3] * vd, w[4] * vd);
                 }
                 else
                 {
-                    F = weno5_flux(w[5] * vd, w[4] * vd, w[3] * vd, w[2] * vd, w[1] * vd);
+                    F = weno5_flux<false>(w[5] * vd, w[4] * vd, w[3] * vd, w[2] * vd, w[1] * vd);
                 }
                 acc += F * coef[k];
             }
@@ -319,6 +325,7 @@ namespace smr::dev
         }
 
         // the WENO5 flux of direction d from six values at base + j * stride
+        template <bool NEWTON>
         __device__ __forceinline__ double weno5_at(const double* __restrict__ base, int64_t stride, double vd)
         {
             double w[6];
@@ -326,8 +333,8 @@ namespace smr::dev
             {
                 w[j] = base[j * stride];
             }
-            return vd >= 0 ? weno5_flux(w[0] * vd, w[1] * vd, w[2] * vd, w[3] * vd, w[4] * vd)
-                           : weno5_flux(w[5] * vd, w[4] * vd, w[3] * vd, w[2] * vd, w[1] * vd);
+            return vd >= 0 ? weno5_flux<NEWTON>(w[0] * vd, w[1] * vd, w[2] * vd, w[3] * vd, w[4] * vd)
+                           : weno5_flux<NEWTON>(w[5] * vd, w[4] * vd, w[3] * vd, w[2] * vd, w[1] * vd);
         }
 
         // make_convection_weno5 on a mesh of one level whose storage is the dense
@@ -337,7 +344,7 @@ namespace smr::dev
         // in the order the interface walk gives them: left then right, except
         // at the low boundary, whose boundary interface comes after the
         // interior ones (the same sums as k_conv_weno5_gather, bit for bit).
-        template <int DIM>
+        template <int DIM, bool NEWTON>
         __global__ __launch_bounds__(BLOCK) void k_weno5_dense(const double* __restrict__ u, double* __restrict__ out, int n, int64_t W,
                                                                double v0, double v1, double v2, double fa)
         {
@@ -356,8 +363,8 @@ namespace smr::dev
                 const int64_t stride = d == 0 ? 1 : (d == 1 ? W : W * W);
                 const int coord      = d == 0 ? x : (d == 1 ? y : z);
                 const double vd      = d == 0 ? v0 : (d == 1 ? v1 : v2);
-                const double fl      = weno5_at(u + c - 3 * stride, stride, vd);
-                const double fr      = weno5_at(u + c - 2 * stride, stride, vd);
+                const double fl      = weno5_at<NEWTON>(u + c - 3 * stride, stride, vd);
+                const double fr      = weno5_at<NEWTON>(u + c - 2 * stride, stride, vd);
                 if (coord == 0)
                 {
                     acc += fr * fa;
@@ -377,6 +384,7 @@ namespace smr::dev
         // first column and row also the ones below and to the left) and shared
         // through LDS; the fluxes and the order of the sums are those of
         // k_weno5_dense<2>, so the results are the same bits.  n >= 64.
+        template <bool NEWTON>
         __global__ __launch_bounds__(256) void k_weno5_dense2d_tiled(const double* __restrict__ u, double* __restrict__ out, int n,
                                                                      int64_t W, double v0, double v1, double fa)
         {
@@ -386,15 +394,15 @@ namespace smr::dev
             const int x = int(blockIdx.x) * 64 + tx, y = int(blockIdx.y) * 4 + ty;
             const int g     = 3;
             const int64_t c = int64_t(y + g) * W + (x + g);
-            fx[ty][tx + 1]  = weno5_at(u + c - 2, 1, v0);
-            fy[ty + 1][tx]  = weno5_at(u + c - 2 * W, W, v1);
+            fx[ty][tx + 1]  = weno5_at<NEWTON>(u + c - 2, 1, v0);
+            fy[ty + 1][tx]  = weno5_at<NEWTON>(u + c - 2 * W, W, v1);
             if (tx == 0)
             {
-                fx[ty][0] = weno5_at(u + c - 3, 1, v0);
+                fx[ty][0] = weno5_at<NEWTON>(u + c - 3, 1, v0);
             }
             if (ty == 0)
             {
-                fy[0][tx] = weno5_at(u + c - 3 * W, W, v1);
+                fy[0][tx] = weno5_at<NEWTON>(u + c - 3 * W, W, v1);
             }
             __syncthreads();
             double acc = 0;
@@ -470,14 +478,14 @@ namespace smr::dev
             double left0 = 0;
             if (lane < R)
             {
-                left0 = weno5_at(u + c - lane + lane * W - 3, 1, v0);
+                left0 = weno5_at<true>(u + c - lane + lane * W - 3, 1, v0);
             }
-            double below = weno5_at(u + c - 3 * W, W, v1);
+            double below = weno5_at<true>(u + c - 3 * W, W, v1);
 #pragma unroll 1
             for (int r = 0; r < R; ++r, c += W)
             {
-                const double frx   = weno5_at(u + c - 2, 1, v0);
-                const double above = weno5_at(u + c - 2 * W, W, v1);
+                const double frx   = weno5_at<true>(u + c - 2, 1, v0);
+                const double above = weno5_at<true>(u + c - 2 * W, W, v1);
                 const double first = __longlong_as_double(readlane64(__double_as_longlong(left0), r));
                 const double shift = wave_shift<0x138>(frx);
                 const double flx   = lane == 0 ? first : shift;
@@ -499,7 +507,7 @@ namespace smr::dev
                 add(y0 + r == 0, below, above);
                 if constexpr (DIM == 3)
                 {
-                    const double flz = weno5_at(u + c - 3 * W * W, W * W, v2), frz = weno5_at(u + c - 2 * W * W, W * W, v2);
+                    const double flz = weno5_at<true>(u + c - 3 * W * W, W * W, v2), frz = weno5_at<true>(u + c - 2 * W * W, W * W, v2);
                     add(z == 0, flz, frz);
                 }
                 out[c] = acc;
@@ -1114,17 +1122,19 @@ namespace smr::dev
         const bool untiled = std::getenv("SMR_WENO5_UNTILED") != nullptr;
         const bool strips  = !untiled && n >= (dim == 3 ? 128 : 1024);
         auto waves        = [&](int rows) { return dim3(unsigned((total / 64 / rows + BLOCK / 64 - 1) / (BLOCK / 64))); };
+        const bool newton = total >= 1 << 17; // weno5_flux
+        const dim3 cells(nblocks(total)), tiles(unsigned(n / 64), unsigned(n / 4));
         if (!strips && dim == 3)
         {
-            hipLaunchKernelGGL(k_weno5_dense<3>, dim3(nblocks(total)), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
+            hipLaunchKernelGGL((newton ? k_weno5_dense<3, true> : k_weno5_dense<3, false>), cells, dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
         }
         else if (!strips && n >= 64 && !untiled)
         {
-            hipLaunchKernelGGL(k_weno5_dense2d_tiled, dim3(unsigned(n / 64), unsigned(n / 4)), dim3(256), 0, s, u, out, n, W, v[0], v[1], fa);
+            hipLaunchKernelGGL(newton ? k_weno5_dense2d_tiled<true> : k_weno5_dense2d_tiled<false>, tiles, dim3(256), 0, s, u, out, n, W, v[0], v[1], fa);
         }
         else if (!strips)
         {
-            hipLaunchKernelGGL(k_weno5_dense<2>, dim3(nblocks(total)), dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
+            hipLaunchKernelGGL((newton ? k_weno5_dense<2, true> : k_weno5_dense<2, false>), cells, dim3(BLOCK), 0, s, u, out, n, W, v[0], v[1], v[2], fa);
         }
         else if (dim == 3)
         {

@@ -35,10 +35,20 @@ def test_kernels_agree(gpu_ctx, dim, level, kind, monkeypatch):
         assert np.array_equal(got[k].view(np.uint64), want[k].view(np.uint64))
 
 
+@pytest.mark.parametrize("level", [8, 9, 10])
+def test_weights_of_larger_meshes_match_plain_divisions(gpu_ctx, level):
+    """The same where the divisions change to the shared reciprocals, and in strips."""
+    weights_match_plain_divisions(gpu_ctx, level)
+
+
 def test_weights_outside_the_range_match_plain_divisions(gpu_ctx):
     """One row of cells whose smoothness indicators grow past 2^300: the flux
     differences against the formula in numpy (IEEE divisions), bit for bit."""
-    level, n = 6, 64
+    weights_match_plain_divisions(gpu_ctx, 6)
+
+
+def weights_match_plain_divisions(gpu_ctx, level):
+    n = 1 << level
     mesh = sa.make_mesh(gpu_ctx, sa.mesh_config(2, level, level, 1, 3))
     u = sa.make_scalar_field("u", mesh)
     sa.make_bc_dirichlet(u, 0.0)
