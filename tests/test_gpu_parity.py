@@ -199,7 +199,7 @@ def test_convection_upwind_matches_oracle(gpu_ctx, dim, lmin, lmax, v):
     out = sa.make_convection_upwind(np.array(v))(u)
     got = out.storage()
     assert np.array_equal(bits(got), bits(ref))
-    # the cached contribution lists are reused for a second field on the mesh
+    # again on the same mesh, whose side table is there by now
     out2 = sa.make_convection_upwind(np.array(v))(u)
     assert np.array_equal(bits(out2.storage()), bits(ref))
 
