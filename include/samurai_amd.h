@@ -273,6 +273,10 @@ int smr_ctx_set_wait_rounds(smr_ctx* ctx, int rounds);
  * incomplete, the next call that waits for the context's work returns
  * SMR_ERR_RUNTIME, and from then on the operators run on term lists. */
 int smr_ctx_set_side_entries(smr_ctx* ctx, int64_t n);
+/* Device bytes the arrays of an adjoint problem made from now on may take in its
+ * dataflow form (by default as many as there are): with less it takes fewer
+ * steps per launch, then the stage programs. */
+int smr_ctx_set_flow_bytes(smr_ctx* ctx, int64_t bytes);
 /* The HIP stream (hipStream_t) the context orders its work on, for timing
  * with HIP events; NULL for a host-only context. */
 void* smr_ctx_stream(smr_ctx* ctx);

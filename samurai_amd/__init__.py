@@ -85,6 +85,7 @@ def lib():
         _sig(L, "smr_ctx_set_tag_form", "argtypes", [vp, i32])
         _sig(L, "smr_ctx_set_wait_rounds", "argtypes", [vp, i32])
         _sig(L, "smr_ctx_set_side_entries", "argtypes", [vp, i64])
+        _sig(L, "smr_ctx_set_flow_bytes", "argtypes", [vp, i64])
         _sig(L, "smr_timers_enable", "argtypes", [i32])
         _sig(L, "smr_timers_report", "restype", i64)
         _sig(L, "smr_timers_report", "argtypes", [ctypes.c_char_p, i64])
@@ -220,6 +221,10 @@ class Context:
     def set_side_entries(self, n):
         """Room for the flux operators' tables of the faces to finer cells (diagnostics)."""
         _check(lib().smr_ctx_set_side_entries(self.h, int(n)))
+
+    def set_flow_bytes(self, n):
+        """Device bytes the arrays of an adjoint problem made from now on may take in its dataflow form."""
+        _check(lib().smr_ctx_set_flow_bytes(self.h, int(n)))
 
     def stream(self):
         """The hipStream_t (as an integer) all work of this context runs on."""

@@ -1394,9 +1394,32 @@ namespace smr
         f.ew     = reinterpret_cast<const double*>(b.dptr(o_ew));
         f.par    = static_cast<const dev::FlowParam*>(flow->params.get(inst_.size() * sizeof(dev::FlowParam), st));
         flow->ticket.get(256, st);
-        const int between   = std::min(every_, kFlowSteps) - 1;
-        const size_t narr   = size_t(nseg_ + 1 + every_ - 1 + 2 + between);
-        flow->ckpt          = static_cast<double*>(flow->arrays.get(narr * size_t(n) * 8, st));
+        auto arrays = [&](int steps) { return size_t(nseg_ + 1 + every_ - 1 + 2 + steps - 1); };
+        auto room   = [&](int steps)
+        {
+            const size_t bytes = arrays(steps) * size_t(n) * 8;
+            if (bytes > ctx_->flow_bytes)
+            {
+                return false;
+            }
+            try
+            {
+                flow->arrays.get(bytes, st);
+            }
+            catch (const std::runtime_error&) // no device memory
+            {
+                (void)hipGetLastError();
+                return false;
+            }
+            flow->lam = steps;
+            return true;
+        };
+        if (!room(std::min(every_, kFlowSteps)) && !room(std::min(every_, 2)))
+        {
+            return nullptr;
+        }
+        const size_t narr   = arrays(flow->lam);
+        flow->ckpt          = static_cast<double*>(flow->arrays.p);
         flow->states        = flow->ckpt + int64_t(nseg_ + 1) * n;
         flow->ends          = flow->states + int64_t(every_ - 1) * n;
         flow->between       = flow->ends + 2 * n;
@@ -1436,7 +1459,7 @@ namespace smr
             dev::adjoint_flow_forward(w.f, states, false, ticket, ctx_->wait, s);
             for (int done = 0; done < every_;)
             {
-                const int k = std::min(kFlowSteps, every_ - done);
+                const int k = std::min(w.lam, every_ - done);
                 const dev::FlowArrays lam{end[cur], w.between, end[1 - cur], k};
                 dev::adjoint_flow_backward(w.f, lam, ticket, ctx_->wait, s);
                 dev::adjoint_flow_velocity(w.f, lam, states, every_ - 1 - done, ga_arena_, s);

@@ -140,10 +140,12 @@ namespace smr
             Blob tables;
             DevBuffer arrays, params, ticket;
             // nseg + 1 checkpoints, every - 1 states, two arrays at the ends of
-            // an adjoint launch and kFlowSteps - 1 between
+            // an adjoint launch of `lam` steps and lam - 1 between
             double *ckpt = nullptr, *states = nullptr, *ends = nullptr, *between = nullptr;
+            int lam      = 1;
         };
-        // adjoint steps per launch (their arrays are all in memory)
+        // adjoint steps per launch (their arrays are all in memory); where there is
+        // no room for them 2, which takes the arrays of the stage programs
         static constexpr int kFlowSteps = 16;
         std::unique_ptr<Flow> flow_;
         bool staged_         = false; // the next forward gives flow_ up

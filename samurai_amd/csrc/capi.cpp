@@ -645,6 +645,17 @@ extern "C"
             });
     }
 
+    int smr_ctx_set_flow_bytes(smr_ctx* ctx, int64_t bytes)
+    {
+        return guarded(
+            [&]
+            {
+                require(ctx && bytes >= 0, "a number of bytes is expected");
+                ctx->c.flow_bytes = size_t(bytes);
+                return 0;
+            });
+    }
+
     int smr_ctx_set_side_entries(smr_ctx* ctx, int64_t n)
     {
         return guarded(

@@ -371,6 +371,7 @@ namespace smr
         dev::FlowWait wait{1 << 17, nullptr};
         void allocate_fault_words();
         int64_t side_entries = INT64_MAX; // room for a side table's entries
+        size_t flow_bytes    = SIZE_MAX;  // and for the arrays of a gradient's dataflow form
         bool no_sides        = false;     // set when one was incomplete
         void mark_runs_back();
         ~Ctx();

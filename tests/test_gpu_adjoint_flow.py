@@ -82,3 +82,38 @@ def test_tuning_between_forward_and_backward(gpu_ctx):
     p.set_velocity([[0.1, -0.3]])
     with pytest.raises(sa.SamuraiError):
         p.backward_ptr(gT.data_ptr(), g0.data_ptr())
+
+
+def test_less_room_means_fewer_steps_per_launch(gpu_ctx):
+    """The arrays of a launch of 12 adjoint steps, of 2, and no room for those:
+    the stage programs.  (A wait without rounds shows which form runs.)"""
+    import samurai_amd as sa
+    import torch
+    print("less room", flush=True)
+    ctx = sa.Context(0)
+    mesh, u = frozen(sa, ctx, 2, 6, 1, 7)
+    steps, every = 24, 12
+    u0 = torch.tensor(u, device="cuda")
+    gT = torch.tensor(np.random.default_rng(3).standard_normal(u0.numel()), device="cuda")
+    uT, g0 = torch.empty_like(u0), torch.empty_like(u0)
+    torch.cuda.synchronize()
+    least = 8 * mesh.nb_cells(sa.REFERENCE) * (steps // every + every + 3)  # what the stage programs take
+    got = []
+    for room, flow in ((1 << 40, True), (least, True), (least - 1, False)):
+        ctx.set_flow_bytes(room)
+        p = sa.AdjointProblem(ctx, [mesh], [0.2 / 64], bc=[0.5], steps=steps, checkpoint_every=every)
+        p.set_velocity([[0.7, -0.3]])
+        p.forward_ptr(u0.data_ptr(), uT.data_ptr())
+        ga = p.backward_ptr(gT.data_ptr(), g0.data_ptr())
+        got.append((uT.cpu().numpy(), g0.cpu().numpy(), ga))
+        ctx.set_wait_rounds(0)
+        if flow:
+            with pytest.raises(sa.SamuraiError, match="adjoint"):
+                p.forward_ptr(u0.data_ptr(), uT.data_ptr())
+        else:
+            p.forward_ptr(u0.data_ptr(), uT.data_ptr())
+        ctx.set_wait_rounds(1 << 17)
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a, b)
+    ctx.close()
