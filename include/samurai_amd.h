@@ -424,7 +424,8 @@ int smr_adjoint_forward(smr_adjoint* adj, const double* u0, double* uT);
 /* grad_uT (device) -> grad_u0 (device) and grad_a (host, n*3) of the last forward */
 int smr_adjoint_backward(smr_adjoint* adj, const double* grad_uT, double* grad_u0, double* grad_a);
 /* runs the adjoint as stage programs of that launch shape (as
- * smr_batch_set_tuning) instead of the dataflow launches */
+ * smr_batch_set_tuning) instead of the dataflow launches, from the next forward
+ * on; a backward before it belongs to the last forward */
 int smr_adjoint_set_tuning(smr_adjoint* adj, int block, int cells_per_thread, int mode);
 
 #ifdef __cplusplus

@@ -2,7 +2,7 @@
 //
 // The update is a chain of stages (per level, finest first: outer ghosts, then
 // the projection into the level below; then the predictions, coarsest level
-// first), about 35 of them on a 2D L4..12 mesh.  Most ghosts do not need that
+// first), 37 of them on a 2D L4..12 mesh.  Most ghosts do not need that
 // order: a ghost waits only for the ghosts it reads, and on graded meshes 94 %
 // of them read cells or ghosts that read cells (2D L4..12: 41 K and 40 K of
 // 87 K ghosts at depth 1 and 2, the deepest at 10).  So every ghost is written
@@ -16,8 +16,8 @@
 // Bound: latency, launch + index chain + one store-to-load trip per depth.
 // The stages were bound by their launches (3 to 4 us each) and, for the small
 // ones, by a block barrier and a chain of five dependent loads per stage.
-// update_ghost_mr + upwind, one step: 2D L4..12 (158 K cells) 28 us against 90
-// with a launch per stage, 3D L2..8 (234 K cells) 38 against 96, 2D L2..7
+// update_ghost_mr + upwind, one step: 2D L4..12 (158 K cells) 27 us against 90
+// with a launch per stage, 3D L2..8 (234 K cells) 36 against 96, 2D L2..7
 // (5.9 K cells) 19 against 26.
 //
 // Every wait ends.  Blocks take their place in the order of the ghosts from a
