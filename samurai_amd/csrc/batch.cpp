@@ -1479,7 +1479,7 @@ namespace smr
                                          return;
                                      }
                                      r.nm = dev_ids ? std::move(nms[size_t(q)]) : build_mesh(c, std::move(cas[size_t(q)]));
-                                     adapted_from(r.nm, m.host);
+                                     adapted_from(r.nm, m.host, true);
                                      if (dev_lists)
                                      {
                                          r.device_lists = true;
@@ -1516,7 +1516,7 @@ namespace smr
                                          return;
                                      }
                                      r.nm = build_mesh(c, std::move(ca));
-                                     adapted_from(r.nm, m.host);
+                                     adapted_from(r.nm, m.host, true);
                                      r.img = build_host_image(r.nm);
                                      build_update_fields_lists(m.host, r.nm, r.copy, r.coarsen, r.refine);
                                  });

@@ -368,8 +368,8 @@ extern "C"
                 {
                     smr::ScopedTimer t3(nullptr, "mesh construction");
                     nm = smr::build_mesh(mm.host.cfg, ca);
-                    smr::adapted_from(nm, mm.host);
                 }
+                smr::adapted_from(nm, mm.host, false);
                 mm.replace(std::move(nm), nullptr);
                 return 0;
             });
@@ -400,7 +400,7 @@ extern "C"
                 {
                     smr::ScopedTimer t3(nullptr, "mesh construction");
                     nm = smr::build_mesh(m.cfg, ca);
-                    smr::adapted_from(nm, m);
+                    smr::adapted_from(nm, m, false);
                 }
                 smr::WorkList copy, coarsen, refine;
                 smr::build_update_fields_lists(m, nm, copy, coarsen, refine);

@@ -415,12 +415,12 @@ namespace smr
         return true;
     }
 
-    void adapted_from(MRMeshData& m, const MRMeshData& old)
+    void adapted_from(MRMeshData& m, const MRMeshData& old, bool whole_families)
     {
         m.graduated = true;
-        // a leaf is replaced by its children or its parent, never by less: the
+        // with whole families a leaf is replaced by its children or its parent: the
         // leaves still cover what they covered
-        m.tiles = tiles_box(m, old.tiles);
+        m.tiles = tiles_box(m, old.tiles && whole_families);
     }
 
     CellArray update_cell_array_from_tag(const MRMeshData& mesh, const uint8_t* tags)

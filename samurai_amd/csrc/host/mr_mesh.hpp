@@ -85,8 +85,10 @@ namespace smr
     // whether m's cells tile the unit box, from their volume alone when they are
     // known to cover it
     bool tiles_box(const MRMeshData& m, bool covered);
-    // sets the properties of m, the graduated mesh that tags made of `old`
-    void adapted_from(MRMeshData& m, const MRMeshData& old);
+    // sets the properties of m, the graduated mesh that tags made of `old`.  An
+    // adaptation's own tags coarsen whole families; a caller's may take single
+    // cells away (the parent comes with the family's first child)
+    void adapted_from(MRMeshData& m, const MRMeshData& old, bool whole_families);
     // mra::make_mesh(unit box, cfg): all cells at max_level (mr/mesh.hpp:510-518)
     MRMeshData build_box_mesh(const MeshConfig& cfg);
 

@@ -2311,7 +2311,6 @@ namespace smr
                 old_sets = o;
             }
             *mesh = device_submesh(ctx, cfg, b, buf[cur], *current, old_sets, lists);
-            adapted_from(*mesh, *current);
             return true;
         }
         ScopedTimer t(&ctx, "leaves to host");
@@ -2523,8 +2522,8 @@ namespace smr
             {
                 ScopedTimer t3(nullptr, "mesh construction");
                 nm = build_mesh(cfg, std::move(new_ca));
-                adapted_from(nm, m.host);
             }
+            adapted_from(nm, m.host, true);
         }
         if (dl.nlists == int(dev::DL_N))
         {

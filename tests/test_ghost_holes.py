@@ -75,6 +75,47 @@ def test_partial_families_have_no_flow(host_ctx):
     assert m.ghost_form() == 0
 
 
+def partial_flags(m, dim):
+    """Flags on a mesh of 16^dim cells that coarsen the first child of one family
+    (its parent then lies over the others) and, of as many families as make up for
+    that, another child (which leaves a hole)."""
+    c = m.cells()
+    at = {tuple(x[1:1 + dim]): x[4] for x in c}
+    tags = np.zeros(m.nb_cells(sa.REFERENCE), dtype=np.uint8)
+    tags[c[:, 4]] = sa.KEEP
+    tags[at[(4,) * dim]] = sa.COARSEN
+    for f in range(1, 1 << dim):
+        tags[at[(1 + 2 * (f % 4), 9, 1 + 2 * (f // 4))[:dim]]] = sa.COARSEN
+    return tags
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+def test_holes_and_overlaps_of_one_volume_have_no_flow(host_ctx, dim):
+    m = sa.make_mesh(host_ctx, sa.mesh_config(dim, 2, 4))
+    assert m.ghost_form() == 1
+    m.rebuild_from_tags(partial_flags(m, dim))
+    assert (2.0 ** (-dim * m.cells()[:, 0].astype(float))).sum() == 1.0
+    assert m.ghost_form() == 0 and m.validate() == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim", [2, 3])
+def test_holes_from_device_flags_have_no_flow(gpu_ctx, dim):
+    import torch
+    print("device flags", dim, flush=True)
+    m = sa.make_mesh(gpu_ctx, sa.mesh_config(dim, 2, 4))
+    gpu_ctx.set_ghost_form(1)
+    try:
+        assert m.ghost_form() == 2
+        tags = torch.tensor(partial_flags(m, dim), device="cuda")
+        torch.cuda.synchronize()
+        assert m.rebuild_from_device_tags(tags.data_ptr(), tags.numel()) == 0
+        assert (2.0 ** (-dim * m.cells()[:, 0].astype(float))).sum() == 1.0
+        assert m.ghost_form() == 0
+    finally:
+        gpu_ctx.set_ghost_form(-1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dim,lmin,lmax,s", MESHES)
 def test_holed_ghosts_match_oracle(gpu_ctx, host_ctx, dim, lmin, lmax, s):
