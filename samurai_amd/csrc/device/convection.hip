@@ -425,7 +425,10 @@ namespace smr::dev
 
         // the first blocks take the cells; the others, 8 slots a thread, zero the
         // slots that are no cells (a clearing of the whole output ahead of the
-        // launch was another 2 us of a small mesh's 18)
+        // launch was another 2 us of a small mesh's 18).  No bound on the registers:
+        // 68 instead of 88 for the 3D velocity field took uniform L7 from 51.1 to
+        // 46.6 us, but small meshes, which wait for their loads together, from 51.5
+        // to 54.7 (L2..4) and 88.4 to 92.3 (L2..5).
         template <int DIM, int OP>
         __global__ __launch_bounds__(CB) void k_convection(List l, ConvSides sd, ConvFields a, double* __restrict__ out, unsigned cell_blocks)
         {

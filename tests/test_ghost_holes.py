@@ -190,3 +190,30 @@ def test_holed_batch_and_gradient(gpu_ctx, host_ctx, dim, lmin, lmax, s):
         assert all(np.isfinite(x).all() for x in got[-1])
     for x, y in zip(*got):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,lmax,s", [(2, 6, 0), (3, 4, 0), (3, 4, 1)])
+def test_jumps_of_several_levels_match_oracle(gpu_ctx, host_ctx, dim, lmax, s):
+    """Leaves that tile the box but are not graduated have the flow: both forms."""
+    from test_gpu_convection_terms import jumps
+    cells = jumps(dim, lmax, 3)
+    print("jumps", dim, lmax, s, len(cells), flush=True)
+    o = OracleSim(dim, 2, lmax, pred_s=s, cells=cells)
+    o.set_poison(False)
+    o.set_dirichlet(0.75)
+    mesh = sa.make_mesh_from_cells(gpu_ctx, sa.mesh_config(dim, 2, lmax, s), cells)
+    u = sa.make_scalar_field("u", mesh)
+    sa.make_bc_dirichlet(u, 0.75)
+    st = np.random.default_rng(1).standard_normal(u.size())
+    o.set_storage(st)
+    o.update_ghost_mr()
+    try:
+        for form in (0, 1):
+            gpu_ctx.set_ghost_form(form)
+            assert mesh.ghost_form() == 2 * form
+            u.set_storage(st)
+            sa.update_ghost_mr(u)
+            assert np.array_equal(o.storage().view(np.uint64), u.storage().view(np.uint64)), form
+    finally:
+        gpu_ctx.set_ghost_form(-1)
