@@ -318,12 +318,56 @@ namespace smr
             m.level_base[MAXL] = n;
             m.nref             = n;
         }
+
+        bool disjoint(const LevelSet& a, const LevelSet& b)
+        {
+            size_t rb = 0;
+            for (size_t ra = 0; ra < a.nrows(); ++ra)
+            {
+                while (rb < b.nrows() && row_less(b.ry[rb], b.rz[rb], a.ry[ra], a.rz[ra]))
+                {
+                    ++rb;
+                }
+                if (rb == b.nrows())
+                {
+                    return true;
+                }
+                if (row_less(a.ry[ra], a.rz[ra], b.ry[rb], b.rz[rb]))
+                {
+                    continue;
+                }
+                for (int64_t i = a.rp[ra], k = b.rp[rb]; i < a.rp[ra + 1] && k < b.rp[rb + 1];)
+                {
+                    const Run& x = a.runs[size_t(i)];
+                    const Run& y = b.runs[size_t(k)];
+                    if (x.s < y.e && y.s < x.e)
+                    {
+                        return false;
+                    }
+                    x.e <= y.s ? ++i : ++k;
+                }
+            }
+            return true;
+        }
+
+        // in units of a cell of the finest level there can be: exact, the box
+        // being 2^60 of them in 3D
+        bool has_box_volume(const MRMeshData& m)
+        {
+            uint64_t volume = 0;
+            for (int l = 0; l < MAXL; ++l)
+            {
+                volume += uint64_t(m.ids[CELLS][size_t(l)].count()) << (m.cfg.dim * (MAXL - 1 - l));
+            }
+            return volume == uint64_t(1) << (m.cfg.dim * (MAXL - 1));
+        }
     } // namespace
 
     void complete_mesh(MRMeshData& m)
     {
         construct_corners(m);
         renumbering(m);
+        m.box_volume = has_box_volume(m);
     }
 
     MRMeshData build_mesh(const MeshConfig& cfg, const CellArray& cells)
@@ -363,8 +407,7 @@ namespace smr
         }
         m.ids[CELLS] = std::move(cells);
         update_sub_mesh(m);
-        construct_corners(m);
-        renumbering(m);
+        complete_mesh(m);
         return m;
     }
 
@@ -380,14 +423,7 @@ namespace smr
 
     bool tiles_box(const MRMeshData& m, bool covered)
     {
-        // in units of a cell of the finest level there can be: exact, the box
-        // being 2^60 of them in 3D
-        uint64_t volume = 0;
-        for (int l = 0; l < MAXL; ++l)
-        {
-            volume += uint64_t(m.ids[CELLS][size_t(l)].count()) << (m.cfg.dim * (MAXL - 1 - l));
-        }
-        if (volume != uint64_t(1) << (m.cfg.dim * (MAXL - 1)))
+        if (!m.box_volume)
         {
             return false;
         }
@@ -407,7 +443,7 @@ namespace smr
                 inside = c.ry[r] >= 0 && c.ry[r] < n && (m.cfg.dim == 2 || (c.rz[r] >= 0 && c.rz[r] < n))
                       && c.runs[size_t(c.rp[r])].s >= 0 && c.runs[size_t(c.rp[r + 1]) - 1].e <= n;
             }
-            if (!inside || !set_intersection(c, m.ids[UNION_CELLS][size_t(l)]).empty())
+            if (!inside || !disjoint(c, m.ids[UNION_CELLS][size_t(l)]))
             {
                 return false;
             }

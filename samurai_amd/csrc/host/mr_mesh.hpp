@@ -66,6 +66,9 @@ namespace smr
         // the cells tile the unit box (no hole, no overlap, none outside) on
         // levels up to max_level
         bool tiles = false;
+        // the cells have the box's volume (a mesh the device builds gets this while
+        // the device is busy with its lists)
+        bool box_volume = false;
 
         const LevelSet& get(int id, int level) const { return ids[id][size_t(level)]; }
         // storage index of a reference cell; throws std::out_of_range if absent
@@ -82,8 +85,8 @@ namespace smr
     // corners and renumbering of a mesh whose five ids are set (the ids built
     // elsewhere, e.g. on the device, as build_mesh would build them)
     void complete_mesh(MRMeshData& m);
-    // whether m's cells tile the unit box, from their volume alone when they are
-    // known to cover it
+    // whether the cells of a complete mesh tile the unit box, from their volume
+    // alone when they are known to cover it
     bool tiles_box(const MRMeshData& m, bool covered);
     // sets the properties of m, the graduated mesh that tags made of `old`.  An
     // adaptation's own tags coarsen whole families; a caller's may take single
